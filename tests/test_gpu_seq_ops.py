@@ -1,0 +1,94 @@
+"""The sequence forms of add, RMSNorm and SwiGLU (kt_hip_ref_*_seq) at the sizes where their grids change: rows that do
+not fill a CTA of four, a row longer or shorter than a wave's stride, the last row count every CTA folds itself and
+the first that takes the one-CTA fold, and tensors with fewer, as many and more values than the first pass has slots
+for. Codes and records equal the oracle's; SwiGLU equals the one-CTA kernel, which its own tests hold to the oracle."""
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def rec(torch, sc):
+    w = np.zeros(4, dtype=np.int64)
+    w[0] = sc[0]
+    w.view(np.int32)[2] = sc[1]
+    return torch.from_numpy(w).cuda()
+
+
+def rd(r):
+    w = r.cpu().numpy()
+    return int(w[0]), int(w.view(np.int32)[2])
+
+
+def dev(torch, a):
+    return torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32).reshape(-1)).cuda()
+
+
+def rand_scale(rng):
+    return int(rng.integers(2**30, 2**31)), int(rng.integers(40, 62))
+
+
+def ws(torch, rows):
+    from tritify_amd import backend as B
+
+    n = B.ref_seq_workspace(rows)
+    return torch.full((n,), 0xA5, dtype=torch.uint8, device="cuda"), n  # its contents must not matter
+
+
+@pytest.mark.parametrize("rows,dim", [(1, 1), (2, 63), (3, 65), (5, 512), (7, 513), (130, 896), (1024, 33),
+                                      (1025, 33), (2500, 16)])
+@pytest.mark.parametrize("mag", [1, 2**28, 2**31 - 1])
+def test_rmsnorm_seq_edges(torch_dev, rows, dim, mag):
+    torch = torch_dev
+    from tritify_amd import backend as B
+
+    print(f"case: rmsnorm_seq rows={rows} dim={dim} mag={mag}", file=sys.stderr, flush=True)
+    rng = np.random.default_rng(rows * 131 + dim)
+    x = rng.integers(-mag, mag + 1, size=(rows, dim)).astype(np.int32)
+    x[rows // 2] = 0  # a row whose factor is the eps alone: the largest, over rows that are all far below it
+    if rows > 4:
+        x[-1] = x[0]  # equal factors: the fold's later row
+        x[1] = np.sign(x[1]) * (np.abs(x[1].astype(np.int64)) >> 9)
+    g = rng.integers(-O.WLEVELS, O.WLEVELS + 1, size=dim).astype(np.int32)
+    if mag == 2**31 - 1:
+        x[0, 0], g[0] = -2**31, -2**31  # the largest product there is
+    gs, eps = rand_scale(rng), B.ref_scale_from_f64(1e-6)
+    w, n = ws(torch, rows)
+    y, ys = torch.zeros(rows * dim, dtype=torch.int32, device="cuda"), rec(torch, (0, 0))
+    for xs in (rand_scale(rng), (0, 0)):
+        B.ref_rmsnorm_seq(dev(torch, x), rec(torch, xs), rows, dim, dev(torch, g), gs, eps, w, n, y, ys)
+        yo, so = O.rd_rmsnorm(x.reshape(-1), rows, dim, xs, g, gs, eps)
+        assert np.array_equal(y.cpu().numpy(), yo) and rd(ys) == so, xs
+
+
+@pytest.mark.parametrize("n", [1, 255, 1024, 1025, 512 * 1024, 512 * 1024 + 3])
+def test_add_and_swiglu_seq_edges(torch_dev, n):
+    torch = torch_dev
+    from tritify_amd import backend as B
+
+    print(f"case: add_seq / swiglu_seq n={n}", file=sys.stderr, flush=True)
+    rng = np.random.default_rng(n)
+    a = rng.integers(-(2**28), 2**28 + 1, size=n).astype(np.int32)
+    b = rng.integers(-(2**28), 2**28 + 1, size=n).astype(np.int32)
+    b[-1] = 2**28 + 7  # the largest value is the last one's
+    w, nw = ws(torch, 1)
+    for sa, sb in ((rand_scale(rng), rand_scale(rng)), (rand_scale(rng), (0, 0)), ((0, 0), (0, 0))):
+        yo, so = O.rd_add(a, sa, b, sb)
+        ad, ar = dev(torch, a), rec(torch, sa)
+        B.ref_add_seq(ad, ar, dev(torch, b), rec(torch, sb), n, w, nw, ad, ar)  # in place, as the residual add
+        assert np.array_equal(ad.cpu().numpy(), yo) and rd(ar) == so, (sa, sb)
+    codes, lut = B.ref_codelut(B.LUT_SILU, -30.0, 30.0, 16, 20, True)
+    cd = torch.from_numpy(codes).cuda()
+    for gshift in (53, 60):
+        gs, us = (int(rng.integers(2**30, 2**31)), gshift), rand_scale(rng)
+        out = []
+        for seq in (False, True):
+            h, hs = torch.zeros(n, dtype=torch.int32, device="cuda"), rec(torch, (0, 0))
+            args = (dev(torch, a), rec(torch, gs), dev(torch, b), rec(torch, us), n, cd, lut)
+            B.ref_swiglu_seq(*args, w, nw, h, hs) if seq else B.ref_swiglu(*args, h, hs)
+            out.append((h.cpu().numpy(), rd(hs)))
+        assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1], gshift

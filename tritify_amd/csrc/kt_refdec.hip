@@ -1359,14 +1359,28 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_combine_kernel(RdAttn
         put_rec(a.os, gmax == 0 ? Sc{0, 0} : sc_mul(from_ratio((u128)(uint64_t)gmax, (u128)ACT_LEVELS), common));
 }
 
-// The same ops over whole-sequence tensors on many CTAs (the batched forward's T-row tensors): one CTA forms the
-// tensor's Scales (and an RMSNorm's row factors) into the workspace and zeroes its max slot, a grid pass takes the
-// largest magnitude, a grid pass requantizes and writes the record. Integers identical to the one-CTA kernels.
+// The same ops over whole-sequence tensors on many CTAs (the batched forward's T-row tensors), two launches each: a
+// grid pass takes the largest magnitude, a grid pass requantizes and writes the record. Integers identical to the
+// one-CTA kernels.
+//  - Every wave forms the tensor's Scales itself on wave-uniform values (two or three Scale steps, under a
+//    microsecond): no one-CTA launch before the pass.
+//  - A CTA's largest magnitude goes to its own slot of the workspace and the second pass takes the largest slot. An
+//    atomic maximum on one word serialized (13 ns a CTA): SwiGLU's first pass at 256 x 4864 went from 28.3 (2,048
+//    CTAs) to 10.1 us, the add's at 256 x 896 from 13.1 (896 CTAs) to 5.5 us.
+//  - RMSNorm's first pass is a wave per row: the exact sum of squares, max |x g|, the row factor's Scale chain, all
+//    rows side by side (8.3 us at 256 x 896; one CTA of 16 waves walking the rows took about 120). A factor f >= 0 keeps
+//    order (Scale::apply rounds |v| monotonely, and f <= 1 so nothing wraps), so the tensor's largest magnitude is
+//    the largest apply(f_row, max |x g| of the row): no pass over the values is needed for it.
+constexpr int RS_PARTS = 512;        // the first pass's CTAs at most
+constexpr int RS_FOLD_ROWS = 1024;   // RMSNorm rows that every CTA of the second pass folds itself
 struct RdSeqWs {
-    Sc par[4];      // add: common, fa, fb; SwiGLU: index factor, identity factor, h scale; RMSNorm: cc
-    uint64_t gmax;  // the largest magnitude
-    Sc frow[1];     // RMSNorm: each row's factor over cc (rows of them)
+    Sc par[4];               // RMSNorm past RS_FOLD_ROWS rows: the common Scale
+    uint64_t gmax;           // and the largest magnitude
+    int64_t part[RS_PARTS];  // the largest magnitude of each CTA of the first pass
+    // then RMSNorm's rows: Sc crow[rows] (the row factor), int64_t pmax[rows] (the largest |x g| of the row)
 };
+__host__ __device__ inline Sc* rs_crow(RdSeqWs* w) { return reinterpret_cast<Sc*>(w + 1); }
+__host__ __device__ inline int64_t* rs_pmax(RdSeqWs* w, int rows) { return reinterpret_cast<int64_t*>(rs_crow(w) + rows); }
 enum { RS_ADD = 0, RS_SWIGLU = 1, RS_NORM = 2 };
 struct RdSeq {
     int op;
@@ -1383,96 +1397,178 @@ struct RdSeq {
     kt_hip_qscale* ys;
 };
 
-__device__ inline int64_t rs_value(const RdSeq& q, const RdSeqWs* w, int64_t i) {
-    if (q.op == RS_ADD) return wadd(sc_apply32(w->par[1], q.a[i]), sc_apply32(w->par[2], q.b[i]));
-    if (q.op == RS_SWIGLU) {
-        const int32_t gd = q.a[i];
-        const int64_t idx = lut_index32(w->par[0], gd, q.lut.lo_index);
-        const int64_t code = idx < 0 ? 0 : (idx >= q.lut.n ? sc_apply32(w->par[1], gd) : lut_code(q.codes, q.lut.n, idx));
-        return wmul(code, q.b[i]);
+// add: common, fa, fb; SwiGLU (as is g's record, bs u's): index factor, identity factor, h scale.
+struct RsPar {
+    Sc p0, p1, p2;
+};
+template <int OP>
+__device__ inline RsPar rs_params(const RdSeq& q, const kt_hip_qscale* as_rec, const kt_hip_qscale* bs_rec) {
+    const Sc as = uni(rec_sc(as_rec)), bs = uni(rec_sc(bs_rec)), z{0, 0};
+    if constexpr (OP == RS_ADD) {
+        const Sc common = sc_ge(as, bs) ? as : bs;
+        if (common.mant == 0) return RsPar{common, z, z};
+        const Sc cinv = sc_recip(common);
+        return RsPar{common, sc_mul(as, cinv), sc_mul(bs, cinv)};
+    } else {
+        const Sc cs{q.lut.code_mant, q.lut.code_shift};
+        return RsPar{sc_mul(as, Sc{q.lut.inv_mant, q.lut.inv_shift}), sc_mul(as, sc_recip(cs)), sc_mul(cs, bs)};
     }
-    return sc_apply(w->frow[i / q.dim], (int64_t)q.a[i] * (int64_t)q.b[i % q.dim]);
+}
+template <int OP>
+__device__ inline int64_t rs_value(const RdSeq& q, const RsPar& p, int32_t a, int32_t b) {
+    if constexpr (OP == RS_ADD) {
+        return wadd(sc_apply32(p.p1, a), sc_apply32(p.p2, b));
+    } else {
+        const int64_t idx = lut_index32(p.p0, a, q.lut.lo_index);
+        const int64_t code = idx < 0 ? 0 : (idx >= q.lut.n ? sc_apply32(p.p1, a) : lut_code(q.codes, q.lut.n, idx));
+        return wmul(code, b);
+    }
 }
 // whether the values are live (a zero common scale gives zeros)
-__device__ inline bool rs_live(const RdSeq& q, const RdSeqWs* w) { return q.op == RS_SWIGLU || w->par[0].mant != 0; }
+template <int OP>
+__device__ inline bool rs_live(const RsPar& p) { return OP == RS_SWIGLU || p.p0.mant != 0; }
 
-__global__ __launch_bounds__(RD_THREADS) void rs_prep_kernel(RdSeq q) {
-    __shared__ ScIdx redsc[RD_THREADS];
-    RdSeqWs* w = q.ws;
-    if (q.op == RS_NORM) {  // as rd_rmsnorm_kernel, the row factors in the workspace
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const Sc xs = rec_sc(q.as), gs{q.g_mant, q.g_shift}, eps{q.e_mant, q.e_shift};
-        for (int r = wave; r < q.rows; r += RD_WAVES) {
-            uint64_t hi = 0, lo = 0;
-            for (int i = lane; i < q.dim; i += 64) {
-                const int64_t v = q.a[(size_t)r * q.dim + i];
-                const uint64_t sq = (uint64_t)(v * v), t = lo + sq;
-                hi += t < lo, lo = t;
-            }
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const uint64_t ohi = __shfl_xor(hi, o, 64), olo = __shfl_xor(lo, o, 64), t = lo + olo;
-                hi += ohi + (t < lo), lo = t;
-            }
-            if (lane == 0) {
-                const Sc mean_sq = sc_mul(sc_mul(from_ratio(((u128)hi << 64) | lo, (u128)q.dim), xs), xs);
-                const Sc denom = sc_add(mean_sq, eps);
-                w->frow[r] = sc_mul(sc_mul(xs, denom.mant == 0 ? Sc{0, 0} : sc_rsqrt(denom)), gs);
-            }
-        }
-        __syncthreads();  // the CTA's own global writes are visible to it past the barrier
-        ScIdx best{Sc{0, 0}, -1};
-        for (int r = threadIdx.x; r < q.rows; r += RD_THREADS) best = sc_pick(best, ScIdx{w->frow[r], r});
-        const Sc cc = block_fold_max(best, redsc, q.rows).s;
-        if (cc.mant != 0) {
-            const Sc cinv = sc_recip(cc);
-            for (int r = threadIdx.x; r < q.rows; r += RD_THREADS) w->frow[r] = sc_mul(w->frow[r], cinv);
-        }
-        if (threadIdx.x == 0) w->par[0] = cc, w->gmax = 0;
-        return;
-    }
-    if (threadIdx.x == 0) {
-        const Sc as = rec_sc(q.as), bs = rec_sc(q.bs);
-        if (q.op == RS_ADD) {
-            const Sc common = sc_ge(as, bs) ? as : bs;
-            w->par[0] = common, w->par[1] = w->par[2] = Sc{0, 0};
-            if (common.mant != 0) {
-                const Sc cinv = sc_recip(common);
-                w->par[1] = sc_mul(as, cinv), w->par[2] = sc_mul(bs, cinv);
-            }
-        } else {  // SwiGLU: as is g's record, bs u's
-            const Sc cs{q.lut.code_mant, q.lut.code_shift};
-            w->par[0] = sc_mul(as, Sc{q.lut.inv_mant, q.lut.inv_shift});
-            w->par[1] = sc_mul(as, sc_recip(cs));
-            w->par[2] = sc_mul(cs, bs);
-        }
-        w->gmax = 0;
-    }
+// the largest of the first pass's slots, in every thread of a 256-thread CTA
+__device__ inline int64_t rs_gmax(const RdSeqWs* w, int nparts, int64_t* red) {
+    int64_t m = 0;
+    for (int i = threadIdx.x; i < nparts; i += 256) m = max64(m, w->part[i]);
+    return block_max_4w(m, red);
 }
 
+template <int OP>
 __global__ __launch_bounds__(256) void rs_max_kernel(RdSeq q) {
     __shared__ int64_t red[4];
-    const RdSeqWs* w = q.ws;
+    const RsPar p = rs_params<OP>(q, q.as, q.bs);
+    const int64_t step = (int64_t)gridDim.x * 256;
     int64_t m = 0;
-    if (rs_live(q, w))
-        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < q.n; i += (int64_t)gridDim.x * 256) {
-            const int64_t v = iabs(rs_value(q, w, i));
-            m = v > m ? v : m;
+    if (rs_live<OP>(p)) {
+        for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < q.n; i0 += 4 * step) {  // 4 loads in flight
+            int32_t a[4], b[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int64_t i = i0 + u * step;
+                a[u] = i < q.n ? q.a[i] : 0, b[u] = i < q.n ? q.b[i] : 0;  // zeros give a zero (add; silu * 0)
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) m = max64(m, iabs(rs_value<OP>(q, p, a[u], b[u])));
         }
+    }
     m = block_max_4w(m, red);
-    if (threadIdx.x == 0 && m > 0) atomicMax(reinterpret_cast<unsigned long long*>(&q.ws->gmax), (unsigned long long)m);
+    if (threadIdx.x == 0) q.ws->part[blockIdx.x] = m;
+    // the record of y may be a's or b's (add in place): its reader takes the inputs' Scales from here
+    if (blockIdx.x == 0 && threadIdx.x == 0) q.ws->par[0] = p.p0, q.ws->par[1] = p.p1, q.ws->par[2] = p.p2;
 }
 
-__global__ __launch_bounds__(256) void rs_out_kernel(RdSeq q) {
+template <int OP>
+__global__ __launch_bounds__(256) void rs_out_kernel(RdSeq q, int nparts) {
+    __shared__ int64_t red[4];
     const RdSeqWs* w = q.ws;
-    const int64_t gmax = (int64_t)w->gmax;
+    const RsPar p{w->par[0], w->par[1], w->par[2]};
+    const int64_t gmax = rs_gmax(w, nparts, red);
     const RqDen rd_gmax = rq_den(gmax);
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < q.n; i += (int64_t)gridDim.x * 256)
-        q.y[i] = gmax == 0 ? 0 : rq_apply(rd_gmax, rs_value(q, w, i));
+        q.y[i] = gmax == 0 ? 0 : rq_apply(rd_gmax, rs_value<OP>(q, p, q.a[i], q.b[i]));
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const Sc sc = q.op == RS_SWIGLU ? w->par[2] : w->par[0];  // the tensor's scale before the requant
+        const Sc sc = OP == RS_SWIGLU ? p.p2 : p.p0;  // the tensor's scale before the requant
         put_rec(q.ys, gmax == 0 ? Sc{0, 0} : sc_mul(from_ratio((u128)(uint64_t)gmax, (u128)ACT_LEVELS), sc));
     }
+}
+
+// RMSNorm's first pass: a wave per row.
+__global__ __launch_bounds__(256) void rs_rows_kernel(RdSeq q) {
+    const int lane = threadIdx.x & 63, r = (int)blockIdx.x * 4 + wave_id();
+    if (r >= q.rows) return;  // the whole wave
+    const int32_t* xr = q.a + (size_t)r * q.dim;
+    uint64_t hi = 0, lo = 0;
+    int64_t pm = 0;
+    for (int i0 = lane; i0 < q.dim; i0 += 8 * 64) {  // 8 loads of each in flight
+        int32_t x[8], g[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const int i = i0 + 64 * u;
+            x[u] = i < q.dim ? xr[i] : 0, g[u] = i < q.dim ? q.b[i] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const uint64_t sq = (uint64_t)((int64_t)x[u] * x[u]), t = lo + sq;
+            hi += t < lo, lo = t;
+            pm = max64(pm, iabs((int64_t)x[u] * g[u]));
+        }
+    }
+    add128_row(hi, lo);
+    u128 ss = 0;
+#pragma unroll
+    for (int l = 0; l < 64; l += 16) ss += ((u128)lane64(hi, l) << 64) | lane64(lo, l);
+    pm = wave_max_i64(pm);
+    const Sc xs = uni(rec_sc(q.as)), gs{q.g_mant, q.g_shift}, eps{q.e_mant, q.e_shift};
+    const Sc mean_sq = sc_mul(sc_mul(from_ratio(ss, (u128)q.dim), xs), xs);
+    const Sc denom = sc_add(mean_sq, eps);
+    const Sc cr = sc_mul(sc_mul(xs, denom.mant == 0 ? Sc{0, 0} : sc_rsqrt(denom)), gs);
+    if (lane == 0) rs_crow(q.ws)[r] = cr, rs_pmax(q.ws, q.rows)[r] = pm;
+}
+
+// The largest row factor by the engine's fold (of equal values the latest row's) and the tensor's largest magnitude
+// over it, from the rows' factors and largest products; NT threads of the CTA.
+template <int NT>
+__device__ inline void rs_norm_fold(const RdSeq& q, uint64_t* redk, int64_t* red, Sc& cc, int64_t& gmax) {
+    const Sc* crow = rs_crow(q.ws);
+    const int64_t* pmax = rs_pmax(q.ws, q.rows);
+    FoldKey k{0, 0, 0};
+    for (int r = threadIdx.x; r < q.rows; r += NT) {
+        const FoldKey u = fold_key(ScIdx{crow[r], r});
+        if (fold_gt(u, k)) k = u;
+    }
+    fold_row(k);
+    const int lane = threadIdx.x & 63;
+    if ((lane & 15) == 0) {
+        uint64_t* d = redk + (threadIdx.x >> 4) * 3;
+        d[0] = k.e, d[1] = k.m, d[2] = k.i;
+    }
+    __syncthreads();
+    k = FoldKey{0, 0, 0};
+    for (int i = lane & 15; i < NT / 16; i += 16) {  // the rows of 16 lanes' keys, in every row of every wave
+        const uint64_t* d = redk + i * 3;
+        const FoldKey u{d[0], d[1], d[2]};
+        if (fold_gt(u, k)) k = u;
+    }
+    fold_row(k);
+    cc = fold_item(fold_lane(k, 0)).s;
+    int64_t m = 0;
+    if (cc.mant != 0) {
+        const Sc cinv = sc_recip(cc);
+        for (int r = threadIdx.x; r < q.rows; r += NT) m = max64(m, sc_apply(sc_mul(crow[r], cinv), pmax[r]));
+    }
+    if constexpr (NT == 256) gmax = block_max_4w(m, red);
+    else gmax = block_max_i64(m, red);
+}
+// past RS_FOLD_ROWS rows: the fold by one CTA
+__global__ __launch_bounds__(RD_THREADS) void rs_norm_fold_kernel(RdSeq q) {
+    __shared__ uint64_t redk[3 * RD_THREADS / 16];
+    __shared__ int64_t red[RD_WAVES];
+    Sc cc;
+    int64_t gmax;
+    rs_norm_fold<RD_THREADS>(q, redk, red, cc, gmax);
+    if (threadIdx.x == 0) q.ws->par[0] = cc, q.ws->gmax = (uint64_t)gmax;
+}
+// RMSNorm's second pass: a CTA per row (grid-stride), FOLD: its CTAs fold the rows themselves.
+template <bool FOLD>
+__global__ __launch_bounds__(256) void rs_norm_out_kernel(RdSeq q) {
+    __shared__ uint64_t redk[FOLD ? 3 * 256 / 16 : 1];
+    __shared__ int64_t red[4];
+    Sc cc;
+    int64_t gmax;
+    if constexpr (FOLD) rs_norm_fold<256>(q, redk, red, cc, gmax);
+    else cc = q.ws->par[0], gmax = (int64_t)q.ws->gmax;
+    const RqDen rd_gmax = rq_den(gmax);
+    const Sc cinv = cc.mant != 0 ? sc_recip(cc) : Sc{0, 0};
+    for (int r = blockIdx.x; r < q.rows; r += gridDim.x) {
+        const Sc f = gmax == 0 ? Sc{0, 0} : sc_mul(rs_crow(q.ws)[r], cinv);
+        const size_t at = (size_t)r * q.dim;
+        for (int i = threadIdx.x; i < q.dim; i += 256)
+            q.y[at + i] = gmax == 0 ? 0 : rq_apply(rd_gmax, sc_apply(f, (int64_t)q.a[at + i] * (int64_t)q.b[i]));
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        put_rec(q.ys, gmax == 0 ? Sc{0, 0} : sc_mul(from_ratio((u128)(uint64_t)gmax, (u128)ACT_LEVELS), cc));
 }
 
 // Embedding::lookup_seq (layers.rs:1138-1145): the code rows of T tokens at the table's scale (a token outside the
@@ -1749,14 +1845,31 @@ hipError_t launch_rd_attention_step(const RdAttn& a_in, hipStream_t s) {
     rd_attention_step_kernel<<<1, RD_THREADS, rd_attention_lds(a.max_seq, a.nh, a.hd, a.hb), s>>>(a);
     return hipGetLastError();
 }
-size_t rd_seq_workspace(int64_t rows) { return (sizeof(RdSeqWs) + (size_t)(rows > 1 ? rows - 1 : 0) * sizeof(Sc) + 255) / 256 * 256; }
+size_t rd_seq_workspace(int64_t rows) {
+    return (sizeof(RdSeqWs) + (size_t)rows * (sizeof(Sc) + sizeof(int64_t)) + 255) / 256 * 256;
+}
 
 hipError_t launch_rd_seq(const RdSeq& q, hipStream_t s) {
-    rs_prep_kernel<<<1, RD_THREADS, 0, s>>>(q);
-    const int64_t g = (q.n + 255) / 256;
-    const unsigned grid = (unsigned)(g < 1 ? 1 : (g > 2048 ? 2048 : g));
-    rs_max_kernel<<<grid, 256, 0, s>>>(q);
-    rs_out_kernel<<<grid, 256, 0, s>>>(q);
+    if (q.op == RS_NORM) {
+        const unsigned grid = (unsigned)(q.rows < 1024 ? q.rows : 1024);
+        rs_rows_kernel<<<(unsigned)((q.rows + 3) / 4), 256, 0, s>>>(q);
+        if (q.rows <= RS_FOLD_ROWS) {
+            rs_norm_out_kernel<true><<<grid, 256, 0, s>>>(q);
+        } else {
+            rs_norm_fold_kernel<<<1, RD_THREADS, 0, s>>>(q);
+            rs_norm_out_kernel<false><<<grid, 256, 0, s>>>(q);
+        }
+        return hipGetLastError();
+    }
+    const int64_t g = (q.n + 255) / 256, g4 = (q.n + 1023) / 1024;
+    const unsigned grid = (unsigned)(g > 2048 ? 2048 : g), parts = (unsigned)(g4 > RS_PARTS ? RS_PARTS : g4);  // n >= 1
+    if (q.op == RS_ADD) {
+        rs_max_kernel<RS_ADD><<<parts, 256, 0, s>>>(q);
+        rs_out_kernel<RS_ADD><<<grid, 256, 0, s>>>(q, (int)parts);
+    } else {
+        rs_max_kernel<RS_SWIGLU><<<parts, 256, 0, s>>>(q);
+        rs_out_kernel<RS_SWIGLU><<<grid, 256, 0, s>>>(q, (int)parts);
+    }
     return hipGetLastError();
 }
 
