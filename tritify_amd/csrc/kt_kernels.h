@@ -22,8 +22,8 @@ hipError_t launch_plane_gemm(int px, int pw, const int8_t* xa, const int8_t* wb,
 // The output columns each CTA of launch_plane_gemm covers (segment boundaries must be multiples of it).
 int plane_gemm_cta_cols(int px, int pw, int M, int N);
 // How many runs of k the digit-plane GEMM of [k0, k1) splits into (1 unless its tiles leave CUs idle); a split
-// launch needs y zeroed, one zeroed counter per tile (the grid's tiles: at most 128) and accumulate = 0.
-int plane_gemm_splits(int px, int pw, int M, int N, int k0, int k1);
+// launch needs y zeroed, one zeroed counter per tile (at most one per 32 x 64 outputs, and 256) and accumulate = 0.
+int plane_gemm_splits(int px, int pw, int M, int N, int kp, int k0, int k1, const QlSeg& seg);
 hipError_t launch_w12b_pack(const int32_t* codes, int64_t n, int64_t k, int8_t* lo, int8_t* hi, hipStream_t s);
 hipError_t launch_stream_read(const uint8_t* src, uint32_t bytes, uint32_t* out, hipStream_t s);
 hipError_t launch_w12b_linear(const int8_t* x, const int8_t* lo, const int8_t* hi, int M, int N, int kp,

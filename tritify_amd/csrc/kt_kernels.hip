@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "kt_kernels.h"
+#include "kt_plane_dma.h"
 #include "kt_w12_core.h"
 
 namespace kt {
@@ -1191,10 +1192,59 @@ static int64_t plane_gemm_shape(int px, int pw, int M, int N, int& wtm, int& wtn
     return ceil_div(N, 64 * wtn) * ceil_div(M, 64 * wtm);
 }
 
-int plane_gemm_splits(int px, int pw, int M, int N, int k0, int k1) {
+// Whether the device gives a CTA the DMA-fed plane kernel's ring; queried once per process.
+static bool plane_dma_lds_ok() {
+    static int ok = -1;
+    if (ok < 0) {
+        hipFuncAttributes fa;
+        int dev = 0, mx = 0;
+        ok = hipGetDevice(&dev) == hipSuccess &&
+             hipDeviceGetAttribute(&mx, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
+             hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&plane_dma_kernel<PlaneTile32>)) == hipSuccess &&
+             fa.sharedSizeBytes + (size_t)PlaneTile32::LDS <= (size_t)mx;
+    }
+    return ok == 1;
+}
+
+// The tile of the DMA-fed plane kernel for a product: 0 = the general kernel, else the rows * 1000 + columns of a tile.
+// It takes 3 x 3 planes of more rows than the skinny kernel where its 32-bit offsets hold (16 rows of k, 64 rows of
+// y). Columns per tile divide every segment boundary. 64 x 128 tiles from 1024 64 x 64 tiles on (4 per CU), where
+// their longer steps are filled, unless the columns they waste outweigh their lower cost per output (0.88 against 0.635
+// us a k-tile and CU; N = 64); 32 x 64 up to 128 64 x 64 tiles, half the chip (256 x 1152, k 896, 72 tiles: 8.4 us
+// against 9.7; but 1000 x 900, k 832, 240 tiles: 16.0 against 13.2); 64 x 64 between (4096 x 448, k 1792, 448 tiles:
+// 36.9 us against 41.0 with 64 x 128).
+static int plane_dma_shape(int px, int pw, int M, int N, int kp, const QlSeg& seg) {
+    if (px != 3 || pw != 3 || M <= KT_PLANE_SKINNY_M || kp > (1 << 24) || N > (1 << 22) || !plane_dma_lds_ok())
+        return 0;
+    bool c64 = true, c128 = true;
+    for (int g = 1; g < seg.n; g++) c64 = c64 && seg.col0[g] % 64 == 0, c128 = c128 && seg.col0[g] % 128 == 0;
+    if (!c64) return 0;
+    const int64_t n64 = ceil_div(N, 64) * ceil_div(M, 64), n128 = ceil_div(N, 128) * ceil_div(M, 64);
+    if (n64 >= 1024 && c128 && n128 * 880 < n64 * 635) return 64128;
+    return n64 <= 128 ? 32064 : 64064;
+}
+
+// k over several CTAs of the 32 x 64 tile: each k-tile of a CTA takes about 0.32 us there, the split costs an atomic
+// pass per share over the M x N sums (7 us a million) and about 1 us of hand-off, and must fit one CTA per CU.
+// 256 x 896, k 4864: 27.4 -> 20.1 us; 27 x 896, k 3584: 20.2 -> 9.0; 17 x 4864, k 896: left whole (7.9 against 8.5).
+static int plane_dma_splits(int M, int N, int nk) {
+    const int64_t tiles = ceil_div(N, 64) * ceil_div(M, 32), mn = (int64_t)M * N;
+    int best = 1;
+    int64_t cost = 320 * (int64_t)nk;  // ns
+    for (int s = 2; s <= 4 && s <= nk && tiles * s <= 256; s *= 2) {
+        const int64_t c = 320 * (int64_t)((nk + s - 1) / s) + 1000 + mn * s * 7 / 1000;
+        if (c < cost) cost = c, best = s;
+    }
+    const int per = (nk + best - 1) / best;
+    return (nk + per - 1) / per;  // every run of k-tiles is non-empty
+}
+
+int plane_gemm_splits(int px, int pw, int M, int N, int kp, int k0, int k1, const QlSeg& seg) {
+    const int nk = (k1 - k0) / 64;
+    const int dma = plane_dma_shape(px, pw, M, N, kp, seg);
+    if (dma) return dma == 32064 && nk > 0 ? plane_dma_splits(M, N, nk) : 1;
     int wtm, wtn;
     const int64_t tiles = plane_gemm_shape(px, pw, M, N, wtm, wtn);
-    const int nk = (k1 - k0) / 64;
     // the split costs atomic passes over the M x N outputs: worth it for long k (down: 76 k-tiles) or one row tile
     // (decode), not for short k over many rows (N = 896 at M = 512, K = 896: measured slower)
     if (M <= KT_PLANE_SKINNY_M || tiles >= 128 || nk < 2 || (nk < 24 && M > 64)) return 1;  // a few rows: skinny
@@ -1228,6 +1278,19 @@ static hipError_t plane_gemm_px_pw(const int8_t* xa, const int8_t* wb, int64_t* 
                                                                                      ql, seg);
         return hipGetLastError();
     }
+    if constexpr (PX == 3 && PW == 3) {
+        const int dma = plane_dma_shape(PX, PW, M, N, kp, seg);
+        const auto run = [&](auto tile) {
+            typedef decltype(tile) C;
+            const dim3 grid((unsigned)(ceil_div(N, C::BN) * ceil_div(M, C::BM)), (unsigned)splits);
+            plane_dma_kernel<C><<<grid, dim3(C::NT), C::LDS, s>>>(xa, wb, y, M, N, kp, k0, k1, accumulate, drop_top,
+                                                                  ql_bias, ql, cnt, seg);
+            return hipGetLastError();
+        };
+        if (dma == 64128) return run(PlaneTile128{});
+        if (dma == 64064) return run(PlaneTile64{});
+        if (dma == 32064) return run(PlaneTile32{});
+    }
     int wtm, wtn;
     const int64_t tiles = plane_gemm_shape(PX, PW, M, N, wtm, wtn);
     const dim3 grid((unsigned)tiles, (unsigned)splits);
@@ -1249,7 +1312,7 @@ hipError_t launch_plane_gemm(int px, int pw, const int8_t* xa, const int8_t* wb,
     if (sg.n < 1 || sg.n > KT_QL_MAX_SEG) return hipErrorInvalidValue;
     if (M <= 0 || N <= 0 || k1 <= k0) return hipSuccess;
     if ((k0 % 64) || (k1 % 64) || k1 > kp || ceil_div(M, 64) * ceil_div(N, 64) > INT32_MAX) return hipErrorInvalidValue;
-    if (splits != 1 && (splits != plane_gemm_splits(px, pw, M, N, k0, k1) || !tile_cnt || accumulate))
+    if (splits != 1 && (splits != plane_gemm_splits(px, pw, M, N, kp, k0, k1, sg) || !tile_cnt || accumulate))
         return hipErrorInvalidValue;
 #define KT_CASE(a, b) \
     if (px == a && pw == b)                                                                                  \

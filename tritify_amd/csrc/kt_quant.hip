@@ -628,9 +628,9 @@ static hipError_t launch_ql_impl(const int32_t* x, int64_t rows, int64_t in, con
     const int64_t kp = (in + 63) / 64 * 64, n = rows * out;
     const int64_t nx = geom ? (int64_t)geom->ci * geom->h * geom->w : rows * in;
     // one k-chunk whose tiles leave CUs idle (the decode row, N = 896 at M = 512): split k across CTAs
-    const int splits = kp <= flush_k ? plane_gemm_splits(3, pw, (int)rows, (int)out, 0, (int)kp) : 1;
-    const int ntiles = splits > 1 ? (int)(((out + 63) / 64) * ((rows + 63) / 64)) : 0;
-    if (ntiles * 4 > KT_QL_PARTS * 8) return hipErrorInvalidValue;  // cannot happen: a split grid has < 128 tiles
+    const int splits = kp <= flush_k ? plane_gemm_splits(3, pw, (int)rows, (int)out, (int)kp, 0, (int)kp, seg) : 1;
+    const int ntiles = splits > 1 ? (int)(((out + 63) / 64) * ((rows + 31) / 32)) : 0;
+    if (ntiles * 4 > KT_QL_PARTS * 8) return hipErrorInvalidValue;  // cannot happen: a split grid has <= 256 tiles
 
     // one row within one k-chunk (the decode step): the quant pass inside the product, then the requant pass
     if (!geom && rows == 1 && ql_sums_ok(in, out, pw, flush_k) && ql_seg_cols_ok(seg)) {
