@@ -92,3 +92,33 @@ def test_add_and_swiglu_seq_edges(torch_dev, n):
             B.ref_swiglu_seq(*args, w, nw, h, hs) if seq else B.ref_swiglu(*args, h, hs)
             out.append((h.cpu().numpy(), rd(hs)))
         assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1], gshift
+
+
+@pytest.mark.parametrize("nh,nkv,hd,T", [(14, 2, 64, 2), (14, 2, 64, 5), (4, 4, 64, 64), (6, 2, 64, 67), (2, 1, 128, 131),
+                                         (4, 2, 96, 66), (1, 1, 64, 300), (2, 1, 64, 2050)])
+@pytest.mark.parametrize("mag", [2**20, 2**28])
+def test_attention_prefill_edges(torch_dev, nh, nkv, hd, T, mag):
+    """The prefill attention where its row groups, lane blocks and runs end: rows that do not fill a group of four,
+    blocks of 64 cached rows with one more and one less, one row per CTA past 2048, each head dimension's kernel."""
+    torch = torch_dev
+    from tritify_amd import backend as B
+
+    print(f"case: attention_prefill nh={nh} nkv={nkv} hd={hd} T={T} mag={mag}", file=sys.stderr, flush=True)
+    rng = np.random.default_rng(nh * 100 + T + hd)
+    model = O.RefModel(3, dict(dim=nh * hd, layers=1, nh=nh, nkv=nkv, hd=hd, hidden=8, vocab=2, eps=1e-6, theta=10000.0,
+                               max_seq=T))
+    q, k, v = (rng.integers(-mag, mag + 1, size=T * n * hd).astype(np.int32) for n in (nh, nkv, nkv))
+    v[:hd] = 0  # row 0 of the first head attends to zeros alone
+    # score scales spread so the softmax is neither flat nor one-hot
+    qs, ks, vs = (int(rng.integers(2**30, 2**31)), 81 if mag == 2**28 else 65), rand_scale(rng), rand_scale(rng)
+    want, wsc = model.attention_prefill(T, q, qs, k, ks, v, vs)
+    cos_t, sin_t = B.ref_rope_tables(T, hd, 10000.0)
+    ec, lut = B.ref_codelut(B.LUT_EXP, -30.0, 0.0, 16, 20, False)
+    n = B.ref_attention_prefill_workspace(T, nh, nkv, hd)
+    w = torch.full((n,), 0xA5, dtype=torch.uint8, device="cuda")
+    o, os_ = torch.zeros(T * nh * hd, dtype=torch.int32, device="cuda"), rec(torch, (0, 0))
+    B.ref_attention_prefill(dev(torch, q), rec(torch, qs), dev(torch, k), rec(torch, ks), dev(torch, v), rec(torch, vs),
+                            T, nh, nkv, hd, T, torch.from_numpy(cos_t.view(np.uint8)).cuda(),
+                            torch.from_numpy(sin_t.view(np.uint8)).cuda(), B.ref_scale_from_f64(1.0 / np.sqrt(hd)),
+                            torch.from_numpy(ec).cuda(), lut, w, n, o, os_)
+    assert np.array_equal(o.cpu().numpy(), want) and rd(os_) == wsc

@@ -25,6 +25,8 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "kt_dpp.h"
 #include "kt_kernels.h"
 #include "kt_scale_dev.h"
@@ -85,9 +87,9 @@ struct RdPrefill {
     const int64_t* exp_codes;
     kt_hip_codelut exp;
     int32_t *qd, *kd;                  // rotated q and k
-    int64_t* hout;                     // [nh][T][hd]: the sums of numerator * v, then the outputs at the common scale
-    int64_t* hsum;                     // [nh][T]: the numerators' sums
-    Sc* fac;                           // [T][nh]: each (row, head)'s scale over the common one
+    int64_t* hout;                     // [T][nh][hd]: the sums of numerator * v
+    int64_t* hmax;                     // [T][nh]: each (row, head)'s largest |sum of numerator * v|
+    Sc* fac;                           // [T][nh]: each (row, head)'s scale
     uint64_t* gmax;                    // the largest |output| at the common scale
     Sc* common;
     int32_t* o;                        // T x nh*hd
@@ -1507,15 +1509,14 @@ __global__ __launch_bounds__(256) void rs_rows_kernel(RdSeq q) {
     if (lane == 0) rs_crow(q.ws)[r] = cr, rs_pmax(q.ws, q.rows)[r] = pm;
 }
 
-// The largest row factor by the engine's fold (of equal values the latest row's) and the tensor's largest magnitude
-// over it, from the rows' factors and largest products; NT threads of the CTA.
+// The largest of n Scales by the engine's fold over their order (of equal values the latest), and the largest
+// magnitude at that scale of the groups they scale, pmax holding each group's largest |value|; NT threads of the CTA.
 template <int NT>
-__device__ inline void rs_norm_fold(const RdSeq& q, uint64_t* redk, int64_t* red, Sc& cc, int64_t& gmax) {
-    const Sc* crow = rs_crow(q.ws);
-    const int64_t* pmax = rs_pmax(q.ws, q.rows);
+__device__ inline void scale_fold(const Sc* scale, const int64_t* pmax, int n, uint64_t* redk, int64_t* red, Sc& cc,
+                                  int64_t& gmax) {
     FoldKey k{0, 0, 0};
-    for (int r = threadIdx.x; r < q.rows; r += NT) {
-        const FoldKey u = fold_key(ScIdx{crow[r], r});
+    for (int r = threadIdx.x; r < n; r += NT) {
+        const FoldKey u = fold_key(ScIdx{scale[r], r});
         if (fold_gt(u, k)) k = u;
     }
     fold_row(k);
@@ -1536,7 +1537,7 @@ __device__ inline void rs_norm_fold(const RdSeq& q, uint64_t* redk, int64_t* red
     int64_t m = 0;
     if (cc.mant != 0) {
         const Sc cinv = sc_recip(cc);
-        for (int r = threadIdx.x; r < q.rows; r += NT) m = max64(m, sc_apply(sc_mul(crow[r], cinv), pmax[r]));
+        for (int r = threadIdx.x; r < n; r += NT) m = max64(m, sc_apply(sc_mul(scale[r], cinv), pmax[r]));
     }
     if constexpr (NT == 256) gmax = block_max_4w(m, red);
     else gmax = block_max_i64(m, red);
@@ -1547,7 +1548,7 @@ __global__ __launch_bounds__(RD_THREADS) void rs_norm_fold_kernel(RdSeq q) {
     __shared__ int64_t red[RD_WAVES];
     Sc cc;
     int64_t gmax;
-    rs_norm_fold<RD_THREADS>(q, redk, red, cc, gmax);
+    scale_fold<RD_THREADS>(rs_crow(q.ws), rs_pmax(q.ws, q.rows), q.rows, redk, red, cc, gmax);
     if (threadIdx.x == 0) q.ws->par[0] = cc, q.ws->gmax = (uint64_t)gmax;
 }
 // RMSNorm's second pass: a CTA per row (grid-stride), FOLD: its CTAs fold the rows themselves.
@@ -1557,7 +1558,7 @@ __global__ __launch_bounds__(256) void rs_norm_out_kernel(RdSeq q) {
     __shared__ int64_t red[4];
     Sc cc;
     int64_t gmax;
-    if constexpr (FOLD) rs_norm_fold<256>(q, redk, red, cc, gmax);
+    if constexpr (FOLD) scale_fold<256>(rs_crow(q.ws), rs_pmax(q.ws, q.rows), q.rows, redk, red, cc, gmax);
     else cc = q.ws->par[0], gmax = (int64_t)q.ws->gmax;
     const RqDen rd_gmax = rq_den(gmax);
     const Sc cinv = cc.mant != 0 ? sc_recip(cc) : Sc{0, 0};
@@ -1585,15 +1586,14 @@ __global__ __launch_bounds__(256) void rd_embed_seq_kernel(const int32_t* __rest
     if (blockIdx.x == 0 && threadIdx.x == 0) put_rec(ys, Sc{e_mant, e_shift});
 }
 
-// Attention::forward_int (attention.rs:467-598) in five launches:
+// Attention::forward_int (attention.rs:467-598) in four launches:
 //  rp_rope    q and k of row i rotated at position i (rope_int, attention.rs:208-229)
-//  rp_head    one CTA per (head, row i): the causal dots j <= i (exact, wrapping i64) at the one score scale
+//  rp_head    per (head, row i): the causal dots j <= i (exact, wrapping i64) at the one score scale
 //             q.scale * k.scale * inv_sqrt, the exp-CodeLut numerators of (dot - max), their sum, the sums of
-//             numerator * v over the rows
-//  rp_common  one CTA: each (row, head)'s scale v.scale / sumc, the largest by the engine's fold over the
-//             [row][head] order, every scale over it
-//  rp_apply   the outputs brought to the common scale, their largest magnitude
-//  rp_out     requant_dyn, and the output's scale
+//             numerator * v over the rows, their largest magnitude, the scale v.scale / sum
+//  rp_fold    one CTA: the largest scale by the engine's fold over the [row][head] order, and the largest magnitude at
+//             that scale, from each (row, head)'s largest sum (Scale::apply keeps order: scale_fold)
+//  rp_out     the outputs brought to the common scale and requantized, and their record
 __global__ __launch_bounds__(256) void rp_rope_kernel(RdPrefill a) {
     const int i = blockIdx.x, half = a.hd / 2, qw = a.nh * a.hd, kw = a.nkv * a.hd;
     for (int e = threadIdx.x; e < (a.nh + a.nkv) * half; e += 256) {
@@ -1609,19 +1609,163 @@ __global__ __launch_bounds__(256) void rp_rope_kernel(RdPrefill a) {
     }
 }
 
+// The score table's index factor: q.scale * k.scale * inv_sqrt * inv_step.
+__device__ inline Sc rp_index_factor(const RdPrefill& a) {
+    const Sc s_score = sc_mul(sc_mul(uni(rec_sc(a.qs)), uni(rec_sc(a.ks))), Sc{a.isq_mant, a.isq_shift});
+    return sc_mul(s_score, Sc{a.exp.inv_mant, a.exp.inv_shift});
+}
+
+// Head dimensions of 64 and 128: R rows of a head per CTA of 4 waves. The dots are 64-bit multiply-adds of one lane per
+// cached row: the lane holds its k row in registers (16-byte loads) and meets each of the R q rows, whose values are
+// wave-uniform and come through scalar registers; the waves take every fourth block of 64 cached rows. For the sums
+// of numerator * v the lanes are the head's dimensions, a numerator is one LDS broadcast, and the waves take every
+// fourth run of 8 rows. Bound by those multiply-adds (about half of the 28 us at 256 rows), R of them per k or v value
+// read. 256 rows, 14 heads of 64: 41.6 -> 27.9 us against one row per CTA with a strided 4-byte k load per product
+// (the whole op 69.4 -> 46.0; at 2048 rows 2045 -> 868).
+template <int HD, int R>
 __global__ __launch_bounds__(256) void rp_head_kernel(RdPrefill a) {
+    typedef const __attribute__((address_space(4))) int32_t* const_i32;  // read through scalar loads
+    constexpr int ND = HD / 64;
+    extern __shared__ int64_t S[];  // [R][T]: the dots, then the numerators
+    __shared__ int64_t red[R][4];
+    __shared__ int64_t part[4][R][HD];
+    const int T = a.T, nb = (T + R - 1) / R, h = (int)blockIdx.x / nb, kv = h / (a.nh / a.nkv), kw = a.nkv * HD;
+    const int i0 = (nb - 1 - (int)blockIdx.x % nb) * R;  // the longest rows first
+    const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+    const int nr = T - i0 < R ? T - i0 : R, jend = i0 + nr;  // rows of this CTA; cached rows any of them attends
+    int64_t m[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) m[r] = INT64_MIN;
+    for (int t0 = 64 * w; t0 < jend; t0 += 256) {
+        const int j = t0 + lane, jc = j < T ? j : T - 1;
+        const v4i* kr = reinterpret_cast<const v4i*>(a.kd + (size_t)jc * kw + kv * HD);
+        v4i k[HD / 4];
+#pragma unroll
+        for (int c = 0; c < HD / 4; c++) k[c] = kr[c];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (r >= nr) break;  // uniform
+            const const_i32 q = (const_i32)(uint64_t)(a.qd + ((size_t)(i0 + r) * a.nh + h) * HD);
+            int64_t dot = 0;
+#pragma unroll
+            for (int d = 0; d < HD; d++) dot = wadd(dot, (int64_t)q[d] * (int64_t)k[d >> 2][d & 3]);
+            if (j <= i0 + r) {
+                S[r * T + j] = dot;
+                m[r] = max64(m[r], dot);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        m[r] = wave_max_i64(m[r]);
+        if (lane == 0) red[r][w] = m[r];
+    }
+    const Sc lm = rp_index_factor(a);
+    __syncthreads();
+    int64_t sum[R], dmax[R];
+    bool wide = false;  // a numerator past 31 bits (no table of 2^20 codes has one)
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        dmax[r] = max64(max64(red[r][0], red[r][1]), max64(red[r][2], red[r][3]));
+        sum[r] = 0;
+    }
+    for (int j = tid; j < jend; j += 256) {  // the rows' table reads in flight together
+        int64_t c[R], idx[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const bool on = r < nr && j <= i0 + r;
+            const int64_t dot = on ? S[r * T + j] : dmax[r];
+            idx[r] = on ? lut_index(lm, (int64_t)((uint64_t)dot - (uint64_t)dmax[r]), a.exp.lo_index) : -1;
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) c[r] = lut_code(a.exp_codes, a.exp.n, idx[r]);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (idx[r] < 0) c[r] = 0;
+            if (r < nr) S[r * T + j] = c[r];  // zero past the row's own position
+            sum[r] = wadd(sum[r], c[r]);
+            wide = wide || ((uint64_t)c[r] >> 31) != 0;
+        }
+    }
+    wide = __syncthreads_or(wide);  // also orders the reads of red before its next writes
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        sum[r] = (int64_t)wave_sum_u64((uint64_t)sum[r]);
+        if (lane == 0) red[r][w] = sum[r];
+    }
+    int64_t acc[R][ND];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int e = 0; e < ND; e++) acc[r][e] = 0;
+    auto weigh = [&](auto narrow) {
+        int32_t v[8][ND], vn[8][ND];
+        auto fetch = [&](int j0, int32_t(&x)[8][ND]) {  // rows past the last read it again, with zero numerators
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int e = 0; e < ND; e++)
+                    x[u][e] = a.v[(size_t)(j0 + u < T ? j0 + u : T - 1) * kw + kv * HD + 64 * e + lane];
+        };
+        fetch(8 * w, vn);
+        for (int j0 = 8 * w; j0 < jend; j0 += 32) {
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int e = 0; e < ND; e++) v[u][e] = vn[u][e];
+            fetch(j0 + 32, vn);  // under this run's products
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (r >= nr) break;  // uniform
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const int64_t s = j0 + u < jend ? S[r * T + j0 + u] : 0;
+#pragma unroll
+                    for (int e = 0; e < ND; e++) {
+                        if constexpr (decltype(narrow)::value)
+                            acc[r][e] = wadd(acc[r][e], (int64_t)(int32_t)s * (int64_t)v[u][e]);
+                        else
+                            acc[r][e] = wadd(acc[r][e], wmul(s, v[u][e]));
+                    }
+                }
+            }
+        }
+    };
+    if (wide) weigh(std::false_type{});
+    else weigh(std::true_type{});
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int e = 0; e < ND; e++) part[w][r][64 * e + lane] = acc[r][e];
+    __syncthreads();
+    if (w >= nr) return;  // wave r finishes row r (R <= 4)
+    const size_t ih = (size_t)(i0 + w) * a.nh + h;
+    const int64_t sumc = wadd(wadd(red[w][0], red[w][1]), wadd(red[w][2], red[w][3]));
+    int64_t pm = 0;
+#pragma unroll
+    for (int e = 0; e < ND; e++) {
+        const int d = 64 * e + lane;
+        int64_t t = wadd(wadd(part[0][w][d], part[1][w][d]), wadd(part[2][w][d], part[3][w][d]));
+        if (sumc <= 0) t = 0;
+        a.hout[ih * HD + d] = t;
+        pm = max64(pm, iabs(t));
+    }
+    pm = wave_max_i64(pm);
+    const int64_t su = uni64(sumc);
+    const Sc sc = su > 0 ? sc_mul(uni(rec_sc(a.vs)), from_ratio(1, (u128)(uint64_t)su)) : Sc{0, 0};
+    if (lane == 0) a.hmax[ih] = pm, a.fac[ih] = sc;
+}
+
+// Any other head dimension (up to 256): a CTA per (head, row).
+__global__ __launch_bounds__(256) void rp_head_any_kernel(RdPrefill a) {
     extern __shared__ int64_t S[];  // T: the dots, then the numerators
     __shared__ int64_t red[4];
     __shared__ int64_t part[256];
     __shared__ int32_t qrow[256];
-    __shared__ Sc lm_s;
     const int h = blockIdx.x / a.T, i = blockIdx.x % a.T, hd = a.hd, kv = h / (a.nh / a.nkv);
     const int kw = a.nkv * a.hd, tid = threadIdx.x;
     for (int d = tid; d < hd; d += 256) qrow[d] = a.qd[(size_t)i * a.nh * hd + h * hd + d];
-    if (tid == 0) {
-        const Sc s_score = sc_mul(sc_mul(rec_sc(a.qs), rec_sc(a.ks)), Sc{a.isq_mant, a.isq_shift});
-        lm_s = sc_mul(s_score, Sc{a.exp.inv_mant, a.exp.inv_shift});
-    }
+    const Sc lm = rp_index_factor(a);
     __syncthreads();
     int64_t m = INT64_MIN;
     for (int j = tid; j <= i; j += 256) {
@@ -1632,7 +1776,6 @@ __global__ __launch_bounds__(256) void rp_head_kernel(RdPrefill a) {
         m = dot > m ? dot : m;
     }
     const int64_t dmax = block_max_4w(m, red);
-    const Sc lm = lm_s;
     int64_t sum = 0;
     for (int j = tid; j <= i; j += 256) {
         const int64_t idx = lut_index(lm, (int64_t)((uint64_t)S[j] - (uint64_t)dmax), a.exp.lo_index);
@@ -1646,59 +1789,40 @@ __global__ __launch_bounds__(256) void rp_head_kernel(RdPrefill a) {
         for (int j = gq; j <= i; j += groups) acc = wadd(acc, wmul(S[j], a.v[(size_t)j * kw + kv * hd + d]));
     part[tid] = acc;
     __syncthreads();
+    const size_t ih = (size_t)i * a.nh + h;
+    int64_t t = 0;
     if (tid < hd) {
-        int64_t t = 0;
         for (int q = 0; q < groups; q++) t = wadd(t, part[q * hd + tid]);
-        a.hout[((size_t)h * a.T + i) * hd + tid] = sumc > 0 ? t : 0;
+        t = sumc > 0 ? t : 0;
+        a.hout[ih * hd + tid] = t;
     }
-    if (tid == 0) a.hsum[(size_t)h * a.T + i] = sumc > 0 ? sumc : 0;
+    const int64_t pm = block_max_4w(iabs(t), red);
+    if (tid == 0) {
+        a.hmax[ih] = pm;
+        a.fac[ih] = sumc > 0 ? sc_mul(rec_sc(a.vs), from_ratio(1, (u128)(uint64_t)sumc)) : Sc{0, 0};
+    }
 }
 
-__global__ __launch_bounds__(RD_THREADS) void rp_common_kernel(RdPrefill a) {
-    __shared__ ScIdx redsc[RD_THREADS];
-    const int n = a.T * a.nh;
-    const Sc vs = rec_sc(a.vs);
-    ScIdx best{Sc{0, 0}, -1};
-    for (int e = threadIdx.x; e < n; e += RD_THREADS) {
-        const int i = e / a.nh, h = e - i * a.nh;
-        const int64_t sumc = a.hsum[(size_t)h * a.T + i];
-        const Sc sc = sumc > 0 ? sc_mul(vs, from_ratio(1, (u128)(uint64_t)sumc)) : Sc{0, 0};
-        a.fac[e] = sc;
-        best = sc_pick(best, ScIdx{sc, e});
-    }
-    const Sc common = block_fold_max(best, redsc, n).s;  // its barriers order the fac writes before the reads
-    if (common.mant != 0) {
-        const Sc cinv = sc_recip(common);
-        for (int e = threadIdx.x; e < n; e += RD_THREADS) a.fac[e] = sc_mul(a.fac[e], cinv);
-    }
-    if (threadIdx.x == 0) *a.common = common, *a.gmax = 0;
+__global__ __launch_bounds__(RD_THREADS) void rp_fold_kernel(RdPrefill a) {
+    __shared__ uint64_t redk[3 * RD_THREADS / 16];
+    __shared__ int64_t red[RD_WAVES];
+    Sc common;
+    int64_t gmax;
+    scale_fold<RD_THREADS>(a.fac, a.hmax, a.T * a.nh, redk, red, common, gmax);
+    if (threadIdx.x == 0) *a.common = common, *a.gmax = (uint64_t)gmax;
 }
 
-__global__ __launch_bounds__(256) void rp_apply_kernel(RdPrefill a) {
-    __shared__ int64_t red[4];
-    const int64_t n = (int64_t)a.T * a.nh * a.hd;
-    const bool live = a.common->mant != 0;
-    int64_t m = 0;
-    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; live && e < n; e += (int64_t)gridDim.x * 256) {
-        const int64_t hi = e / a.hd, h = hi / a.T, i = hi - h * a.T;  // e indexes hout[h][i][d]
-        const int64_t v = sc_apply(a.fac[i * a.nh + h], a.hout[e]);
-        a.hout[e] = v;
-        m = iabs(v) > m ? iabs(v) : m;
-    }
-    m = block_max_4w(m, red);
-    if (threadIdx.x == 0 && m > 0) atomicMax(reinterpret_cast<unsigned long long*>(a.gmax), (unsigned long long)m);
-}
-
-__global__ __launch_bounds__(256) void rp_out_kernel(RdPrefill a) {
+__global__ __launch_bounds__(256) void rp_out_kernel(RdPrefill a) {  // a wave per (row, head)
     const int64_t gmax = (int64_t)*a.gmax;
     const RqDen rd_gmax = rq_den(gmax);
-    const Sc common = *a.common;
+    const Sc common = uni(*a.common);
     const bool live = common.mant != 0 && gmax > 0;
-    const int qw = a.nh * a.hd;
-    const int64_t n = (int64_t)a.T * qw;
-    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
-        const int64_t i = e / qw, r = e - i * qw, h = r / a.hd, d = r - h * a.hd;  // e indexes o[i][h][d]
-        a.o[e] = live ? rq_apply(rd_gmax, a.hout[((size_t)h * a.T + i) * a.hd + d]) : 0;
+    const int ih = (int)blockIdx.x * 4 + wave_id();
+    if (ih < a.T * a.nh) {  // the whole wave
+        const Sc f = live ? sc_mul(uni(a.fac[ih]), sc_recip(common)) : Sc{0, 0};
+        const size_t at = (size_t)ih * a.hd;
+        for (int d = threadIdx.x & 63; d < a.hd; d += 64)
+            a.o[at + d] = live ? rq_apply(rd_gmax, sc_apply(f, a.hout[at + d])) : 0;
     }
     if (blockIdx.x == 0 && threadIdx.x == 0)
         put_rec(a.os, live ? sc_mul(from_ratio((u128)(uint64_t)gmax, (u128)ACT_LEVELS), common) : Sc{0, 0});
@@ -1881,7 +2005,7 @@ hipError_t launch_rd_embed_seq(const int32_t* emb, int64_t e_mant, int32_t e_shi
     return hipGetLastError();
 }
 
-// The prefill attention's workspace: rotated q and k, the head sums, the numerators' sums, the factors, gmax and
+// The prefill attention's workspace: rotated q and k, the head sums, their largest magnitudes, the scales, gmax and
 // the common scale, each part 256-byte aligned.
 size_t rd_prefill_workspace(int64_t T, int64_t nh, int64_t nkv, int64_t hd, size_t off[7]) {
     const size_t sizes[7] = {(size_t)(T * nh * hd * 4), (size_t)(T * nkv * hd * 4), (size_t)(nh * T * hd * 8),
@@ -1899,15 +2023,24 @@ hipError_t launch_rd_attention_prefill(RdPrefill a, void* ws, hipStream_t s) {
     rd_prefill_workspace(a.T, a.nh, a.nkv, a.hd, off);
     char* b = (char*)ws;
     a.qd = (int32_t*)(b + off[0]), a.kd = (int32_t*)(b + off[1]), a.hout = (int64_t*)(b + off[2]);
-    a.hsum = (int64_t*)(b + off[3]), a.fac = (Sc*)(b + off[4]), a.gmax = (uint64_t*)(b + off[5]);
+    a.hmax = (int64_t*)(b + off[3]), a.fac = (Sc*)(b + off[4]), a.gmax = (uint64_t*)(b + off[5]);
     a.common = (Sc*)(b + off[6]);
     rp_rope_kernel<<<(unsigned)a.T, 256, 0, s>>>(a);
-    rp_head_kernel<<<(unsigned)(a.T * a.nh), 256, (size_t)a.T * 8, s>>>(a);
-    rp_common_kernel<<<1, RD_THREADS, 0, s>>>(a);
-    const int64_t n = (int64_t)a.T * a.nh * a.hd, g = (n + 255) / 256;
-    const unsigned grid = (unsigned)(g < 1 ? 1 : (g > 2048 ? 2048 : g));
-    rp_apply_kernel<<<grid, 256, 0, s>>>(a);
-    rp_out_kernel<<<grid, 256, 0, s>>>(a);
+    // R rows of dots in 64 KB of LDS: 4 rows up to 2048 positions, one beyond
+    const unsigned ctas4 = (unsigned)((a.T + 3) / 4 * a.nh), ctas1 = (unsigned)(a.T * a.nh);
+    const size_t lds = (size_t)a.T * 8;
+    const bool four = a.T <= 2048;
+    if (a.hd == 64) {
+        if (four) rp_head_kernel<64, 4><<<ctas4, 256, 4 * lds, s>>>(a);
+        else rp_head_kernel<64, 1><<<ctas1, 256, lds, s>>>(a);
+    } else if (a.hd == 128) {
+        if (four) rp_head_kernel<128, 4><<<ctas4, 256, 4 * lds, s>>>(a);
+        else rp_head_kernel<128, 1><<<ctas1, 256, lds, s>>>(a);
+    } else {
+        rp_head_any_kernel<<<ctas1, 256, lds, s>>>(a);
+    }
+    rp_fold_kernel<<<1, RD_THREADS, 0, s>>>(a);
+    rp_out_kernel<<<(unsigned)((a.T * a.nh + 3) / 4), 256, 0, s>>>(a);
     return hipGetLastError();
 }
 
