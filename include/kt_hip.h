@@ -123,6 +123,22 @@ int kt_hip_quant_linear_multi(int dev, const int32_t* x_dev, int64_t rows, int64
                               const int* has_bias, const int64_t* b_mant, const int32_t* b_shift, void* ws_dev,
                               size_t ws_bytes, int32_t* const* y_devs, kt_hip_qscale* os_dev, void* stream);
 int64_t kt_hip_quant_linear_multi_align(int64_t rows, int64_t out_f, int pw);
+/* kt_hip_quant_linear_multi with what the caller knows of max |x|, which then takes no pass over x:
+ *   KT_QL_X_ANY     nothing (kt_hip_quant_linear_multi itself);
+ *   KT_QL_X_CLOSED  x is the whole output of one op that closes with requant_dyn (RMSNorm, SwiGLU, the attention, add)
+ *                   with its record in xs_dev: its largest |code| is 2^28, or every code is 0 at Scale::ZERO. A part of
+ *                   such an output, or a changed one, is KT_QL_X_ANY;
+ *   KT_QL_X_PARTS   xmax_dev holds KT_QL_PARTS values whose largest is max |x| (kt_hip_quant_linear_gelu's ymax_dev).
+ * xmax_dev is read for KT_QL_X_PARTS only. Same integers as kt_hip_quant_linear_multi. */
+#define KT_QL_X_ANY 0
+#define KT_QL_X_CLOSED 1
+#define KT_QL_X_PARTS 2
+int kt_hip_quant_linear_multi_x(int dev, const int32_t* x_dev, int64_t rows, int64_t in_f, const kt_hip_qscale* xs_dev,
+                                int x_kind, const uint32_t* xmax_dev, int nseg, const int64_t* seg_out,
+                                const int8_t* w_planes_dev, int pw, const int64_t* w_mant, const int32_t* w_shift,
+                                const int64_t* bias_dev, const int* has_bias, const int64_t* b_mant,
+                                const int32_t* b_shift, void* ws_dev, size_t ws_bytes, int32_t* const* y_devs,
+                                kt_hip_qscale* os_dev, void* stream);
 /* The decode row's QuantLinear calls up to their exact sums: kt_hip_quant_linear_multi at rows = 1 with no bias and
  * no codes out -- the quantization of x and the digit product, one launch -- leaving each call's i64 sums and state
  * (max |x|, c = from_ratio(xmax, WLEVELS) * xs * ws, the mode) in ws_dev for the op that reads the output next,
@@ -295,6 +311,15 @@ int kt_hip_ref_swiglu_sums(int dev, const kt_hip_ql_sums* g, const kt_hip_ql_sum
 int kt_hip_ref_gelu(int dev, const int32_t* x_dev, const kt_hip_qscale* xs_dev, int64_t n,
                     const int64_t* gelu_codes_dev, const kt_hip_codelut* gelu, int32_t* y_dev, kt_hip_qscale* ys_dev,
                     void* stream);
+/* kt_hip_quant_linear followed by kt_hip_ref_gelu of its output (FeedForward's proj_in and GELU, kt-model-vision/src/
+ * hiera.rs:336-340), without the layer's own codes in between: y_dev (rows x out_f) and ys_dev are kt_hip_ref_gelu's
+ * outputs, and ymax_dev receives KT_QL_PARTS values whose largest is max |y|, for the layer that reads y next
+ * (KT_QL_X_PARTS). The same integers as the two calls. Arguments, workspace and requirements as theirs. */
+int kt_hip_quant_linear_gelu(int dev, const int32_t* x_dev, int64_t rows, int64_t in_f, const kt_hip_qscale* xs_dev,
+                             const int8_t* w_planes_dev, int pw, int64_t out_f, int64_t w_mant, int32_t w_shift,
+                             const int64_t* bias_dev, int64_t b_mant, int32_t b_shift, void* ws_dev, size_t ws_bytes,
+                             const int64_t* gelu_codes_dev, const kt_hip_codelut* gelu, int32_t* y_dev,
+                             kt_hip_qscale* ys_dev, uint32_t* ymax_dev, void* stream);
 /* Conv2d::forward_int (crates/01-engine/kt-core/src/conv.rs:68-130), SAM's PatchEmbed (kt-model-vision/src/
  * hiera.rs:187-190): the image x_dev [ci][h][w] of i32 codes at xs_dev, quant_to by its whole-image max, the
  * convolution against co x (ci kh kw) weight codes in the reference's [co][ci][kh][kw] order held as digit planes

@@ -148,6 +148,10 @@ def _declare(L: C.CDLL) -> None:
         "kt_hip_ref_moe_bucket": (_I, [_I, _P, _I64, _I, _I64, _P, _P, _P, _P]),
         "kt_hip_quant_linear_multi": (_I, [_I, _P, _I64, _I64, _P, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P,
                                             _SZ, _P, _P, _P]),
+        "kt_hip_quant_linear_multi_x": (_I, [_I, _P, _I64, _I64, _P, _I, _P, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P,
+                                              _P, _SZ, _P, _P, _P]),
+        "kt_hip_quant_linear_gelu": (_I, [_I, _P, _I64, _I64, _P, _P, _I, _I64, _I64, C.c_int32, _P, _I64, C.c_int32,
+                                          _P, _SZ, _P, _P, _P, _P, _P, _P]),
         "kt_hip_quant_linear_multi_align": (_I64, [_I64, _I64, _I]),
         "kt_hip_quant_linear_sums_ok": (_I, [_I64, _I64, _I]),
         "kt_hip_quant_linear_multi_sums": (_I, [_I, _P, _I64, _P, _I, _P, _P, _I, _P, _P, _P, _SZ, _P]),
@@ -449,18 +453,26 @@ def quant_linear_multi_align(rows: int, out_f: int, pw: int) -> int:
     return lib().kt_hip_quant_linear_multi_align(rows, out_f, pw)
 
 
+X_ANY, X_CLOSED, X_PARTS = 0, 1, 2  # KT_QL_X_*: what is known of max |x|
+QL_PARTS = 1024  # KT_QL_PARTS
+
+
 def quant_linear_multi(x_dev, rows: int, in_f: int, xs_dev, seg_out, w_planes_dev, pw: int, w_scales, bias_dev,
-                       b_scales, ws_dev, ws_bytes: int, y_devs, os_dev, stream=None, dev: int = 0) -> None:
+                       b_scales, ws_dev, ws_bytes: int, y_devs, os_dev, stream=None, dev: int = 0,
+                       x_kind: int = X_ANY, xmax_dev=None) -> None:
     """Several QuantLinear::forward_int calls on one x, computed together (their weights stacked by rows in
     w_planes_dev): y_devs[g] and record os_dev[g] equal call g's own. b_scales[g]: None where call g has no bias
-    (bias_dev: None, or the stacked bias codes with zeros there)."""
+    (bias_dev: None, or the stacked bias codes with zeros there). x_kind, xmax_dev: what the caller knows of max |x|
+    (X_CLOSED: x is the whole output of an op that closes with requant_dyn; X_PARTS: xmax_dev holds its partial
+    maxima)."""
     n = len(seg_out)
     arr = lambda t, v: (t * n)(*v)  # noqa: E731
     hb = [0 if (bias_dev is None or b is None) else 1 for b in b_scales]
-    check(lib().kt_hip_quant_linear_multi(
-        dev, _ptr(x_dev), rows, in_f, _ptr(xs_dev), n, arr(C.c_int64, [int(v) for v in seg_out]), _ptr(w_planes_dev),
-        pw, arr(C.c_int64, [int(w[0]) for w in w_scales]), arr(C.c_int32, [int(w[1]) for w in w_scales]),
-        _ptr(bias_dev), arr(C.c_int, hb), arr(C.c_int64, [int(b[0]) if b else 0 for b in b_scales]),
+    check(lib().kt_hip_quant_linear_multi_x(
+        dev, _ptr(x_dev), rows, in_f, _ptr(xs_dev), x_kind, _ptr(xmax_dev), n,
+        arr(C.c_int64, [int(v) for v in seg_out]), _ptr(w_planes_dev), pw, arr(C.c_int64, [int(w[0]) for w in w_scales]),
+        arr(C.c_int32, [int(w[1]) for w in w_scales]), _ptr(bias_dev), arr(C.c_int, hb),
+        arr(C.c_int64, [int(b[0]) if b else 0 for b in b_scales]),
         arr(C.c_int32, [int(b[1]) if b else 0 for b in b_scales]), _ptr(ws_dev), ws_bytes,
         arr(C.c_void_p, [_ptr(y) for y in y_devs]), _ptr(os_dev), _stream(stream)), "quant linear multi")
 
@@ -780,6 +792,18 @@ def ref_gelu(x_dev, xs_dev, n: int, gelu_codes_dev, gelu: CodeLut, y_dev, ys_dev
     """apply_gelu (kt-model-vision/src/nonlin.rs:30-45) of n codes: y at the table's code scale."""
     check(lib().kt_hip_ref_gelu(dev, _ptr(x_dev), _ptr(xs_dev), n, _ptr(gelu_codes_dev), C.byref(gelu), _ptr(y_dev),
                                 _ptr(ys_dev), _stream(stream)), "ref gelu")
+
+
+def quant_linear_gelu(x_dev, rows: int, in_f: int, xs_dev, w_planes_dev, pw: int, out_f: int, w_scale, bias_dev, b_scale,
+                      ws_dev, ws_bytes: int, gelu_codes_dev, gelu: CodeLut, y_dev, ys_dev, ymax_dev, stream=None,
+                      dev: int = 0) -> None:
+    """quant_linear, then ref_gelu of its output (whose own codes are not kept): y and its record, and in ymax_dev
+    (QL_PARTS uint32) partial maxima of |y| for the layer that reads it next. Asynchronous."""
+    bm, bs = b_scale if b_scale is not None else (0, 0)
+    check(lib().kt_hip_quant_linear_gelu(
+        dev, _ptr(x_dev), rows, in_f, _ptr(xs_dev), _ptr(w_planes_dev), pw, out_f, int(w_scale[0]), int(w_scale[1]),
+        _ptr(bias_dev), int(bm), int(bs), _ptr(ws_dev), ws_bytes, _ptr(gelu_codes_dev), C.byref(gelu), _ptr(y_dev),
+        _ptr(ys_dev), _ptr(ymax_dev), _stream(stream)), "quant linear gelu")
 
 
 def ref_from_reals(real, levels: int = 1 << 28):

@@ -242,11 +242,14 @@ int kt_hip_quant_linear(int dev, const int32_t* x_dev, int64_t rows, int64_t in_
                                         (hipStream_t)stream);
 }
 
-int kt_hip_quant_linear_multi(int dev, const int32_t* x_dev, int64_t rows, int64_t in_f, const kt_hip_qscale* xs_dev,
-                              int nseg, const int64_t* seg_out, const int8_t* w_planes_dev, int pw,
-                              const int64_t* w_mant, const int32_t* w_shift, const int64_t* bias_dev,
-                              const int* has_bias, const int64_t* b_mant, const int32_t* b_shift, void* ws_dev,
-                              size_t ws_bytes, int32_t* const* y_devs, kt_hip_qscale* os_dev, void* stream) {
+int kt_hip_quant_linear_multi_x(int dev, const int32_t* x_dev, int64_t rows, int64_t in_f, const kt_hip_qscale* xs_dev,
+                                int x_kind, const uint32_t* xmax_dev, int nseg, const int64_t* seg_out,
+                                const int8_t* w_planes_dev, int pw, const int64_t* w_mant, const int32_t* w_shift,
+                                const int64_t* bias_dev, const int* has_bias, const int64_t* b_mant,
+                                const int32_t* b_shift, void* ws_dev, size_t ws_bytes, int32_t* const* y_devs,
+                                kt_hip_qscale* os_dev, void* stream) {
+    if (x_kind < KT_QL_X_ANY || x_kind > KT_QL_X_PARTS || (x_kind == KT_QL_X_PARTS && !xmax_dev))
+        return (int)hipErrorInvalidValue;
     if (nseg < 1 || nseg > KT_QL_MAX_SEGMENTS || !seg_out || !w_mant || !w_shift || !y_devs || rows < 1 ||
         in_f < 1 || (pw != 1 && pw != 3 && pw != 5) || (bias_dev && (!has_bias || !b_mant || !b_shift)))
         return (int)hipErrorInvalidValue;
@@ -269,7 +272,37 @@ int kt_hip_quant_linear_multi(int dev, const int32_t* x_dev, int64_t rows, int64
     KT_TRY(hipSetDevice(dev));
     return (int)kt::launch_quant_linear_multi(x_dev, rows, in_f, xs_dev, w_planes_dev, pw, nseg, seg_out, w_mant,
                                               w_shift, bias_dev, has_bias, b_mant, b_shift, flush_of(3, pw), ws_dev,
-                                              y_devs, os_dev, (hipStream_t)stream);
+                                              y_devs, os_dev, (hipStream_t)stream, x_kind, xmax_dev);
+}
+
+int kt_hip_quant_linear_multi(int dev, const int32_t* x_dev, int64_t rows, int64_t in_f, const kt_hip_qscale* xs_dev,
+                              int nseg, const int64_t* seg_out, const int8_t* w_planes_dev, int pw,
+                              const int64_t* w_mant, const int32_t* w_shift, const int64_t* bias_dev,
+                              const int* has_bias, const int64_t* b_mant, const int32_t* b_shift, void* ws_dev,
+                              size_t ws_bytes, int32_t* const* y_devs, kt_hip_qscale* os_dev, void* stream) {
+    return kt_hip_quant_linear_multi_x(dev, x_dev, rows, in_f, xs_dev, KT_QL_X_ANY, nullptr, nseg, seg_out,
+                                       w_planes_dev, pw, w_mant, w_shift, bias_dev, has_bias, b_mant, b_shift, ws_dev,
+                                       ws_bytes, y_devs, os_dev, stream);
+}
+
+int kt_hip_quant_linear_gelu(int dev, const int32_t* x_dev, int64_t rows, int64_t in_f, const kt_hip_qscale* xs_dev,
+                             const int8_t* w_planes_dev, int pw, int64_t out_f, int64_t w_mant, int32_t w_shift,
+                             const int64_t* bias_dev, int64_t b_mant, int32_t b_shift, void* ws_dev, size_t ws_bytes,
+                             const int64_t* gelu_codes_dev, const kt_hip_codelut* gelu, int32_t* y_dev,
+                             kt_hip_qscale* ys_dev, uint32_t* ymax_dev, void* stream) {
+    if (rows < 1 || in_f < 1 || out_f < 1 || (pw != 1 && pw != 3 && pw != 5) || w_mant < 0 || b_mant < 0)
+        return (int)hipErrorInvalidValue;
+    const int64_t kp = kp_of(in_f);
+    if (rows * kp >= ((int64_t)1 << 31) || rows * out_f >= ((int64_t)1 << 31) || kp > INT_MAX)
+        return (int)hipErrorInvalidValue;
+    if (!x_dev || !xs_dev || !w_planes_dev || !ws_dev || !y_dev || !ys_dev || !ymax_dev || !gelu_codes_dev || !gelu ||
+        gelu->n < 1 || !gelu->right_identity ||
+        ws_bytes < kt_hip_quant_linear_workspace(rows, in_f, out_f, nullptr))
+        return (int)hipErrorInvalidValue;
+    KT_TRY(hipSetDevice(dev));
+    return (int)kt::launch_quant_linear_gelu(x_dev, rows, in_f, xs_dev, w_planes_dev, pw, out_f, w_mant, w_shift,
+                                             bias_dev, b_mant, b_shift, flush_of(3, pw), ws_dev, gelu_codes_dev, gelu,
+                                             y_dev, ys_dev, ymax_dev, (hipStream_t)stream);
 }
 
 int kt_hip_quant_linear_sums_ok(int64_t in_f, int64_t out_f, int pw) {

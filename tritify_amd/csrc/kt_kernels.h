@@ -96,7 +96,12 @@ hipError_t launch_quant_linear_multi(const int32_t* x, int64_t rows, int64_t in,
                                      const int64_t* w_mant, const int32_t* w_shift, const int64_t* bias,
                                      const int* has_bias, const int64_t* b_mant, const int32_t* b_shift,
                                      int64_t flush_k, void* ws, int32_t* const* y, kt_hip_qscale* os,
-                                     hipStream_t s);
+                                     hipStream_t s, int x_kind = KT_QL_X_ANY, const uint32_t* xmax = nullptr);
+hipError_t launch_quant_linear_gelu(const int32_t* x, int64_t rows, int64_t in, const kt_hip_qscale* xs,
+                                    const int8_t* wb, int pw, int64_t out, int64_t w_mant, int32_t w_shift,
+                                    const int64_t* bias, int64_t b_mant, int32_t b_shift, int64_t flush_k, void* ws,
+                                    const int64_t* codes, const kt_hip_codelut* lut, int32_t* y, kt_hip_qscale* ys,
+                                    uint32_t* ymax, hipStream_t s);
 hipError_t launch_quant_linear(const int32_t* x, int64_t rows, int64_t in, const kt_hip_qscale* xs,
                                const int8_t* wb, int pw, int64_t out, int64_t w_mant, int32_t w_shift,
                                const int64_t* bias, int64_t b_mant, int32_t b_shift, int64_t flush_k, void* ws,

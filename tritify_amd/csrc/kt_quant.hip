@@ -174,6 +174,7 @@ template <bool CONV>
 __global__ __launch_bounds__(QL_THREADS) void ql_quant_kernel(const int32_t* __restrict__ x, int64_t nx,
                                                               int64_t rows, int64_t in, int64_t kp, ConvGeom geom,
                                                               const uint32_t* __restrict__ part, int nparts,
+                                                              int closed,
                                                               const kt_hip_qscale* __restrict__ xs, QlSeg seg,
                                                               QlScales sc, QlState* __restrict__ st,
                                                               int8_t* __restrict__ xa, uint64_t* __restrict__ zacc,
@@ -186,7 +187,9 @@ __global__ __launch_bounds__(QL_THREADS) void ql_quant_kernel(const int32_t* __r
         for (int64_t i = i0; i < nzcnt; i += st_) zcnt[i] = 0;
     }
     uint32_t m = 0;
-    if (nparts > 0) {
+    if (closed) {  // the whole output of an op that closed with requant_dyn: its largest code is 2^28, or all are zero
+        m = xs->mant != 0 ? (uint32_t)ACT_LEVELS : 0u;
+    } else if (nparts > 0) {
         for (int i = threadIdx.x; i < nparts; i += QL_THREADS) m = part[i] > m ? part[i] : m;
     } else {  // a short x (QL_FUSED_MAX values at most): every CTA takes max |x| itself, no ql_absmax pass
         for (int64_t i0 = threadIdx.x; i0 < nx; i0 += 8 * QL_THREADS) {  // 8 loads in flight per thread
@@ -200,7 +203,7 @@ __global__ __launch_bounds__(QL_THREADS) void ql_quant_kernel(const int32_t* __r
             }
         }
     }
-    m = block_max(m, red);
+    if (!closed) m = block_max(m, red);
     if (blockIdx.x == 0 && threadIdx.x < KT_QL_YSLOTS * seg.n)
         st[threadIdx.x / KT_QL_YSLOTS].ymax[threadIdx.x % KT_QL_YSLOTS].v = 0;
     if (blockIdx.x == 0 && (int)threadIdx.x < seg.n) {  // each segment's record, for the GEMM epilogue and ql_requant
@@ -388,8 +391,8 @@ __global__ __launch_bounds__(QS_THREADS) void ql_skinny_kernel(const int32_t* __
 
 // y = requant_dyn(acc, ACT_LEVELS, ymax) per segment (layers.rs:33-39, 321-327). The grid's last CTA only writes
 // each segment's record (its Scale products run beside the other CTAs' divisions); the others requantize. Each
-// thread's first accumulator and the segments' states are read before the maximum is known. The maximum comes from
-// the state's slots, or with `part` from the one-row product's maximum per CTA of QS_COLS columns.
+// thread's first accumulator and the segments' states are read before the maximum is known. The
+// one-row product's: the maximum comes from `part`, that product's maximum per CTA of QS_COLS columns.
 __global__ __launch_bounds__(QL_THREADS) void ql_requant_kernel(const int64_t* __restrict__ acc, int64_t n,
                                                                 int64_t out, const int64_t* __restrict__ bias,
                                                                 const QlState* __restrict__ st, QlSeg seg,
@@ -411,7 +414,7 @@ __global__ __launch_bounds__(QL_THREADS) void ql_requant_kernel(const int64_t* _
         mode = q->mode, xmax = q->xmax, c_mant = q->c_mant, c_shift = q->c_shift;
     }
     int64_t ymax = 0;
-    if (part) {  // each segment's maximum over its CTAs' slots
+    {  // each segment's maximum over its CTAs' slots
         if (tid < KT_QL_MAX_SEG) s_pmax[tid] = 0;
         __syncthreads();
         unsigned long long pm[KT_QL_MAX_SEG] = {};
@@ -442,10 +445,6 @@ __global__ __launch_bounds__(QL_THREADS) void ql_requant_kernel(const int64_t* _
         }
         __syncthreads();
         if (tid < seg.n) ymax = (int64_t)s_pmax[tid];
-    } else if (tid < seg.n) {
-        const QlState* q = st + tid;
-#pragma unroll
-        for (int i = 0; i < KT_QL_YSLOTS; i++) ymax = (int64_t)q->ymax[i].v > ymax ? (int64_t)q->ymax[i].v : ymax;
     }
     if (rec_cta) {  // each segment's record
         if (tid < seg.n) {
@@ -479,6 +478,138 @@ __global__ __launch_bounds__(QL_THREADS) void ql_requant_kernel(const int64_t* _
         }
         const int64_t w = seg.col0[g + 1] - seg.col0[g];
         yo.y[g][r * w + (o - seg.col0[g])] = v32;
+    }
+}
+
+// The same for more rows (the general digit GEMM's sums, each segment's maximum in its state's slots): V consecutive
+// outputs of a row per step (V = 2 where every boundary is even and every output 8-byte aligned) and 4 steps of loads
+// in flight per thread. GELU (one segment): the codes go on through apply_gelu's table (kt-model-vision/src/nonlin.rs:
+// 30-45) at the layer's own output Scale, only its codes and record are written, and each CTA leaves its largest
+// |code| in ge.part (KT_QL_PARTS slots, the unused ones zeroed), so that the layer that reads them needs no pass for it.
+// Without GELU bound by memory, 8 bytes read and 4 written per output (4096 x 448: 10.5 us). With it by the table
+// reads, a cache line per lane (4096 x 1792: 52 us, against 22.8 + 35.5 + 9.8 for the requant, the table pass and the
+// maximum as three passes).
+struct QlGelu {
+    const int64_t* codes;
+    kt_hip_codelut lut;
+    kt_hip_qscale* ys;
+    uint32_t* part;
+};
+template <int V, bool GELU>
+__global__ __launch_bounds__(QL_THREADS) void ql_requant_rows_kernel(const int64_t* __restrict__ acc, int64_t n,
+                                                                     int out, const int64_t* __restrict__ bias,
+                                                                     const QlState* __restrict__ st, QlSeg seg,
+                                                                     QlScales sc, QlOut yo, QlGelu ge) {
+    typedef long long accv __attribute__((ext_vector_type(V)));
+    constexpr int U = 4;
+    __shared__ int64_t s_ymax[KT_QL_MAX_SEG];
+    __shared__ double s_rinv[KT_QL_MAX_SEG];
+    __shared__ int32_t s_mode[KT_QL_MAX_SEG];
+    __shared__ Sc s_gelu[2];
+    __shared__ uint32_t red[QL_THREADS / 64];
+    const int tid = threadIdx.x;
+    const int64_t nv = n / V, v0 = (int64_t)blockIdx.x * QL_THREADS + tid, step = (int64_t)(gridDim.x - 1) * QL_THREADS;
+    const bool rec_cta = blockIdx.x == gridDim.x - 1;
+    accv a[U];
+    auto fetch = [&](int64_t v) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (v + u * step < nv) a[u] = reinterpret_cast<const accv*>(acc)[v + u * step];
+    };
+    if (!rec_cta) fetch(v0);  // in flight while the maxima are read
+    if (tid < seg.n) {
+        const QlState* q = st + tid;
+        int64_t ymax = 0;
+#pragma unroll
+        for (int i = 0; i < KT_QL_YSLOTS; i++) ymax = (int64_t)q->ymax[i].v > ymax ? (int64_t)q->ymax[i].v : ymax;
+        const int mode = q->mode;
+        s_ymax[tid] = ymax, s_mode[tid] = mode, s_rinv[tid] = rq_den(ymax).rinv;
+        if (rec_cta || GELU) {  // each segment's record
+            kt_hip_qscale o{};
+            o.xmax = q->xmax;
+            if (mode == 1) {
+                if (sc.has_bias[tid]) o.mant = sc.b_mant[tid], o.shift = sc.b_shift[tid];
+            } else if (mode == 0 && ymax > 0) {
+                const Sc s2 = sc_mul(from_ratio((u128)(uint64_t)ymax, (u128)ACT_LEVELS), Sc{q->c_mant, q->c_shift});
+                o.mant = s2.mant, o.shift = s2.shift, o.ymax = ymax;
+            }
+            if constexpr (GELU) {  // the table's index and identity factors at this Scale
+                const Sc ys{o.mant, o.shift}, cs{ge.lut.code_mant, ge.lut.code_shift};
+                s_gelu[0] = sc_mul(ys, Sc{ge.lut.inv_mant, ge.lut.inv_shift});
+                s_gelu[1] = sc_mul(ys, sc_recip(cs));
+                o = kt_hip_qscale{};
+                o.mant = cs.mant, o.shift = cs.shift;
+                if (rec_cta) *ge.ys = o;
+            } else {
+                *yo.os[tid] = o;
+            }
+        }
+    }
+    if (rec_cta) {
+        if constexpr (GELU)
+            for (int i = (int)gridDim.x - 1 + tid; i < KT_QL_PARTS; i += QL_THREADS) ge.part[i] = 0;
+        return;
+    }
+    __syncthreads();
+    const Sc mi = GELU ? s_gelu[0] : Sc{0, 0}, idf = GELU ? s_gelu[1] : Sc{0, 0};
+    uint32_t gm = 0;
+    const int outv = out / V;
+    const int64_t dstep = step % outv, rstep = step / outv;
+    int64_t o = v0 % outv, r = v0 / outv;  // (row, vector of columns), advanced incrementally
+    for (int64_t v = v0; v < nv; v += U * step) {
+        if (v != v0) fetch(v);
+        int32_t y[U][V];
+        int g[U], c0[U];
+        int64_t row[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (o >= outv) o -= outv, r++;
+            c0[u] = (int)o * V, row[u] = r;
+            o += dstep, r += rstep;
+            g[u] = GELU ? 0 : ql_seg_of(seg, c0[u]);
+            const int64_t ym = s_ymax[g[u]];
+            const int md = s_mode[g[u]];
+#pragma unroll
+            for (int t = 0; t < V; t++) {
+                y[u][t] = 0;
+                if (v + u * step >= nv) continue;
+                if (md == 1) y[u][t] = sc.has_bias[g[u]] && bias ? (int32_t)bias[c0[u] + t] : 0;
+                else if (md == 0 && ym > 0)  // requant_dyn(v, 2^28, ymax)
+                    y[u][t] = rq_apply(RqDen{ym, (uint64_t)(ym / 2), s_rinv[g[u]]}, (int64_t)a[u][t]);
+            }
+        }
+        if constexpr (GELU) {
+            int64_t idx[U][V], code[U][V];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int t = 0; t < V; t++) {
+                    idx[u][t] = sc_apply32(mi, y[u][t]) - ge.lut.lo_index;
+                    const int64_t i = idx[u][t] < 0 ? 0 : (idx[u][t] > ge.lut.n - 1 ? ge.lut.n - 1 : idx[u][t]);
+                    code[u][t] = ge.codes[i];
+                }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int t = 0; t < V; t++) {
+                    const int64_t c = idx[u][t] < 0 ? 0 : (idx[u][t] >= ge.lut.n ? sc_apply32(idf, y[u][t]) : code[u][t]);
+                    y[u][t] = (int32_t)c;
+                    const uint32_t m = y[u][t] < 0 ? 0u - (uint32_t)y[u][t] : (uint32_t)y[u][t];
+                    if (v + u * step < nv) gm = m > gm ? m : gm;
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (v + u * step >= nv) continue;
+            const int64_t w = seg.col0[g[u] + 1] - seg.col0[g[u]];
+            int32_t* d = yo.y[g[u]] + row[u] * w + (c0[u] - seg.col0[g[u]]);
+            if constexpr (V == 2) *reinterpret_cast<v2i*>(d) = v2i{y[u][0], y[u][1]};
+            else *d = y[u][0];
+        }
+    }
+    if constexpr (GELU) {
+        gm = block_max(gm, red);
+        if (tid == 0) ge.part[blockIdx.x] = gm;
     }
 }
 
@@ -616,7 +747,8 @@ static hipError_t launch_ql_skinny(const int32_t* x, int64_t in, const kt_hip_qs
 static hipError_t launch_ql_impl(const int32_t* x, int64_t rows, int64_t in, const ConvGeom* geom,
                                  const kt_hip_qscale* xs, const int8_t* wb, int pw, int64_t out, const QlSeg& seg,
                                  const QlScales& sc, const int64_t* bias, int64_t flush_k, void* ws, const QlOut& yo,
-                                 hipStream_t s) {
+                                 hipStream_t s, int x_kind = KT_QL_X_ANY, const uint32_t* xmax = nullptr,
+                                 const QlGelu* gelu = nullptr) {
     size_t off[KT_QL_WS_PARTS];
     ql_workspace_bytes(rows, in, out, off);
     char* base = (char*)ws;
@@ -633,7 +765,7 @@ static hipError_t launch_ql_impl(const int32_t* x, int64_t rows, int64_t in, con
     if (ntiles * 4 > KT_QL_PARTS * 8) return hipErrorInvalidValue;  // cannot happen: a split grid has <= 256 tiles
 
     // one row within one k-chunk (the decode step): the quant pass inside the product, then the requant pass
-    if (!geom && rows == 1 && ql_sums_ok(in, out, pw, flush_k) && ql_seg_cols_ok(seg)) {
+    if (!geom && !gelu && rows == 1 && ql_sums_ok(in, out, pw, flush_k) && ql_seg_cols_ok(seg)) {
         const hipError_t e = launch_ql_skinny(x, in, xs, wb, pw, out, seg, sc, bias, ws, s);
         if (e != hipSuccess) return e;
         const int ctas = (int)((out + QS_COLS - 1) / QS_COLS);
@@ -642,16 +774,19 @@ static hipError_t launch_ql_impl(const int32_t* x, int64_t rows, int64_t in, con
         return hipGetLastError();
     }
     // max |x| by its own pass, or inside every quant CTA when x is short (one launch fewer for a decode row)
-    const int gx = nx <= QL_FUSED_MAX ? 0 : grid_for(nx, 8);
-    if (gx > 0) ql_absmax_kernel<<<gx, QL_THREADS, 0, s>>>(x, nx, part_x);
+    // -- or known: the input closed at 2^28, or its partial maxima given
+    const int closed = x_kind == KT_QL_X_CLOSED;
+    int gx = closed || nx <= QL_FUSED_MAX ? 0 : grid_for(nx, 8);
+    if (x_kind == KT_QL_X_PARTS) part_x = const_cast<uint32_t*>(xmax), gx = KT_QL_PARTS;
+    else if (gx > 0) ql_absmax_kernel<<<gx, QL_THREADS, 0, s>>>(x, nx, part_x);
     uint64_t* zacc = splits > 1 ? reinterpret_cast<uint64_t*>(acc) : nullptr;
     const int64_t nzacc = splits > 1 ? n : 0;
     const int gq = grid_for(rows * kp / 4, 1);
     if (geom)
-        ql_quant_kernel<true><<<gq, QL_THREADS, 0, s>>>(x, nx, rows, in, kp, *geom, part_x, gx, xs, seg, sc, st, xa,
+        ql_quant_kernel<true><<<gq, QL_THREADS, 0, s>>>(x, nx, rows, in, kp, *geom, part_x, gx, closed, xs, seg, sc, st, xa,
                                                         zacc, nzacc, tile_cnt, ntiles);
     else
-        ql_quant_kernel<false><<<gq, QL_THREADS, 0, s>>>(x, nx, rows, in, kp, ConvGeom{}, part_x, gx, xs, seg, sc, st,
+        ql_quant_kernel<false><<<gq, QL_THREADS, 0, s>>>(x, nx, rows, in, kp, ConvGeom{}, part_x, gx, closed, xs, seg, sc, st,
                                                          xa, zacc, nzacc, tile_cnt, ntiles);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -667,9 +802,15 @@ static hipError_t launch_ql_impl(const int32_t* x, int64_t rows, int64_t in, con
         ql_requant_conv_kernel<<<grid, QL_THREADS, 0, s>>>(acc, rows, out, st, yo.y[0], yo.os[0]);
         return hipGetLastError();
     }
-    // one output per thread for short outputs (a decode row: its divisions then run side by side, not 8 in a row)
-    ql_requant_kernel<<<grid_for(n, n <= 65536 ? 1 : 2) + 1, QL_THREADS, 0, s>>>(acc, n, out, bias, st, seg, sc, yo,
-                                                                                 nullptr, 0);
+    bool two = out % 2 == 0;  // pairs of outputs: even boundaries, 8-byte aligned outputs
+    for (int g = 0; g < seg.n; g++) two = two && seg.col0[g] % 2 == 0 && ((uintptr_t)yo.y[g] & 7) == 0;
+    const QlGelu ge = gelu ? *gelu : QlGelu{};
+    const int64_t nv = two ? n / 2 : n;
+    const int grid = grid_for(nv, nv <= 65536 ? 1 : 4) + 1;  // short outputs: a vector per thread
+#define KT_RQ(V, G) ql_requant_rows_kernel<V, G><<<grid, QL_THREADS, 0, s>>>(acc, n, (int)out, bias, st, seg, sc, yo, ge)
+    if (gelu) two ? KT_RQ(2, true) : KT_RQ(1, true);
+    else two ? KT_RQ(2, false) : KT_RQ(1, false);
+#undef KT_RQ
     return hipGetLastError();
 }
 
@@ -699,7 +840,7 @@ hipError_t launch_quant_linear_multi(const int32_t* x, int64_t rows, int64_t in,
                                      const int64_t* w_mant, const int32_t* w_shift, const int64_t* bias,
                                      const int* has_bias, const int64_t* b_mant, const int32_t* b_shift,
                                      int64_t flush_k, void* ws, int32_t* const* y, kt_hip_qscale* os,
-                                     hipStream_t s) {
+                                     hipStream_t s, int x_kind, const uint32_t* xmax) {
     QlSeg seg{nseg, {0, 0, 0, 0, 0}};
     QlScales sc{};
     QlOut yo{};
@@ -712,7 +853,21 @@ hipError_t launch_quant_linear_multi(const int32_t* x, int64_t rows, int64_t in,
         yo.y[g] = y[g], yo.os[g] = os + g;
     }
     for (int g = nseg; g <= KT_QL_MAX_SEG; g++) seg.col0[g] = (int)at;
-    return launch_ql_impl(x, rows, in, nullptr, xs, wb, pw, at, seg, sc, bias, flush_k, ws, yo, s);
+    return launch_ql_impl(x, rows, in, nullptr, xs, wb, pw, at, seg, sc, bias, flush_k, ws, yo, s, x_kind, xmax);
+}
+
+hipError_t launch_quant_linear_gelu(const int32_t* x, int64_t rows, int64_t in, const kt_hip_qscale* xs,
+                                    const int8_t* wb, int pw, int64_t out, int64_t w_mant, int32_t w_shift,
+                                    const int64_t* bias, int64_t b_mant, int32_t b_shift, int64_t flush_k, void* ws,
+                                    const int64_t* codes, const kt_hip_codelut* lut, int32_t* y, kt_hip_qscale* ys,
+                                    uint32_t* ymax, hipStream_t s) {
+    QlSeg seg;
+    QlScales sc;
+    QlOut yo;
+    ql_one(out, w_mant, w_shift, bias, b_mant, b_shift, y, ys, seg, sc, yo);
+    const QlGelu ge{codes, *lut, ys, ymax};
+    return launch_ql_impl(x, rows, in, nullptr, xs, wb, pw, out, seg, sc, bias, flush_k, ws, yo, s, KT_QL_X_ANY,
+                          nullptr, &ge);
 }
 
 hipError_t launch_quant_linear_sums(const int32_t* x, int64_t in, const kt_hip_qscale* xs, const int8_t* wb, int pw,

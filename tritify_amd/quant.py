@@ -81,17 +81,24 @@ class QuantLinear:
             self._ws[rows] = (self.torch.empty(n, dtype=self.torch.uint8, device=self.device), n)
         return self._ws[rows]
 
-    def forward_int(self, x_dev, xs_dev, rows: int, y_dev=None, os_dev=None, stream=None):
+    def forward_int(self, x_dev, xs_dev, rows: int, y_dev=None, os_dev=None, stream=None, x_kind: int = B.X_ANY,
+                    xmax_dev=None):
         """y (rows x out_features i32 codes, device) and its scale record from x_dev (rows x in_features i32 codes)
-        at the scale record xs_dev. Asynchronous on `stream`."""
+        at the scale record xs_dev. x_kind, xmax_dev: what is known of max |x| (B.quant_linear_multi). Asynchronous on
+        `stream`."""
         torch = self.torch
         if y_dev is None:
             y_dev = torch.empty(rows * self.out_features, dtype=torch.int32, device=self.device)
         if os_dev is None:
-            os_dev = torch.zeros(4, dtype=torch.int64, device=self.device)
+            os_dev = torch.empty(4, dtype=torch.int64, device=self.device)  # the record is written whole
         ws, n = self.workspace(rows)
-        B.quant_linear(x_dev, rows, self.in_features, xs_dev, self.w_planes, self.pw, self.out_features,
-                       self.w_scale, self.bias, self.b_scale, ws, n, y_dev, os_dev, stream=stream, dev=self.dev)
+        if x_kind == B.X_ANY:
+            B.quant_linear(x_dev, rows, self.in_features, xs_dev, self.w_planes, self.pw, self.out_features,
+                           self.w_scale, self.bias, self.b_scale, ws, n, y_dev, os_dev, stream=stream, dev=self.dev)
+        else:
+            B.quant_linear_multi(x_dev, rows, self.in_features, xs_dev, [self.out_features], self.w_planes, self.pw,
+                                 [self.w_scale], self.bias, [self.b_scale], ws, n, [y_dev], os_dev, stream=stream,
+                                 dev=self.dev, x_kind=x_kind, xmax_dev=xmax_dev)
         return y_dev, os_dev
 
     def sums_ok(self) -> bool:
@@ -177,9 +184,9 @@ class QuantLinearGroup:
             self._ws[rows] = (self.torch.empty(n, dtype=self.torch.uint8, device=self.device), n)
         return self._ws[rows]
 
-    def forward_int(self, x_dev, xs_dev, rows: int, y_devs=None, os_dev=None, stream=None):
+    def forward_int(self, x_dev, xs_dev, rows: int, y_devs=None, os_dev=None, stream=None, x_kind: int = B.X_ANY):
         """Each member's (y rows x out i32 codes, its record): y_devs / os_dev given (os_dev: one record per member,
-        consecutive) or allocated. Asynchronous on `stream`."""
+        consecutive) or allocated. x_kind: what is known of max |x|. Asynchronous on `stream`."""
         torch = self.torch
         if y_devs is None:
             y_devs = [torch.empty(rows * o, dtype=torch.int32, device=self.device) for o in self.outs]
@@ -187,7 +194,7 @@ class QuantLinearGroup:
             os_dev = torch.empty(4 * len(self.outs), dtype=torch.int64, device=self.device)
         ws, n = self.workspace(rows)
         B.quant_linear_multi(x_dev, rows, self.in_features, xs_dev, self.outs, self.w_planes, self.pw, self.w_scales,
-                             self.bias, self.b_scales, ws, n, y_devs, os_dev, stream=stream, dev=self.dev)
+                             self.bias, self.b_scales, ws, n, y_devs, os_dev, stream=stream, dev=self.dev, x_kind=x_kind)
         return [(y, os_dev[4 * g:4 * g + 4]) for g, y in enumerate(y_devs)]
 
     def sums_ok(self) -> bool:

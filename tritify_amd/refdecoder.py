@@ -250,8 +250,9 @@ class RefDecoder:
         if toks.min() < 0 or toks.max() >= self.vocab:
             raise ValueError("forward: a token outside the vocabulary")
         d, dv = self.device, self.dev
+        closed = B.X_CLOSED if T > 1 else B.X_ANY  # every projection reads a norm's, the attention's or SwiGLU's output
         z = lambda n: torch.empty(n, dtype=torch.int32, device=d)  # noqa: E731
-        rec = lambda: torch.zeros(4, dtype=torch.int64, device=d)  # noqa: E731
+        rec = lambda: torch.empty(4, dtype=torch.int64, device=d)  # noqa: E731  (records are written whole)
         qd, kvd = self.nh * self.hd, self.nkv * self.hd
         x, xr, h, hr = z(T * self.dim), rec(), z(T * self.dim), rec()
         t_dev = torch.from_numpy(toks).to(d)
@@ -267,28 +268,28 @@ class RefDecoder:
         for blk in self.blocks:
             norm(x, xr, blk["in_norm"], h, hr)
             if self.grouped:
-                (q, qr), (k, kr), (v, vr) = blk["qkv"].forward_int(h, hr, T, stream=stream)
+                (q, qr), (k, kr), (v, vr) = blk["qkv"].forward_int(h, hr, T, stream=stream, x_kind=closed)
             else:
-                q, qr = blk["wq"].forward_int(h, hr, T, stream=stream)
-                k, kr = blk["wk"].forward_int(h, hr, T, stream=stream)
-                v, vr = blk["wv"].forward_int(h, hr, T, stream=stream)
+                q, qr = blk["wq"].forward_int(h, hr, T, stream=stream, x_kind=closed)
+                k, kr = blk["wk"].forward_int(h, hr, T, stream=stream, x_kind=closed)
+                v, vr = blk["wv"].forward_int(h, hr, T, stream=stream, x_kind=closed)
             B.ref_attention_prefill(q, qr, k, kr, v, vr, T, self.nh, self.nkv, self.hd, self.max_seq, self.cos,
                                     self.sin, self.inv_sqrt, self.exp_codes, self.exp_lut, ws, nws, cat, cr, stream,
                                     dv)
-            blk["wo"].forward_int(cat, cr, T, y_dev=a, os_dev=ar, stream=stream)
+            blk["wo"].forward_int(cat, cr, T, y_dev=a, os_dev=ar, stream=stream, x_kind=closed)
             add(x, xr, a, ar)
             norm(x, xr, blk["post_norm"], h, hr)
             if self.grouped:
-                (gt, gtr), (up, upr) = blk["gu"].forward_int(h, hr, T, stream=stream)
+                (gt, gtr), (up, upr) = blk["gu"].forward_int(h, hr, T, stream=stream, x_kind=closed)
             else:
-                gt, gtr = blk["gate"].forward_int(h, hr, T, stream=stream)
-                up, upr = blk["up"].forward_int(h, hr, T, stream=stream)
+                gt, gtr = blk["gate"].forward_int(h, hr, T, stream=stream, x_kind=closed)
+                up, upr = blk["up"].forward_int(h, hr, T, stream=stream, x_kind=closed)
             B.ref_swiglu_seq(gt, gtr, up, upr, T * self.hidden, self.silu_codes, self.silu_lut, wsq, nsq, hh, hhr,
                              stream, dv)
-            m, mr = blk["down"].forward_int(hh, hhr, T, stream=stream)
+            m, mr = blk["down"].forward_int(hh, hhr, T, stream=stream, x_kind=closed)
             add(x, xr, m, mr)
         norm(x, xr, self.final_norm, h, hr)
-        return self.lm_head.forward_int(h, hr, T, stream=stream)
+        return self.lm_head.forward_int(h, hr, T, stream=stream, x_kind=closed)
 
     def decode_step(self, token: int, pos: int):
         """The logits of `token` at `pos` against the cache: (codes, (mant, shift)) on the host."""

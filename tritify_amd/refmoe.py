@@ -187,7 +187,8 @@ class RefMoeLayer:
         wsq = torch.empty(nsq, dtype=torch.uint8, device=self.device)
         B.ref_swiglu_seq(sg, sgs, su, sus, T * self.shared_hidden, self.silu_codes, self.silu_lut, wsq, nsq, sh, shs,
                          stream, self.dev)
-        sd, sds = self.shared["down"].forward_int(sh, shs, T, os_dev=rec(), stream=stream)
+        sd, sds = self.shared["down"].forward_int(sh, shs, T, os_dev=rec(), stream=stream,
+                                                  x_kind=B.X_CLOSED if T > 1 else B.X_ANY)
         out = torch.empty(T * dim, dtype=torch.int32, device=self.device)
         orec = rec()
         B.ref_add_seq(routed, rrec, sd, sds, T * dim, wsq, nsq, out, orec, stream, self.dev)

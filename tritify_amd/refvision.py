@@ -7,7 +7,8 @@ Conv2d (crates/01-engine/kt-core/src/conv.rs:22-130) and GELU CodeLut (nonlin.rs
                                              the im2col rows through the digit-plane GEMM, bias, whole-output
                                              requant_dyn, stored [c_out][oh][ow]
   proj_in, proj_out  kt_hip_quant_linear     QuantLinear::forward_int (+ bias)          (layers.rs:275-328)
-  GELU               kt_hip_ref_gelu         apply_gelu by the A&S-erf CodeLut          (nonlin.rs:24-45)
+  GELU               kt_hip_quant_linear_gelu  with proj_in: apply_gelu by the A&S-erf   (nonlin.rs:24-45)
+                     (one row: kt_hip_ref_gelu)  CodeLut
 
 The weights come in as the engine builds them (codes and Scales, `Conv2d::from_weights` / `with_bias`); the GELU
 table is built here as `build_gelu_lut` builds it. torch holds the device buffers; it computes nothing.
@@ -83,7 +84,7 @@ class RefConv2d:
         if y_dev is None:
             y_dev = torch.empty(self.co * oh * ow, dtype=torch.int32, device=self.device)
         if os_dev is None:
-            os_dev = torch.zeros(4, dtype=torch.int64, device=self.device)
+            os_dev = torch.empty(4, dtype=torch.int64, device=self.device)  # written whole
         ws, n = self.workspace(h, w)
         B.ref_conv2d(x_dev, xs_rec, self.ci, h, w, self.w_planes, self.pw, self.co, self.kh, self.kw, self.stride,
                      self.pad, self.w_scale, self.bias, self.b_scale, ws, n, y_dev, os_dev, stream, self.dev)
@@ -109,9 +110,15 @@ class RefFeedForward:
 
     def forward_int(self, x_dev, xs_rec, rows: int, stream=None):
         """FeedForward::forward_int (hiera.rs:336-340) of rows x dim codes: (y rows x dim codes, record)."""
-        torch = self.torch
-        h, hs = self.proj_in.forward_int(x_dev, xs_rec, rows, stream=stream)
+        torch, pi = self.torch, self.proj_in
         g = torch.empty(rows * self.hidden, dtype=torch.int32, device=self.device)
-        gs = torch.zeros(4, dtype=torch.int64, device=self.device)
-        B.ref_gelu(h, hs, rows * self.hidden, self.gelu_codes, self.gelu, g, gs, stream, self.dev)
-        return self.proj_out.forward_int(g, gs, rows, stream=stream)
+        gs = torch.empty(4, dtype=torch.int64, device=self.device)  # (every record is written whole)
+        if rows == 1:  # the one-row products take their own maxima
+            h, hs = pi.forward_int(x_dev, xs_rec, rows, stream=stream)
+            B.ref_gelu(h, hs, rows * self.hidden, self.gelu_codes, self.gelu, g, gs, stream, self.dev)
+            return self.proj_out.forward_int(g, gs, rows, stream=stream)
+        gmax = torch.empty(B.QL_PARTS, dtype=torch.int32, device=self.device)
+        ws, n = pi.workspace(rows)
+        B.quant_linear_gelu(x_dev, rows, self.dim, xs_rec, pi.w_planes, pi.pw, self.hidden, pi.w_scale, pi.bias,
+                            pi.b_scale, ws, n, self.gelu_codes, self.gelu, g, gs, gmax, stream, self.dev)
+        return self.proj_out.forward_int(g, gs, rows, stream=stream, x_kind=B.X_PARTS, xmax_dev=gmax)
