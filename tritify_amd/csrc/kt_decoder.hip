@@ -96,12 +96,12 @@ __global__ __launch_bounds__(256) void dec_rope_kv_kernel(int8_t* __restrict__ q
 // threads per v row (16 dimensions each, 16-byte loads) and 64 rows in flight, the 64 row groups summed through
 // LDS, and o = div_round(sum, sum e). The partial sums fit int32: each thread adds at most max_pos / 64 <= 256
 // products of |e| <= 2^15 and |v| <= 127.
-__global__ __launch_bounds__(256) void dec_attention_kernel(const int8_t* __restrict__ qkv, int nqkv,
-                                                            const int32_t* __restrict__ pos,
-                                                            const int8_t* __restrict__ kc,
-                                                            const int8_t* __restrict__ vc, int nh, int nkv,
-                                                            const int32_t* __restrict__ exp_tab,
-                                                            int8_t* __restrict__ o, int max_pos) {
+__global__ __launch_bounds__(256) void dec_attention_row_kernel(const int8_t* __restrict__ qkv, int nqkv,
+                                                                const int32_t* __restrict__ pos,
+                                                                const int8_t* __restrict__ kc,
+                                                                const int8_t* __restrict__ vc, int nh, int nkv,
+                                                                const int32_t* __restrict__ exp_tab,
+                                                                int8_t* __restrict__ o, int max_pos) {
     constexpr int HD = 64;
     extern __shared__ int s_sc[];  // max_pos scores, then weights
     __shared__ int s_red[8];
@@ -170,6 +170,199 @@ __global__ __launch_bounds__(256) void dec_attention_kernel(const int8_t* __rest
         const int64_t dn = (int64_t)s_red[4] + s_red[5] + s_red[6] + s_red[7];
         o[(size_t)t * nh * HD + h * HD + tid] = (int8_t)clamp127(div_round(sum, dn));
     }
+}
+
+// round(a / b) half away from zero clamped to [-127, 127], b > 0: floor((2 |a| + b) / (2 b)) by a double estimate (within
+// one of the exact quotient, which is below 2^8 past the first test) and the exact remainder.
+__device__ __forceinline__ int div_round_q8(int64_t a, int64_t b) {
+    const uint64_t aa = a < 0 ? 0 - (uint64_t)a : (uint64_t)a, n = 2 * aa + (uint64_t)b, d = 2 * (uint64_t)b;
+    if (aa >= 128 * (uint64_t)b) return a < 0 ? -127 : 127;
+    int q = (int)((double)n / (double)d);
+    const int64_t rem = (int64_t)(n - (uint64_t)q * d);
+    if (rem < 0) q--;
+    else if (rem >= (int64_t)d) q++;
+    q = q > 127 ? 127 : q;
+    return a < 0 ? -q : q;
+}
+
+// Prefill attention, hd = 64: a CTA of 8 waves per (q head h, 32 rows), blocks of 32 positions dealt to the waves.
+// Both products run on 32x32x32 int8 MFMAs. S^T = K Q^T puts a row's scores in one lane's registers (lane l: row l % 32;
+// register r of half l / 32: position 8 (r / 4) + 4 (l / 32) + r % 4), which is an operand order of O^T = V^T P^T as it
+// stands: the MFMA pairs equal k slots of its operands, so only V is rearranged, by 4 x 4 byte transposes into the
+// wave's own LDS, to 16 bytes of the same 16 positions for each dimension. Pass 1 takes each row's largest score; pass 2
+// forms the scores again (two MFMAs a block), reads the weights e = EXP[(m - s + 64) >> 7] (0 past 1024) from LDS and
+// multiplies V by their three base-128 digits (e within [-2^20, 2^20): EXP is at most 2^15); the waves' digit sums meet
+// in 64-bit LDS sums, and o = div_round(sum e v, sum e). A table with larger entries takes a plain loop instead.
+// 512 rows, 14 heads: 31.1 -> 10.4 us against the kernel above, 2048 rows 312 -> 51; bound by the chain of a block's
+// lookups, digits and transposes in each wave, the products are 8 MFMAs. Keeping a wave's first blocks of scores in
+// registers between the passes changed nothing.
+constexpr int DA_WAVES = 8;
+__global__ __launch_bounds__(64 * DA_WAVES) void dec_attention_kernel(
+    const int8_t* __restrict__ qkv, int T, int nqkv, const int32_t* __restrict__ pos, const int8_t* __restrict__ kc,
+    const int8_t* __restrict__ vc, int nh, int nkv, const int32_t* __restrict__ exp_tab, int8_t* __restrict__ o,
+    int max_pos) {
+    constexpr int HD = 64, OS = 33;  // sO's row of one dimension: 32 rows of the tile and a pad
+    __shared__ __attribute__((aligned(16))) int8_t sV[DA_WAVES][HD * 32];
+    __shared__ int64_t sO[HD * OS], sDen[DA_WAVES][32];
+    __shared__ int sE[1025], sM[DA_WAVES][32];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, ql = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nqb = (T + 31) / 32, h = (int)blockIdx.x % nh, q0 = 32 * (nqb - 1 - (int)blockIdx.x / nh);
+    const int g = h / (nh / nkv), p0 = pos[0], ks = nkv * HD;
+    const int rows = T - q0 < 32 ? T - q0 : 32;
+    const int plast = p0 + q0 + rows - 1 < max_pos ? p0 + q0 + rows - 1 : max_pos - 1;  // the last position any row attends
+    const int ntile = plast / 32 + 1, pq = p0 + q0 + ql;                                // this lane's row's own position
+    const int8_t* kb = kc + (size_t)g * HD;
+    const int8_t* vb = vc + (size_t)g * HD;
+    const int8_t* qr = qkv + (size_t)(q0 + (ql < rows ? ql : rows - 1)) * nqkv + h * HD;
+    v4i qf[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) qf[c] = *reinterpret_cast<const v4i*>(qr + 32 * c + 16 * half);
+    bool big = false;
+    for (int i = tid; i < 1025; i += 64 * DA_WAVES) {
+        const int e = i < 1024 ? exp_tab[i] : 0;
+        sE[i] = e;
+        big = big || e >= (1 << 20) || e < -(1 << 20);
+    }
+    for (int i = tid; i < HD * OS; i += 64 * DA_WAVES) sO[i] = 0;
+    auto scores = [&](int t) {  // S^T of positions 32 t .. 32 t + 31
+        const int j = 32 * t + ql < plast ? 32 * t + ql : plast;
+        const int8_t* kr = kb + (size_t)j * ks + 16 * half;
+        const v4i k0 = *reinterpret_cast<const v4i*>(kr), k1 = *reinterpret_cast<const v4i*>(kr + 32);
+        return mfma32(k1, qf[1], mfma32(k0, qf[0], v16i{}));
+    };
+    auto position = [&](int t, int r) { return 32 * t + 8 * (r >> 2) + 4 * half + (r & 3); };
+
+    // V: 4 x 4 byte blocks (4 positions from 4 jg, 4 dimensions from 4 dg), two per lane
+    struct VBlk {
+        int32_t w[2][4];
+    };
+    auto vfetch = [&](int t, VBlk& v) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int blk = lane + 64 * i, jg = blk & 7, dg = blk >> 3;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const int j = 32 * t + 4 * jg + b < plast ? 32 * t + 4 * jg + b : plast;
+                v.w[i][b] = *reinterpret_cast<const int32_t*>(vb + (size_t)j * ks + 4 * dg);
+            }
+        }
+    };
+
+    int mx = INT_MIN;
+    for (int t = w; t < ntile; t += DA_WAVES) {
+        const v16i s = scores(t);
+#pragma unroll
+        for (int r = 0; r < 16; r++) mx = position(t, r) <= pq && s[r] > mx ? s[r] : mx;
+    }
+    {
+        const int u = __shfl_xor(mx, 32);
+        mx = u > mx ? u : mx;
+    }
+    if (half == 0) sM[w][ql] = mx;
+    big = __syncthreads_or(big);
+#pragma unroll
+    for (int q = 0; q < DA_WAVES; q++) mx = sM[q][ql] > mx ? sM[q][ql] : mx;
+
+    int64_t den = 0;
+    if (big) {  // uniform: 16 threads per row, 4 dimensions each
+        const int q = tid >> 4, c = tid & 15;
+        int m = INT_MIN;
+        for (int i = 0; i < DA_WAVES; i++) m = sM[i][q] > m ? sM[i][q] : m;
+        const int32_t* qw = reinterpret_cast<const int32_t*>(qkv + (size_t)(q0 + (q < rows ? q : rows - 1)) * nqkv + h * HD);
+        int64_t sum[4] = {0, 0, 0, 0}, dn = 0;
+        for (int j = 0; j <= p0 + q0 + q && j <= plast; j++) {
+            const int32_t* kw = reinterpret_cast<const int32_t*>(kb + (size_t)j * ks);
+            int s = 0;
+            for (int i = 0; i < HD / 4; i++) s = __builtin_amdgcn_sdot4(qw[i], kw[i], s, false);
+            const int idx = (m - s + 64) >> 7;
+            const int64_t e = sE[idx < 1024 ? idx : 1024];
+            dn += e;
+#pragma unroll
+            for (int i = 0; i < 4; i++) sum[i] += e * vb[(size_t)j * ks + 4 * c + i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) sO[(4 * c + i) * OS + q] = sum[i];
+        if (c == 0) sDen[0][q] = dn;
+        if (c > 0 && c < DA_WAVES) sDen[c][q] = 0;
+    } else {
+        v16i acc[2][3];
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int p = 0; p < 3; p++) acc[b][p] = v16i{};
+        int8_t* sv = sV[w];
+        for (int t = w; t < ntile; t += DA_WAVES) {
+            VBlk v;
+            vfetch(t, v);
+            const v16i s = scores(t);
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int blk = lane + 64 * i, jg = blk & 7, dg = blk >> 3;
+                const uint32_t lo01 = __builtin_amdgcn_perm(v.w[i][1], v.w[i][0], 0x05010400);  // j0d0 j1d0 j0d1 j1d1
+                const uint32_t hi01 = __builtin_amdgcn_perm(v.w[i][1], v.w[i][0], 0x07030602);  // j0d2 j1d2 j0d3 j1d3
+                const uint32_t lo23 = __builtin_amdgcn_perm(v.w[i][3], v.w[i][2], 0x05010400);
+                const uint32_t hi23 = __builtin_amdgcn_perm(v.w[i][3], v.w[i][2], 0x07030602);
+                // position group jg = 2 a + half: dword 4 half + a of the dimension's 32 bytes
+                uint32_t* d = reinterpret_cast<uint32_t*>(sv + 4 * dg * 32) + 4 * (jg & 1) + (jg >> 1);
+                d[0] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100);
+                d[8] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302);
+                d[16] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100);
+                d[24] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302);
+            }
+            v4i P[3];
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                int dg[3] = {0, 0, 0};
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    const int r = 4 * a + b;
+                    const int idx = (mx - s[r] + 64) >> 7;  // masked scores are not: their weight is dropped below
+                    int e = sE[(uint32_t)idx < 1024u ? idx : 1024];
+                    e = position(t, r) <= pq ? e : 0;
+                    den += e;
+                    dg[0] |= (e & 127) << (8 * b);
+                    dg[1] |= ((e >> 7) & 127) << (8 * b);
+                    dg[2] |= ((e >> 14) & 255) << (8 * b);
+                }
+#pragma unroll
+                for (int p = 0; p < 3; p++) P[p][a] = dg[p];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            v4i vf[2];
+#pragma unroll
+            for (int b = 0; b < 2; b++) vf[b] = *reinterpret_cast<const v4i*>(sv + (32 * b + ql) * 32 + 16 * half);
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int p = 0; p < 3; p++) acc[b][p] = mfma32(vf[b], P[p], acc[b][p]);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            __builtin_amdgcn_wave_barrier();  // the next block's V goes to the same place
+        }
+        if (w < ntile) {
+#pragma unroll
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int d = 32 * b + 8 * (r >> 2) + 4 * half + (r & 3);
+                    const int64_t v = (int64_t)acc[b][0][r] + ((int64_t)acc[b][1][r] << 7) + ((int64_t)acc[b][2][r] << 14);
+                    atomicAdd(reinterpret_cast<unsigned long long*>(&sO[d * OS + ql]), (unsigned long long)v);
+                }
+        }
+        den += __shfl_xor(den, 32);
+        if (half == 0) sDen[w][ql] = den;
+    }
+    __syncthreads();
+    const int q = tid >> 4, c = tid & 15;  // row q, dimensions 4 c .. 4 c + 3
+    if (q >= rows) return;
+    int64_t dn = 0;
+#pragma unroll
+    for (int i = 0; i < DA_WAVES; i++) dn += sDen[i][q];
+    uint32_t out = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) out |= (uint32_t)(uint8_t)div_round_q8(sO[(4 * c + i) * OS + q], dn) << (8 * i);
+    *reinterpret_cast<uint32_t*>(o + (size_t)(q0 + q) * nh * HD + h * HD + 4 * c) = out;
 }
 
 // Greedy argmax over n int32 logits (the first maximum, argmax_codes of generate.rs:48-56), one CTA of 1024 threads:
@@ -540,9 +733,15 @@ hipError_t launch_dec_attention(const int8_t* qkv, int T, int nqkv, const int32_
                                 const int8_t* vc, int nh, int nkv, const int32_t* exp_tab, int8_t* o, int max_pos,
                                 hipStream_t s) {
     if (T <= 0) return hipSuccess;
-    const size_t lds = (size_t)max_pos * sizeof(int);
-    dec_attention_kernel<<<dim3((unsigned)(T * nh)), dim3(256), lds, s>>>(qkv, nqkv, pos, kc, vc, nh, nkv, exp_tab, o,
-                                                                          max_pos);
+    // short calls stay on a CTA per (row, head), which has fewer steps before its first product: 17 rows 4.0 us against
+    // 6.0 (behind 800 positions 8.4 against 12.2), 64 rows 4.9 against 6.2, 128 rows 6.2 against 6.4, 300 rows 14.4
+    // against 8.7
+    if (T < 128)
+        dec_attention_row_kernel<<<dim3((unsigned)(T * nh)), dim3(256), (size_t)max_pos * sizeof(int), s>>>(
+            qkv, nqkv, pos, kc, vc, nh, nkv, exp_tab, o, max_pos);
+    else
+        dec_attention_kernel<<<dim3((unsigned)((T + 31) / 32 * nh)), dim3(64 * DA_WAVES), 0, s>>>(
+            qkv, T, nqkv, pos, kc, vc, nh, nkv, exp_tab, o, max_pos);
     return hipGetLastError();
 }
 
