@@ -511,8 +511,8 @@ __device__ __forceinline__ void w12_gemm_epilogue(const v16i (&acc0)[C::WTM][C::
             // bytes are moved with shifts, never through the vector's address: an addressed vector becomes a
             // per-thread LDS slot whose indexing reads the dispatch packet, a long stall before the stores
             int8_t* dst = reinterpret_cast<int8_t*>(y) + (size_t)m * N + n;
-            if (full && (N & 15) == 0) {
-                *reinterpret_cast<v4i*>(dst) = v;
+            if (m < M && n + 16 <= N) {
+                store16(dst, v);
             } else if (m < M) {
 #pragma unroll
                 for (int t = 0; t < 16; t++)
@@ -846,7 +846,7 @@ __global__ __launch_bounds__(64 * NW) void w12_skinny_kernel(const int8_t* __res
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// W12 skinny GEMM for 64 < M <= 128 with x staged through LDS. Loaded straight into the MFMA operand lanes (the skinny
+// W12 skinny GEMM for M > 64 with x staged through LDS. Loaded straight into the MFMA operand lanes (the skinny
 // kernel above), each x load instruction touches 16 rows x 64 bytes, half of every 128-byte line it requests, and
 // every one of the N / 16 CTAs reads all of x: at N = K = 4096, 128 MB of x requests for 25 MB of weights, and the
 // requests, not the bytes, set the time. Here a CTA owns 64 rows x one 32-column block (CTAs 8 apart, on one XCD,
@@ -860,6 +860,8 @@ __global__ __launch_bounds__(64 * NW) void w12_skinny_kernel(const int8_t* __res
 // nothing needs masking. Wave w takes pair w % 4 of a stage's four k64 pairs and column half w / 4, all 4 row tiles,
 // and the row sums of tiles 2 (w / 4) and 2 (w / 4) + 1; the waves' partial sums then meet in the ring's LDS.
 // ------------------------------------------------------------------------------------------------------------------
+// Also the product of more rows where its tiles are at most one per CU (w12_linear_out): row blocks of 64, the CTAs
+// of one column block 8 apart whatever their number.
 // 3 stages: 11.6-12.1 us at M = 128, N = K = 4096, against 12.2 for 4 and 12.6-12.9 for 5
 constexpr int SK_NS = 3, SK_X = 64 * 256, SK_LO = 32 * 256, SK_NIB = 32 * 128;  // ring stages; bytes per stage
 constexpr int SK_STAGE = SK_X + SK_LO + SK_NIB, SK_DMAS = 4;                     // 28 KB; DMAs per wave per stage
@@ -877,11 +879,11 @@ __global__ __launch_bounds__(512) void w12_skinny_lds_kernel(const int8_t* __res
     __shared__ int32_t sX[4][64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int b = blockIdx.x, rh = (b >> 3) & 1, cb = (b & 7) | ((b >> 4) << 3);
-    const int m0 = 64 * rh, n0 = 32 * cb;
+    const int b = blockIdx.x, nrb = (M + 63) / 64, rb = (b >> 3) % nrb, cb = (b & 7) | ((b >> 3) / nrb << 3);
+    const int m0 = 64 * rb, n0 = 32 * cb;
     if (n0 >= N) return;  // past the last column block: the whole CTA idles
     const int KB = kp / 32, nst = (kp + 255) / 256;  // k32 blocks, stages
-    const int Mr = M - m0 < 64 ? M - m0 : 64;        // rows of this CTA (>= 1: M > 64)
+    const int Mr = M - m0 < 64 ? M - m0 : 64;        // rows of this CTA (>= 1)
 
     const __amdgpu_buffer_rsrc_t rL = make_rsrc(wlo + (size_t)cb * KB * 1024, (uint32_t)KB * 1024);
     const __amdgpu_buffer_rsrc_t rN = make_rsrc(wnib + (size_t)cb * KB * 512, (uint32_t)KB * 512);
@@ -1339,6 +1341,17 @@ static bool skinny_lds_ok() {
     return ok == 1;
 }
 
+// CTA b of w12_skinny_lds_kernel: row block (b >> 3) % nrb, column block (b & 7) | ((b >> 3) / nrb << 3), so the CTAs of
+// a column block are 8 apart; the ones past the last column block idle.
+template <int OUT>
+static hipError_t skinny_lds(const int8_t* x, const int8_t* lo, const uint8_t* nib, int M, int N, int kp,
+                             const int32_t* mant, const int32_t* shift, const int8_t* lut, void* y, hipStream_t s) {
+    const int64_t grid = 8 * ceil_div(M, 64) * ceil_div(ceil_div(N, 32), 8);
+    w12_skinny_lds_kernel<OUT><<<dim3((unsigned)grid), dim3(512), (size_t)SK_NS * SK_STAGE, s>>>(x, lo, nib, y, M, N, kp,
+                                                                                               mant, shift, lut);
+    return hipGetLastError();
+}
+
 template <int OUT>
 static hipError_t w12_linear_out(const int8_t* x, const int8_t* lo, const uint8_t* nib, int M, int N, int kp,
                                  const int32_t* mant, const int32_t* shift, const int8_t* lut, void* y, hipStream_t s) {
@@ -1365,20 +1378,19 @@ static hipError_t w12_linear_out(const int8_t* x, const int8_t* lo, const uint8_
             KT_SKINNY(1, 8, 2)
         }
         // 65-128 rows with int32 dots: x staged through LDS (w12_skinny_lds_kernel)
-        if (M > 64 && kp <= KT_SMALL_KP && skinny_lds_ok()) {
-            // CTA b: rows 64 ((b >> 3) & 1), column block (b & 7) | ((b >> 4) << 3): 16 * ceil(ncb / 8) CTAs, the
-            // ones past the last column block idle
-            const int64_t ncb = ceil_div(N, 32), grid_l = 16 * ceil_div(ncb, 8);
-            w12_skinny_lds_kernel<OUT><<<dim3((unsigned)grid_l), dim3(512), (size_t)SK_NS * SK_STAGE, s>>>(
-                x, lo, nib, y, M, N, kp, mant, shift, lut);
-            return hipGetLastError();
-        }
+        if (M > 64 && kp <= KT_SMALL_KP && skinny_lds_ok())
+            return skinny_lds<OUT>(x, lo, nib, M, N, kp, mant, shift, lut, y, s);
         // otherwise 65-128 rows: 8 waves x 2 pairs (21.8 us at M = 128, N = K = 4096, against 22.4 for 4 waves x 4
         // pairs, 25.3 for 4 x 8 and 31.0 for 8 x 4)
         KT_SKINNY(1, 8, 4) KT_SKINNY(2, 8, 4) KT_SKINNY(4, 8, 2) KT_SKINNY(8, 8, 2)
 #undef KT_SKINNY
     }
     const bool small = kp <= KT_SMALL_KP;
+    // at most a CTA per CU of 64 x 32 tiles: the LDS-staged kernel, whose 8 waves split each 256-deep stage of k. 512 x
+    // 896, k 4864: 18.1 -> 12.9 us; 200 x 896, k 4864: 17.8 -> 11.8; 512 x 896, k 896: 6.3 -> 5.5. A second round costs
+    // more than it saves (512 x 1152, k 896, 288 tiles: 9.3 against 7.3).
+    if (small && ceil_div(M, 64) * ceil_div(N, 32) <= 256 && (int64_t)M * kp <= (int64_t)UINT32_MAX && skinny_lds_ok())
+        return skinny_lds<OUT>(x, lo, nib, M, N, kp, mant, shift, lut, y, s);
     constexpr int WM = KT_W12_WM, WTM = KT_W12_WTM, WTN = KT_W12_WTN, WV = KT_W12_WAVES, NS = KT_W12_NSLOT;
     const int64_t tiles4 = ceil_div(N, 32 * WTN * 4) * ceil_div(M, 32 * WTM * WM);
     // Fewer 128 x 128 tiles than CUs: 64 x 128 tiles, or 64 x 64 (128 threads) when even those leave CUs idle, so
@@ -1401,9 +1413,12 @@ static hipError_t w12_linear_out(const int8_t* x, const int8_t* lo, const uint8_
     }
 #if KT_W12_DMA
     // enough 256 x 128 tiles to give at least 7/8 of the CUs one: the DMA-fed kernel (config 5's MLP in, 224 tiles:
-    // 4-6% faster than its 448 tiles of 128 x 128, which leave the same CU time idle in their second round)
-    const int64_t tiles_d = ceil_div(N, 128) * ceil_div(M, 256);
-    if (tiles_d >= 224 && dma_lds_ok()) {
+    // 4-6% faster than its 448 tiles of 128 x 128, which leave the same CU time idle in their second round). Past one
+    // round only where its last round is nearly full: one CTA per CU, it pays for the rest of a round where two 128 x
+    // 128 CTAs per CU do not (2048 x 6000, k 4096, 1.47 rounds: 115 us against 99; 1500 x 8192, k 2000, 1.5 rounds: 69.6
+    // against 55.9; 3500 x 8000, k 1500, 3.4: 110 against 95; whole rounds: 63.0 against 63.7, 447 against 449)
+    const int64_t tiles_d = ceil_div(N, 128) * ceil_div(M, 256), rounds_d = ceil_div(tiles_d, 256);
+    if (tiles_d * 100 >= rounds_d * 256 * (rounds_d == 1 ? 87 : 97) && dma_lds_ok()) {
         const size_t lds = (size_t)KT_DMA_NS * KT_DMA_STAGE;
         if (small)
             w12_gemm_dma_kernel<OUT, true><<<dim3((unsigned)tiles_d), dim3(512), lds, s>>>(x, lo, nib, y, M, N, kp,

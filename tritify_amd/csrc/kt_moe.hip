@@ -152,15 +152,14 @@ __device__ __forceinline__ void grouped_epilogue(const v16i (&acc0)[C::WTM][1], 
         if constexpr (XR != 0) w12_requant_strip8<BN>(*xs, sRow, gm, gs, n0, N, [](int n) { return n; }, smem);
         __syncthreads();
         constexpr int CH = BM * BN / 16;
-        const bool vec = n0 + BN <= N && (ystride & 15) == 0;
 #pragma unroll
         for (int i = 0; i < (CH + NT - 1) / NT; i++) {
             const int idx = tid + NT * i, r = idx / (BN / 16), c = (idx % (BN / 16)) * 16;
             if (idx >= CH || r >= rows) continue;
             const v4i v = *reinterpret_cast<const v4i*>(smem + r * BN + c);
             int8_t* dst = yg + (size_t)r * ystride + n0 + c;
-            if (vec) {
-                *reinterpret_cast<v4i*>(dst) = v;
+            if (n0 + c + 16 <= N) {
+                store16(dst, v);
             } else {  // bytes by shifts: an addressed vector would live in scratch memory
 #pragma unroll
                 for (int q = 0; q < 16; q++)
@@ -523,8 +522,23 @@ hipError_t launch_w12_grouped(const int8_t* x, size_t x_bytes, const int32_t* li
     if (ub * GTile::BN > INT32_MAX) return hipErrorInvalidValue;
     const int64_t grid = ub < 512 ? (ub + 7) / 8 * 8 : 512;  // two CTAs per CU, a multiple of 8 (XCDs)
     if (epi != KT_EPI_I8 && epi != KT_EPI_SWIGLU) return hipErrorInvalidValue;
-    // enough 256-row tiles (at full groups) to give every CU one: the DMA-fed kernel, one CTA per CU
-    if (max_rows / 256 * tiles_n >= 256 && grouped_dma_lds_ok()) {
+    // One group (a dense product): the tile with the least time by rounds of 256 CTAs of what a CTA of it takes alone,
+    // in 10 ns: 4.4 us + 0.26 a k-tile for 64 x 128, 8.8 + 0.35 for 128 x 128 (0.8 of that from two rounds on, where two
+    // CTAs share a CU), 11.5 + 0.58 for 256 x 128 (DMA-fed). SwiGLU, measured with 64, 128 and 256 rows: 512 x 4864, k
+    // 896: 23.5, 22.0, 19.8 us; 300 x 4864: 17.1, 15.1, 19.3; 150 x 4864: 11.8, 13.7, 17.1; 600 x 4864: 25.4, 23.0, 21.5;
+    // 2000 x 4864: 75.3, 52.9, 59.1; 1024 x 1408, k 4096: 41.6, 34.7, 48.3; 256 x 1408, k 4096: 20.9, 31.3, 47.2.
+    int one = 0;  // rows of the tile
+    if (groups == 1) {
+        const int64_t nk = kp / 64;
+        const auto cost = [&](int64_t bm, int64_t c, int64_t per) {
+            return ((max_rows + bm - 1) / bm * tiles_n + 255) / 256 * (c + per * nk);
+        };
+        const int64_t ch = cost(64, 440, 26), cd = cost(256, 1150, 58), c1 = cost(128, 880, 35);
+        const int64_t ca = c1 > 880 + 35 * nk ? c1 * 4 / 5 : c1;
+        one = cd < ca && cd < ch && grouped_dma_lds_ok() ? 256 : (ca < ch ? 128 : 64);
+    }
+    // several: enough 256-row tiles (at full groups) to give every CU one: the DMA-fed kernel, one CTA per CU
+    if (one == 256 || (groups > 1 && max_rows / 256 * tiles_n >= 256 && grouped_dma_lds_ok())) {
         const size_t lds = (size_t)KT_DMA_NS * dma_stage_x<KT_DMA_XR>();  // the 288-row tile's stages
         const int64_t ub2 = ((max_rows + 255) / 256 + groups) * tiles_n;
         const unsigned grid2 = (unsigned)(ub2 < 256 ? (ub2 + 7) / 8 * 8 : 256);
@@ -544,8 +558,7 @@ hipError_t launch_w12_grouped(const int8_t* x, size_t x_bytes, const int32_t* li
                                                                        shift, silu, h_shift, y, ystride, off,      \
                                                                        (int)max_rows)
     const int64_t tiles_h = (max_rows + GTileH::BM - 1) / GTileH::BM * tiles_n;
-    if (groups == 1 && (max_rows + GTile::BM - 1) / GTile::BM * tiles_n < 512) {
-        // a short dense batch, fewer 128-row tiles than CTA slots (two per CU): 64-row tiles, twice the tiles
+    if (one == 64) {
         const unsigned grid_h = (unsigned)(tiles_h < 512 ? (tiles_h + 7) / 8 * 8 : 512);
         if (epi == KT_EPI_I8)
             w12_grouped_kernel<KT_EPI_I8, GT_HALF><<<dim3(grid_h), dim3(256), 0, s>>>(

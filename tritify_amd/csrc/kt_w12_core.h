@@ -84,6 +84,11 @@ __device__ __forceinline__ v4i bload16nt(__amdgpu_buffer_rsrc_t r, uint32_t voff
 __device__ __forceinline__ v2i bload8nt(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
     return __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 2);
 }
+// 16 bytes to any address: the hardware takes unaligned vector stores, so an odd row length costs no byte stores.
+__device__ __forceinline__ void store16(int8_t* p, v4i v) {
+    typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+    *reinterpret_cast<v4i_any*>(p) = v;
+}
 // An offset that is out of range for every buffer here (buffers are below 4 GB - 16 B).
 #define KT_OOB 0xFFFFFFF0u
 
