@@ -75,6 +75,32 @@ int digits_for(const int32_t* v, size_t n) {
     return 5;
 }
 
+// plane_class(digits_for(v, n)) with one OR per value for the common ranges (v ^ (v >> 31) is v, or -1 - v below zero):
+// all within [-128, 127], or within +-2^22, well inside three digits. A few microseconds of a call's host time at 64
+// rows of 896 (11.7 -> 3.1 us for the scan).
+int planes_of(const int32_t* v, size_t n) {
+    uint32_t any = 0;
+    for (size_t i = 0; i < n; i++) any |= (uint32_t)(v[i] ^ (v[i] >> 31));
+    if (any < 128u) return 1;
+    if (any < (1u << 22)) return 3;
+    return plane_class(digits_for(v, n));
+}
+
+// A pinned host buffer.
+struct PinBuf {
+    void* ptr = nullptr;
+    hipError_t need(size_t bytes) { return ptr ? hipSuccess : hipHostMalloc(&ptr, bytes, hipHostMallocDefault); }
+    void release() {
+        if (ptr) (void)hipHostFree(ptr);
+        ptr = nullptr;
+    }
+};
+
+// Results come back through two pinned blocks, one being filled by the copy engine while the other is moved to the
+// caller's memory: the runtime's own staging of a pageable copy does one after the other (2.5 MB: 155 us, against 53 for
+// the transfer and 80 for the move).
+constexpr size_t Y_BLOCK = 512 << 10;
+
 // k-chunk of the int32 accumulators: a group sums at most min(px, pw) plane pairs per k, each at most 128^2 in
 // magnitude, so floor((2^31 - 1) / (min(px,pw) * 16384)) terms cannot wrap; rounded down to 256.
 int64_t flush_of(int px, int pw) {
@@ -121,6 +147,8 @@ struct kt_hip_backend {
     std::map<Key, Entry> cache;
     uint64_t bytes = 0, tick = 0;
     DevBuf xcodes, xplanes, ydev, wcodes;
+    PinBuf ypin[2];
+    hipEvent_t yev[2] = {nullptr, nullptr};
 };
 
 #define KT_TRY(expr)                          \
@@ -185,7 +213,7 @@ const char* kt_hip_error_string(int e) { return hipGetErrorString((hipError_t)e)
 
 int64_t kt_hip_kp(int64_t k) { return kp_of(k); }
 
-int kt_hip_planes_for(const int32_t* codes, size_t n) { return plane_class(digits_for(codes, n)); }
+int kt_hip_planes_for(const int32_t* codes, size_t n) { return planes_of(codes, n); }
 
 int kt_hip_pack_planes(int dev, const int32_t* codes_dev, int64_t rows, int64_t k, int planes, int8_t* planes_dev,
                        void* stream) {
@@ -410,6 +438,10 @@ void kt_hip_close(kt_hip_backend* b) {
         b->xplanes.release();
         b->ydev.release();
         b->wcodes.release();
+        for (int i = 0; i < 2; i++) {
+            b->ypin[i].release();
+            if (b->yev[i]) (void)hipEventDestroy(b->yev[i]);
+        }
         (void)hipStreamDestroy(b->stream);
     }
     delete b;
@@ -454,7 +486,7 @@ static hipError_t weights_for(kt_hip_backend* b, const int32_t* w, const uint64_
             return hipSuccess;
         }
     }
-    const int p = plane_class(digits_for(w, out * k));
+    const int p = planes_of(w, out * k);
     const int64_t kp = kp_of((int64_t)k);
     const uint64_t bytes = (uint64_t)p * out * (uint64_t)kp;
     hipError_t e = b->wcodes.grow(out * k * sizeof(int32_t));
@@ -492,6 +524,33 @@ static hipError_t weights_for(kt_hip_backend* b, const int32_t* w, const uint64_
     return hipSuccess;
 }
 
+// The call's result (bytes of ydev) into the caller's memory, once the stream has come to it.
+static hipError_t fetch(kt_hip_backend* b, int64_t* y, size_t bytes) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < 2 && e == hipSuccess; i++) {
+        e = b->ypin[i].need(Y_BLOCK);
+        if (e == hipSuccess && !b->yev[i]) e = hipEventCreateWithFlags(&b->yev[i], hipEventDisableTiming);
+    }
+    if (e != hipSuccess) return e;
+    char* dst = reinterpret_cast<char*>(y);
+    const char* src = static_cast<const char*>(b->ydev.ptr);
+    const size_t blocks = (bytes + Y_BLOCK - 1) / Y_BLOCK;
+    auto len = [&](size_t i) { return bytes - i * Y_BLOCK < Y_BLOCK ? bytes - i * Y_BLOCK : Y_BLOCK; };
+    auto start = [&](size_t i) {
+        const hipError_t c = hipMemcpyAsync(b->ypin[i & 1].ptr, src + i * Y_BLOCK, len(i), hipMemcpyDeviceToHost, b->stream);
+        return c != hipSuccess ? c : hipEventRecord(b->yev[i & 1], b->stream);
+    };
+    for (size_t i = 0; i < 2 && i < blocks && e == hipSuccess; i++) e = start(i);
+    for (size_t i = 0; i < blocks && e == hipSuccess; i++) {
+        e = hipEventSynchronize(b->yev[i & 1]);
+        if (e != hipSuccess) break;
+        memcpy(dst + i * Y_BLOCK, b->ypin[i & 1].ptr, len(i));
+        if (i + 2 < blocks) e = start(i + 2);
+    }
+    if (e != hipSuccess) (void)hipStreamSynchronize(b->stream);  // no copy may still write the blocks
+    return e;
+}
+
 // TcLinear::run (backend.rs:156-172) on the device.
 static int run(kt_hip_backend* b, const int32_t* x, const int32_t* w, const uint64_t* id, size_t rows, size_t out,
                size_t k, int64_t* y) {
@@ -504,7 +563,7 @@ static int run(kt_hip_backend* b, const int32_t* x, const int32_t* w, const uint
     if (rows > INT_MAX || out > INT_MAX || kp > INT_MAX) return (int)hipErrorInvalidValue;
     std::lock_guard<std::mutex> g(b->mu);
     KT_TRY(hipSetDevice(b->dev));
-    const int px = plane_class(digits_for(x, rows * k));
+    const int px = planes_of(x, rows * k);
     int8_t* wplanes = nullptr;
     int pw = 0;
     bool temp = false;
@@ -535,10 +594,7 @@ static int run(kt_hip_backend* b, const int32_t* x, const int32_t* w, const uint
                                        b->plant == KT_PLANT_DROP_TOP, b->stream)) != hipSuccess)
             return fail(e);
     }
-    if ((e = hipMemcpyAsync(y, b->ydev.ptr, rows * out * sizeof(int64_t), hipMemcpyDeviceToHost, b->stream)) !=
-        hipSuccess)
-        return fail(e);
-    if ((e = hipStreamSynchronize(b->stream)) != hipSuccess) return fail(e);
+    if ((e = fetch(b, y, rows * out * sizeof(int64_t))) != hipSuccess) return fail(e);
     if (temp) KT_TRY(hipFree(wplanes));
     return 0;
 }
