@@ -431,6 +431,28 @@ int kt_hip_ref_moe_route(int dev, const int32_t* logits_dev, int64_t tokens, int
                          const kt_hip_qscale* ls_dev, int sigmoid, int norm_topk, const int64_t* codes_dev,
                          const kt_hip_codelut* lut, const int64_t* bias_dev, int32_t* sel_dev, int64_t* ec_dev,
                          int64_t* sumc_dev, void* stream);
+/* The routed experts of MoeMlp over bucketed rows: per row its expert's gate and up QuantLinears, SiLU(gate) * up and
+ * the down QuantLinear, each quantized and requantized by the row's own maxima (SwiGluMlp::forward_int of one row per
+ * (token, expert), layers.rs:609-640, 988-1020): the same integers as kt_hip_quant_linear_rows for gate and for up,
+ * kt_hip_ref_swiglu of the rows and kt_hip_quant_linear_rows for down, in six launches on one tile plan. x, xidx, x_rows,
+ * rows, xs, xs_step, groups and off as kt_hip_quant_linear_rows's; y_dev (rows x dim) and ys_dev (rows records) are the
+ * down product's. gu_planes: per group the planes of its gate codes over its up codes, a (2 hidden) x dim matrix
+ * (kt_hip_pack_planes_tiled); down_planes: dim x hidden. Scales: one (mant, shift) per group, device arrays. hidden <=
+ * 4096 (kt_hip_ref_moe_experts_workspace returns 0 past it). */
+typedef struct {
+    const int8_t* gu_planes;
+    const int8_t* down_planes;
+    size_t gu_group_bytes, down_group_bytes;
+    const int64_t *gate_mant, *up_mant, *down_mant;
+    const int32_t *gate_shift, *up_shift, *down_shift;
+    int32_t gu_pw, down_pw;
+} kt_hip_moe_weights;
+size_t kt_hip_ref_moe_experts_workspace(int64_t rows, int64_t dim, int64_t hidden, int64_t groups);
+int kt_hip_ref_moe_experts(int dev, const int32_t* x_dev, const int32_t* xidx_dev, int64_t x_rows, int64_t rows,
+                           int64_t dim, int64_t hidden, const kt_hip_qscale* xs_dev, int xs_step, int64_t groups,
+                           const int64_t* off_dev, const kt_hip_moe_weights* w, const int64_t* silu_codes_dev,
+                           const kt_hip_codelut* silu, void* ws_dev, size_t ws_bytes, int32_t* y_dev,
+                           kt_hip_qscale* ys_dev, void* stream);
 /* MoeMlp's bucket (layers.rs:928-937, forward_one_int's expert calls for every token) on the device: the tokens x
  * top_k pairs of sel_dev (expert ids, as kt_hip_ref_moe_route writes them) grouped by expert for
  * kt_hip_quant_linear_rows -- off_dev (experts + 1 offsets), xidx_dev (row -> token), pos_dev (pair t * top_k + i ->

@@ -145,6 +145,9 @@ def _declare(L: C.CDLL) -> None:
                                           _P, _P, _SZ, _P, _P, _P]),
         "kt_hip_ref_moe_route": (_I, [_I, _P, _I64, _I64, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
         "kt_hip_ref_moe_combine": (_I, [_I, _P, _P, _I64, _I64, _P, _P, _P, _I64, _I, _P, _P, _P]),
+        "kt_hip_ref_moe_experts_workspace": (_SZ, [_I64, _I64, _I64, _I64]),
+        "kt_hip_ref_moe_experts": (_I, [_I, _P, _P, _I64, _I64, _I64, _I64, _P, _I, _I64, _P, _P, _P, _P, _P, _SZ, _P,
+                                        _P, _P]),
         "kt_hip_ref_moe_bucket": (_I, [_I, _P, _I64, _I, _I64, _P, _P, _P, _P]),
         "kt_hip_quant_linear_multi": (_I, [_I, _P, _I64, _I64, _P, _I, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P,
                                             _SZ, _P, _P, _P]),
@@ -989,6 +992,30 @@ def ref_moe_route(logits_dev, tokens: int, experts: int, top_k: int, ls_dev, sig
     check(lib().kt_hip_ref_moe_route(dev, _ptr(logits_dev), tokens, experts, top_k, _ptr(ls_dev), int(sigmoid),
                                      int(norm_topk), _ptr(codes_dev), C.byref(lut), _ptr(bias_dev), _ptr(sel_dev),
                                      _ptr(ec_dev), _ptr(sumc_dev), _stream(stream)), "ref moe route")
+
+
+class MoeWeights(C.Structure):
+    """kt_hip_moe_weights: the routed experts' tiled planes (gate over up, and down) and per-expert Scales."""
+
+    _fields_ = [("gu_planes", _P), ("down_planes", _P), ("gu_group_bytes", _SZ), ("down_group_bytes", _SZ),
+                ("gate_mant", _P), ("up_mant", _P), ("down_mant", _P), ("gate_shift", _P), ("up_shift", _P),
+                ("down_shift", _P), ("gu_pw", C.c_int32), ("down_pw", C.c_int32)]
+
+
+def ref_moe_experts_workspace(rows: int, dim: int, hidden: int, groups: int) -> int:
+    """Bytes of ref_moe_experts' workspace; 0 where it does not take the shape (hidden > 4096)."""
+    return lib().kt_hip_ref_moe_experts_workspace(rows, dim, hidden, groups)
+
+
+def ref_moe_experts(x_dev, xidx_dev, x_rows: int, rows: int, dim: int, hidden: int, xs_dev, xs_step: int, groups: int,
+                    off_dev, weights: MoeWeights, silu_codes_dev, silu: CodeLut, ws_dev, ws_bytes: int, y_dev, ys_dev,
+                    stream=None, dev: int = 0) -> None:
+    """The routed experts (gate, up, SiLU * up, down) of rows grouped by expert, as quant_linear_rows three times around
+    ref_swiglu. `weights` holds addresses: its tensors must outlive the call."""
+    check(lib().kt_hip_ref_moe_experts(dev, _ptr(x_dev), _ptr(xidx_dev), x_rows, rows, dim, hidden, _ptr(xs_dev),
+                                       xs_step, groups, _ptr(off_dev), C.byref(weights), _ptr(silu_codes_dev),
+                                       C.byref(silu), _ptr(ws_dev), ws_bytes, _ptr(y_dev), _ptr(ys_dev),
+                                       _stream(stream)), "ref moe experts")
 
 
 def ref_moe_combine(y_dev, ys_dev, y_rows: int, dim: int, pos_dev, ec_dev, sumc_dev, tokens: int, top_k: int, out_dev,

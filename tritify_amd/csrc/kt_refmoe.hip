@@ -13,12 +13,16 @@
 //   rm_combine                          MoeMlp::combine, one token per CTA (layers.rs:893-923)
 //   rm_merge_*                          merge_rows, the sequence's per-token outputs at one scale (layers.rs:873-891)
 //
-// The SwiGLU between the products is rd_swiglu_kernel (kt_refdec.hip) run one row per CTA, and the shared expert is a
+//   rq_act                              the SwiGLU between the experts' products (layers.rs:615-637) and down's
+//                                       quantization
+//
+// Experts wider than rq_act takes use rd_swiglu_kernel (kt_refdec.hip) one row per CTA, and the shared expert is a
 // whole-tensor SwiGluMlp added with rd_add (layers.rs:757-780, 121-136).
 #include <hip/hip_runtime.h>
 #include <limits.h>
 #include <stdint.h>
 
+#include "kt_dpp.h"
 #include "kt_kernels.h"
 #include "kt_scale_dev.h"
 #include "kt_w12_core.h"
@@ -102,6 +106,7 @@ __device__ __forceinline__ int64_t rq_a_off(int64_t ti, int64_t nkt, int p, int 
 
 // Row r: xmax of its input row, quant_to into 3 balanced base-256 planes (tiled as rq_a_off), and its record:
 // c = from_ratio(xmax, WLEVELS) * xs * ws_g (QuantLinear::forward_int steps 1-4).
+// Without wm the record stops at from_ratio(xmax, WLEVELS) * xs, for a product whose outputs are of several weights.
 __global__ __launch_bounds__(RQ_ROW_THREADS) void rq_quant_kernel(const int32_t* __restrict__ x,
                                                                   const int32_t* __restrict__ xidx, int64_t x_rows,
                                                                   int64_t in, int64_t kp,
@@ -149,7 +154,8 @@ __global__ __launch_bounds__(RQ_ROW_THREADS) void rq_quant_kernel(const int32_t*
             s.mode = 1;
         } else {
             const kt_hip_qscale* xrec = xs + (int64_t)xs_step * r;
-            const Sc c = sc_mul(sc_mul(from_ratio((u128)m, (u128)WLEVELS), rec_sc(xrec)), Sc{wm[g], wsh[g]});
+            Sc c = sc_mul(from_ratio((u128)m, (u128)WLEVELS), rec_sc(xrec));
+            if (wm) c = sc_mul(c, Sc{wm[g], wsh[g]});
             s.c_mant = c.mant, s.c_shift = c.shift, s.mode = c.mant == 0 ? 2 : 0;
         }
         st[r] = s;
@@ -263,6 +269,125 @@ __global__ __launch_bounds__(RQ_ROW_THREADS) void rq_requant_kernel(const int64_
             o.mant = sc.mant, o.shift = sc.shift, o.ymax = ymax;
         }
         ys[r] = o;
+    }
+}
+
+// The experts between their products: row r's gate and up sums (acc row r: hidden gate outputs, then hidden up, in
+// `splits` slices) -> each one's requant_dyn by its own maximum, SiLU(gate) * up through the table, its requant_dyn
+// (SwiGluMlp::forward_int, layers.rs:615-637), and the down product's input: quant_to of those codes, whose largest is
+// 2^28 (so it is a shift), into the down planes (tiled as rq_a_off), with the row's down record. The same integers as
+// rq_requant for gate and for up, the SwiGLU of the row and rq_quant for down in one launch, with no codes in memory
+// between them (64 tokens x top 4, hidden 1408: 10.6 + 10.6 + 8.7 + 6.9 -> 14.6 us). One CTA per row: a row's three
+// maxima and its Scales are a serial chain that bounds it, not its 22 KB of sums a slice. hidden <= RQ_ACT_MAX, what
+// the threads hold in registers; the caller runs wider experts as the separate calls.
+constexpr int RQ_ACT_VPT = 4, RQ_ACT_MAX = RQ_ROW_THREADS * RQ_ACT_VPT;
+struct RqAct {
+    const int64_t *gm, *um, *dm;  // per-group weight Scales: gate, up, down
+    const int32_t *gsh, *ush, *dsh;
+    const int64_t* silu;
+    kt_hip_codelut lut;
+};
+__global__ __launch_bounds__(RQ_ROW_THREADS) void rq_act_kernel(const int64_t* __restrict__ acc, int64_t rows,
+                                                                int hidden, int splits, const RqState* __restrict__ st, RqAct w,
+                                                                int groups, const int64_t* __restrict__ off,
+                                                                const int32_t* __restrict__ tb, int64_t cap,
+                                                                RqState* __restrict__ st2, int8_t* __restrict__ xa) {
+    __shared__ int64_t red[2][RQ_ROW_THREADS / 64];
+    __shared__ int64_t ymax[2];  // gate's and up's maximum, 0 where the output is Scale::ZERO
+    __shared__ Sc par[3];        // index factor, identity factor, h scale
+    const int tid = threadIdx.x;
+    const int64_t r = blockIdx.x, slice = rows * 2 * hidden;
+    const int64_t* a = acc + r * 2 * hidden;
+    int64_t v[2][RQ_ACT_VPT];  // gate, up
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int i = 0; i < RQ_ACT_VPT; i++) v[h][i] = 0;
+    for (int q = 0; q < splits; q++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int i = 0; i < RQ_ACT_VPT; i++) {
+                const int c = tid + RQ_ROW_THREADS * i;
+                if (RQ_ROW_THREADS * i < hidden)  // a block of columns past the row, the same for the whole CTA
+                    v[h][i] = wadd(v[h][i], a[q * slice + (int64_t)h * hidden + (c < hidden ? c : hidden - 1)]);
+            }
+    const RqState s = st[r];
+    const int g = group_of(off, groups, r);
+    int64_t ym[2] = {0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int i = 0; i < RQ_ACT_VPT; i++) ym[h] = iabs(v[h][i]) > ym[h] ? iabs(v[h][i]) : ym[h];
+    // both maxima over the CTA: each wave's by DPP, then the waves'
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        ym[h] = wave_max_i64(ym[h]);
+        if ((tid & 63) == 0) red[h][tid >> 6] = ym[h];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+        for (int q = 0; q < RQ_ROW_THREADS / 64; q++) ym[h] = red[h][q] > ym[h] ? red[h][q] : ym[h];
+    // each output's Scale product (zeros at Scale::ZERO for a zero input, a zero product or zero sums)
+    const Sc c0{s.c_mant, s.c_shift};
+    if (tid == 0 || tid == 64) {
+        const int h = tid >> 6;
+        const Sc c = s.mode == 0 ? sc_mul(c0, h ? Sc{w.um[g], w.ush[g]} : Sc{w.gm[g], w.gsh[g]}) : Sc{0, 0};
+        const bool live = c.mant != 0 && ym[h] > 0;
+        const Sc y = live ? sc_mul(from_ratio((u128)(uint64_t)ym[h], (u128)ACT_LEVELS), c) : Sc{0, 0};
+        const Sc cs{w.lut.code_mant, w.lut.code_shift};
+        ymax[h] = live ? ym[h] : 0;
+        if (h == 0) par[0] = sc_mul(y, Sc{w.lut.inv_mant, w.lut.inv_shift}), par[1] = sc_mul(y, sc_recip(cs));
+        else par[2] = sc_mul(cs, y);
+    }
+    __syncthreads();
+    const Sc mi = par[0], idf = par[1];
+    const int64_t gmax = ymax[0], umax = ymax[1];
+    const RqDen dg = rq_den(gmax), du = rq_den(umax);
+    int64_t hv[RQ_ACT_VPT], m = 0;
+#pragma unroll
+    for (int i = 0; i < RQ_ACT_VPT; i++) {
+        hv[i] = 0;
+        if (tid + RQ_ROW_THREADS * i >= hidden) continue;
+        const int32_t gd = gmax ? rq_apply(dg, v[0][i]) : 0, ud = umax ? rq_apply(du, v[1][i]) : 0;
+        const int64_t idx = sc_apply32(mi, gd) - w.lut.lo_index;
+        const int64_t at = idx < 0 ? 0 : (idx > w.lut.n - 1 ? w.lut.n - 1 : idx);
+        const int64_t code = idx < 0 ? 0 : (idx >= w.lut.n ? sc_apply32(idf, gd) : w.silu[at]);
+        hv[i] = wmul(code, ud);
+        m = iabs(hv[i]) > m ? iabs(hv[i]) : m;
+    }
+    const int64_t hmax = block_max_t(m, red[0]);
+    const RqDen dh = rq_den(hmax);
+    if (tid == 0) {
+        RqState t{};
+        t.mode = 1;
+        if (hmax != 0) {
+            const Sc hs = sc_mul(from_ratio((u128)(uint64_t)hmax, (u128)ACT_LEVELS), par[2]);
+            const Sc c = sc_mul(sc_mul(from_ratio((u128)ACT_LEVELS, (u128)WLEVELS), hs), Sc{w.dm[g], w.dsh[g]});
+            t.xmax = ACT_LEVELS, t.c_mant = c.mant, t.c_shift = c.shift, t.mode = c.mant == 0 ? 2 : 0;
+        }
+        st2[r] = t;
+    }
+    const int64_t j = r - off[g], ti = tb[g] + j / RQ_BM, kp = (hidden + 63) / 64 * 64, nkt = kp / RQ_BK;
+    const int rr = (int)(j % RQ_BM);
+    if (ti >= cap) return;  // never, by the table's capacity
+#pragma unroll
+    for (int i = 0; i < RQ_ACT_VPT; i++) {
+        const int c = tid + RQ_ROW_THREADS * i;
+        if (c >= kp) continue;
+        int64_t q = 0;
+        if (hmax != 0 && c < hidden) {  // quant_to(code, 2^28) = round_half_away(code WLEVELS / 2^28)
+            const int64_t code = rq_apply(dh, hv[i]);
+            const uint64_t u = ((uint64_t)(code < 0 ? -code : code) * (uint64_t)WLEVELS + (1u << 27)) >> 28;
+            q = code < 0 ? -(int64_t)u : (int64_t)u;
+        }
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            const int64_t d = ((q + 128) & 255) - 128;
+            xa[rq_a_off(ti, nkt, p, rr, c)] = (int8_t)d;
+            q = (q - d) >> 8;
+        }
     }
 }
 
@@ -813,6 +938,14 @@ static hipError_t rq_product(const int8_t* xa, int64_t rows, int64_t kp, const i
     return hipGetLastError();
 }
 
+static hipError_t rq_product_pw(int pw, const int8_t* xa, int64_t rows, int64_t kp, const int8_t* wb, size_t wgroup,
+                                int64_t* acc, int64_t N, const int64_t* off_s, const int2* em, const int32_t* hdr,
+                                int64_t cap, int S, hipStream_t s) {
+    return pw == 1   ? rq_product<1>(xa, rows, kp, wb, wgroup, acc, N, off_s, em, hdr, cap, S, s)
+           : pw == 3 ? rq_product<3>(xa, rows, kp, wb, wgroup, acc, N, off_s, em, hdr, cap, S, s)
+                     : rq_product<5>(xa, rows, kp, wb, wgroup, acc, N, off_s, em, hdr, cap, S, s);
+}
+
 hipError_t launch_quant_linear_rows(const int32_t* x, const int32_t* xidx, int64_t x_rows, int64_t rows, int64_t in,
                                     const kt_hip_qscale* xs, int xs_step, int groups, const int64_t* off_dev,
                                     const int8_t* wb, size_t wgroup, int pw, int64_t out, const int64_t* wm_dev,
@@ -835,11 +968,64 @@ hipError_t launch_quant_linear_rows(const int32_t* x, const int32_t* xidx, int64
                                                               tb, cap, wm_dev, wsh_dev, st, xa);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    e = pw == 1   ? rq_product<1>(xa, rows, kp, wb, wgroup, acc, out, off_s, em, hdr, cap, S, s)
-        : pw == 3 ? rq_product<3>(xa, rows, kp, wb, wgroup, acc, out, off_s, em, hdr, cap, S, s)
-                  : rq_product<5>(xa, rows, kp, wb, wgroup, acc, out, off_s, em, hdr, cap, S, s);
+    e = rq_product_pw(pw, xa, rows, kp, wb, wgroup, acc, out, off_s, em, hdr, cap, S, s);
     if (e != hipSuccess) return e;
     rq_requant_kernel<<<(unsigned)rows, RQ_ROW_THREADS, 0, s>>>(acc, rows, out, S, st, y, ys);
+    return hipGetLastError();
+}
+
+// The routed experts in six launches: one tile plan and one quantization of x for gate and up, whose 2 hidden outputs
+// are one product (64 tokens x top 4 of 16 experts, 2048 -> 1408: two of 37 us -> one of 61, its CTAs twice as many and
+// the ragged end once), rq_act, down's product on the same plan, its requantization. The layer: 352 -> 290 us.
+// The experts' workspace: the x planes, the down planes, the sums of either product (one after the other), the two
+// row records, the offsets with each group's first tile, the tile table.
+size_t rm_experts_workspace_bytes(int64_t rows, int64_t dim, int64_t hidden, int64_t groups, size_t off[7]) {
+    const int64_t kp1 = (dim + 63) / 64 * 64, kp2 = (hidden + 63) / 64 * 64, fk = kt_hip_flush_k(3, 3);
+    const size_t cap = (size_t)rq_tile_cap(rows, groups);
+    const size_t a1 = (size_t)rq_splits(rows, groups, 2 * hidden, kp1, fk) * (size_t)rows * 2 * (size_t)hidden * 8;
+    const size_t a2 = (size_t)rq_splits(rows, groups, dim, kp2, fk) * (size_t)rows * (size_t)dim * 8;
+    const size_t sizes[7] = {cap * RQ_BM * 3 * (size_t)kp1, cap * RQ_BM * 3 * (size_t)kp2, a1 > a2 ? a1 : a2,
+                             (size_t)rows * sizeof(RqState), (size_t)rows * sizeof(RqState),
+                             (size_t)(groups + 1) * 8 + (size_t)groups * 4, 16 + 8 * cap};
+    size_t at = 0;
+    for (int i = 0; i < 7; i++) {
+        off[i] = at;
+        at += (sizes[i] + 255) / 256 * 256;
+    }
+    return at;
+}
+
+hipError_t launch_rm_experts(const int32_t* x, const int32_t* xidx, int64_t x_rows, int64_t rows, int64_t dim,
+                             int64_t hidden, const kt_hip_qscale* xs, int xs_step, int groups, const int64_t* off_dev,
+                             const int8_t* wgu, size_t gu_group, int pw_gu, const int8_t* wd, size_t d_group, int pw_d,
+                             const RqAct& act, void* ws, int32_t* y, kt_hip_qscale* ys, hipStream_t s) {
+    size_t off[7];
+    rm_experts_workspace_bytes(rows, dim, hidden, groups, off);
+    const int64_t cap = rq_tile_cap(rows, groups), kp1 = (dim + 63) / 64 * 64, kp2 = (hidden + 63) / 64 * 64;
+    const int S1 = rq_splits(rows, groups, 2 * hidden, kp1, kt_hip_flush_k(3, pw_gu));
+    const int S2 = rq_splits(rows, groups, dim, kp2, kt_hip_flush_k(3, pw_d));
+    char* base = (char*)ws;
+    int8_t *xa = (int8_t*)(base + off[0]), *ha = (int8_t*)(base + off[1]);
+    int64_t* acc = (int64_t*)(base + off[2]);
+    RqState *st = (RqState*)(base + off[3]), *st2 = (RqState*)(base + off[4]);
+    int64_t* off_s = (int64_t*)(base + off[5]);
+    int32_t* tb = (int32_t*)(off_s + groups + 1);
+    int32_t* hdr = (int32_t*)(base + off[6]);
+    int2* em = (int2*)(hdr + 4);
+    rq_plan_kernel<<<1, 1024, 0, s>>>(off_dev, groups, rows, off_s, tb, hdr, em, cap);
+    rq_quant_kernel<<<(unsigned)rows, RQ_ROW_THREADS, 0, s>>>(x, xidx, x_rows, dim, kp1, xs, xs_step, groups, off_s, tb,
+                                                              cap, nullptr, nullptr, st, xa);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    e = rq_product_pw(pw_gu, xa, rows, kp1, wgu, gu_group, acc, 2 * hidden, off_s, em, hdr, cap, S1, s);
+    if (e != hipSuccess) return e;
+    rq_act_kernel<<<(unsigned)rows, RQ_ROW_THREADS, 0, s>>>(acc, rows, (int)hidden, S1, st, act, groups, off_s, tb, cap,
+                                                            st2, ha);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    e = rq_product_pw(pw_d, ha, rows, kp2, wd, d_group, acc, dim, off_s, em, hdr, cap, S2, s);
+    if (e != hipSuccess) return e;
+    rq_requant_kernel<<<(unsigned)rows, RQ_ROW_THREADS, 0, s>>>(acc, rows, dim, S2, st2, y, ys);
     return hipGetLastError();
 }
 
@@ -937,6 +1123,49 @@ extern "C" int kt_hip_quant_linear_rows(int dev, const int32_t* x_dev, const int
     return (int)kt::launch_quant_linear_rows(x_dev, xidx_dev, x_rows, rows, in_f, xs_dev, xs_step, (int)groups,
                                              off_dev, w_planes_dev, w_group_bytes, pw, out_f, w_mant_dev, w_shift_dev,
                                              kt_hip_flush_k(3, pw), ws_dev, y_dev, ys_dev, (hipStream_t)stream);
+}
+
+extern "C" size_t kt_hip_ref_moe_experts_workspace(int64_t rows, int64_t dim, int64_t hidden, int64_t groups) {
+    size_t off[7];
+    if (rows < 1 || dim < 1 || hidden < 1 || hidden > kt::RQ_ACT_MAX || groups < 1 || groups > INT32_MAX - 1) return 0;
+    return kt::rm_experts_workspace_bytes(rows, dim, hidden, groups, off);
+}
+
+extern "C" int kt_hip_ref_moe_experts(int dev, const int32_t* x_dev, const int32_t* xidx_dev, int64_t x_rows,
+                                      int64_t rows, int64_t dim, int64_t hidden, const kt_hip_qscale* xs_dev,
+                                      int xs_step, int64_t groups, const int64_t* off_dev,
+                                      const kt_hip_moe_weights* w, const int64_t* silu_codes_dev,
+                                      const kt_hip_codelut* silu, void* ws_dev, size_t ws_bytes, int32_t* y_dev,
+                                      kt_hip_qscale* ys_dev, void* stream) {
+    if (!x_dev || !xs_dev || !off_dev || !w || !silu_codes_dev || !silu || silu->n < 1 || !silu->right_identity ||
+        !ws_dev || !y_dev || !ys_dev || rows < 1 || rows > INT32_MAX || dim < 1 || dim > INT32_MAX || hidden < 1 ||
+        hidden > kt::RQ_ACT_MAX || x_rows < 1 || groups < 1 || groups > INT32_MAX - 1 || (xs_step != 0 && xs_step != 1))
+        return (int)hipErrorInvalidValue;
+    if (!w->gu_planes || !w->down_planes || !w->gate_mant || !w->gate_shift || !w->up_mant || !w->up_shift ||
+        !w->down_mant || !w->down_shift || (w->gu_pw != 1 && w->gu_pw != 3 && w->gu_pw != 5) ||
+        (w->down_pw != 1 && w->down_pw != 3 && w->down_pw != 5))
+        return (int)hipErrorInvalidValue;
+    const int64_t kp1 = (dim + 63) / 64 * 64, kp2 = (hidden + 63) / 64 * 64;
+    if (rows * kp1 * 3 >= ((int64_t)1 << 40) || rows * hidden >= ((int64_t)1 << 31) ||
+        rows * dim >= ((int64_t)1 << 31) || kp1 > INT_MAX)
+        return (int)hipErrorInvalidValue;
+    if (ws_bytes < kt_hip_ref_moe_experts_workspace(rows, dim, hidden, groups) ||
+        w->gu_group_bytes < kt::rq_tiled_bytes(2 * hidden, dim, w->gu_pw) ||
+        w->down_group_bytes < kt::rq_tiled_bytes(dim, hidden, w->down_pw) ||
+        (int64_t)w->gu_pw * kt::RQ_BN * kp1 >= ((int64_t)1 << 32))
+        return (int)hipErrorInvalidValue;
+    const int64_t cap = kt::rq_tile_cap(rows, groups);
+    const int64_t S1 = kt::rq_splits(rows, groups, 2 * hidden, kp1, kt_hip_flush_k(3, w->gu_pw));
+    const int64_t S2 = kt::rq_splits(rows, groups, dim, kp2, kt_hip_flush_k(3, w->down_pw));
+    if ((2 * hidden + kt::RQ_BN - 1) / kt::RQ_BN * cap * S1 > INT32_MAX ||
+        (dim + kt::RQ_BN - 1) / kt::RQ_BN * cap * S2 > INT32_MAX)
+        return (int)hipErrorInvalidValue;
+    RM_TRY(hipSetDevice(dev));
+    const kt::RqAct act{w->gate_mant, w->up_mant, w->down_mant, w->gate_shift, w->up_shift, w->down_shift,
+                        silu_codes_dev, *silu};
+    return (int)kt::launch_rm_experts(x_dev, xidx_dev, x_rows, rows, dim, hidden, xs_dev, xs_step, (int)groups, off_dev,
+                                      w->gu_planes, w->gu_group_bytes, w->gu_pw, w->down_planes, w->down_group_bytes,
+                                      w->down_pw, act, ws_dev, y_dev, ys_dev, (hipStream_t)stream);
 }
 
 extern "C" size_t kt_hip_pack_planes_tiled_bytes(int64_t rows, int64_t k, int planes) {

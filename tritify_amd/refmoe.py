@@ -9,9 +9,9 @@ groups only the exact integer products:
   router                   kt_hip_quant_linear_rows (one group: every token row quantized on its own)
   route / route_sigmoid    kt_hip_ref_moe_route     (exp or sigmoid CodeLut numerators, top-k, sumc)
   bucket                   kt_hip_ref_moe_bucket    (the (token, expert) rows ordered by expert, on the device)
-  experts gate / up        kt_hip_quant_linear_rows (E groups; x rows by index)
-  SiLU * up                kt_hip_ref_swiglu        (one row per (token, expert))
-  experts down             kt_hip_quant_linear_rows (E groups; per-row input scales)
+  experts                  kt_hip_ref_moe_experts   (gate and up as one product of E groups, x rows by index; SiLU * up
+                           and down's quantization per (token, expert) row; down's product); experts of more than
+                           4096 hidden features: kt_hip_quant_linear_rows for each and kt_hip_ref_swiglu
   combine                  kt_hip_ref_moe_combine   (per token: common scale, ec-weighted sum, 1/sumc)
   merge_rows               kt_hip_ref_merge_rows    (a sequence: the tokens at one scale)
   shared expert + add      kt_hip_quant_linear(_multi), kt_hip_ref_swiglu_seq, kt_hip_ref_add_seq (the whole tensor, many
@@ -53,7 +53,20 @@ class RefMoeLayer:
         i64 = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.int64)).to(d)  # noqa: E731
         i32 = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).to(d)  # noqa: E731
         self.router = self._pack_groups([router])
-        self.w = {n: self._pack_groups([e[n] for e in experts]) for n in ("gate", "up", "down")}
+        # one product over gate's and up's outputs where kt_hip_ref_moe_experts takes the width (else each on its own)
+        self.fused = B.ref_moe_experts_workspace(1, self.dim, self.hidden, 1) > 0
+        if self.fused:
+            gu = self._pack_groups([e["gate"] for e in experts], [e["up"] for e in experts])
+            down = self._pack_groups([e["down"] for e in experts])
+            up = [e["up"][1] for e in experts]
+            gu["up_mant"], gu["up_shift"] = i64([int(m) for m, _ in up]), i32([int(s) for _, s in up])
+            self.w = {"gu": gu, "down": down}
+            p = lambda t: t.data_ptr()  # noqa: E731
+            self.experts = B.MoeWeights(p(gu["planes"]), p(down["planes"]), gu["gbytes"], down["gbytes"],
+                                        p(gu["mant"]), p(gu["up_mant"]), p(down["mant"]), p(gu["shift"]),
+                                        p(gu["up_shift"]), p(down["shift"]), gu["pw"], down["pw"])
+        else:
+            self.w = {n: self._pack_groups([e[n] for e in experts]) for n in ("gate", "up", "down")}
         self.sigmoid = sigmoid_bias is not None
         if self.sigmoid:
             codes, self.route_lut = B.ref_codelut(B.LUT_SIGMOID, -16.0, 16.0, 16, 20, False)
@@ -80,17 +93,21 @@ class RefMoeLayer:
         self._i32 = i32
         self._route_off = {}  # T -> the router's one-group offsets [0, T] on the device
 
-    def _pack_groups(self, mats):
+    def _pack_groups(self, mats, below=None):
         """Digit planes of each (codes out x in, scale) in one buffer (all at the largest plane count, in the grouped
-        product's tiled layout), with the per-group Scales on the device."""
+        product's tiled layout), with the per-group Scales on the device. below: a second matrix per group whose rows
+        follow the first's."""
         torch = self.torch
-        codes = [np.ascontiguousarray(m[0], dtype=np.int32) for m in mats]
-        out, inp = codes[0].shape
-        pw = max(B.planes_for(c) for c in codes)
+        inp = np.asarray(mats[0][0]).shape[1]
+        parts = [[np.ascontiguousarray(m[0], dtype=np.int32) for m in (ms if below else ms[:1])]
+                 for ms in zip(mats, below or mats)]
+        out = sum(c.shape[0] for c in parts[0])
+        pw = max(B.planes_for(c) for cs in parts for c in cs)
         gbytes = B.pack_planes_tiled_bytes(out, inp, pw)
-        planes = torch.empty(len(codes) * gbytes, dtype=torch.int8, device=self.device)
-        for g, c in enumerate(codes):
-            B.pack_planes_tiled(torch.from_numpy(c.reshape(-1)).to(self.device), out, inp, pw, planes[g * gbytes:],
+        planes = torch.empty(len(parts) * gbytes, dtype=torch.int8, device=self.device)
+        for g, cs in enumerate(parts):
+            codes = [torch.from_numpy(c.reshape(-1)).to(self.device) for c in cs]
+            B.pack_planes_tiled(torch.cat(codes) if below else codes[0], out, inp, pw, planes[g * gbytes:],
                                 dev=self.dev)
         mant = torch.from_numpy(np.array([int(m[1][0]) for m in mats], np.int64)).to(self.device)
         shift = torch.from_numpy(np.array([int(m[1][1]) for m in mats], np.int32)).to(self.device)
@@ -156,12 +173,20 @@ class RefMoeLayer:
         sel, ec, sumc, _, _ = self.route(x_dev, xs_rec, T, stream)
         P = T * K
         off_d, xidx_d, pos_d = self.bucket(sel, T, stream)
-        g, gs = self._rows_ql(self.w["gate"], x_dev, xidx_d, T, P, xs_rec, 0, off_d, E, stream)
-        u, us = self._rows_ql(self.w["up"], x_dev, xidx_d, T, P, xs_rec, 0, off_d, E, stream)
-        h = torch.empty(P * self.hidden, dtype=torch.int32, device=self.device)
-        hs = torch.empty(P * 4, dtype=torch.int64, device=self.device)  # (every record below is written whole)
-        B.ref_swiglu(g, gs, u, us, self.hidden, self.silu_codes, self.silu_lut, h, hs, stream, self.dev, rows=P)
-        y, ys = self._rows_ql(self.w["down"], h, None, P, P, hs, 1, off_d, E, stream)
+        if self.fused:
+            n = B.ref_moe_experts_workspace(P, dim, self.hidden, E)
+            ws = torch.empty(n, dtype=torch.uint8, device=self.device)
+            y = torch.empty(P * dim, dtype=torch.int32, device=self.device)
+            ys = torch.empty(P * 4, dtype=torch.int64, device=self.device)  # (every record below is written whole)
+            B.ref_moe_experts(x_dev, xidx_d, T, P, dim, self.hidden, xs_rec, 0, E, off_d, self.experts,
+                              self.silu_codes, self.silu_lut, ws, n, y, ys, stream=stream, dev=self.dev)
+        else:
+            g, gs = self._rows_ql(self.w["gate"], x_dev, xidx_d, T, P, xs_rec, 0, off_d, E, stream)
+            u, us = self._rows_ql(self.w["up"], x_dev, xidx_d, T, P, xs_rec, 0, off_d, E, stream)
+            h = torch.empty(P * self.hidden, dtype=torch.int32, device=self.device)
+            hs = torch.empty(P * 4, dtype=torch.int64, device=self.device)
+            B.ref_swiglu(g, gs, u, us, self.hidden, self.silu_codes, self.silu_lut, h, hs, stream, self.dev, rows=P)
+            y, ys = self._rows_ql(self.w["down"], h, None, P, P, hs, 1, off_d, E, stream)
         rows = torch.empty(T * dim, dtype=torch.int32, device=self.device)
         rs = torch.empty(T * 4, dtype=torch.int64, device=self.device)
         B.ref_moe_combine(y, ys, P, dim, pos_d, ec, sumc, T, K, rows, rs, stream=stream, dev=self.dev)
