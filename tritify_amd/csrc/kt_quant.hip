@@ -237,61 +237,67 @@ __global__ __launch_bounds__(QL_THREADS) void ql_quant_kernel(const int32_t* __r
 
 // One row (the decode step): the quant pass and the digit product in one launch. Every CTA takes max |x| over the
 // row and forms the row's three digit planes in LDS itself (at most MAXKP values, read from L2 by each CTA) while
-// its first weight chunks are in flight, then runs the product of plane_skinny_kernel over its 8 output columns
+// all of its weights are in flight, then runs the product of plane_skinny_kernel over its 8 output columns
 // (4 waves x 2 columns, the lanes striding k in 16-byte chunks, int32 plane-group sums by sdot4, a butterfly across
-// the wave). The CTA's largest |result| goes to its own slot part[blockIdx.x] (overwritten on every call, so no
-// pass has to clear it); ql_requant_kernel takes each segment's maximum over its CTAs' slots. CTA 0 writes each
+// the wave); with KS > 1, KS groups of 4 waves take the k chunks in turn and their sums (int32, the whole row within
+// the flush bound) are added in LDS. The CTA's largest |result| goes to its own slot part[blockIdx.x] (overwritten on
+// every call, so no pass has to clear it); ql_requant_kernel takes each segment's maximum over its CTAs' slots. CTA 0 writes each
 // segment's state for ql_requant_kernel. A CTA whose segment has a bias forms the bias factor itself. Requires
 // kp <= MAXKP and a single k-chunk (kp within the flush bound). launch_ql_impl takes this path for outputs of at
 // most QS_FUSED_OUT columns: rows up to QS_MAX_KP values, and for 3 weight planes rows up to QS_LONG_KP values in an
-// instantiation with the larger LDS image (the 4864-value down row: 13.6 us against 8.8 + 9.0 for the quant pass and
-// the product; the small instantiation keeps the short rows' registers and LDS low).
+// instantiation with the larger LDS image, where one wave per SIMD quantizing 32 values a thread and then waiting for
+// one weight chunk after another is the time: 4 k slices give 8 values a thread and every chunk in flight at once (the
+// 4864-value down row, 896 columns: 12.1 -> 10.6 us, 8.7 with half the columns a CTA).
 constexpr int QS_MAX_KP = 1024, QS_LONG_KP = 8192;
 constexpr int64_t QS_FUSED_OUT = 16384;
 constexpr int QS_THREADS = 256, QS_WAVES = QS_THREADS / 64;
-constexpr int QS_CPW = 2;  // output columns per wave
-constexpr int QS_COLS = QS_WAVES * QS_CPW;
+constexpr int QS_COLS = QS_WAVES * 2;  // a CTA's columns (CPW = 2 per wave); long rows of few columns take CPW = 1
 
-template <int PW, int MAXKP>
-__global__ __launch_bounds__(QS_THREADS) void ql_skinny_kernel(const int32_t* __restrict__ x, int in, int kp,
+template <int PW, int MAXKP, int KS, int CPW>
+__global__ __launch_bounds__(QS_THREADS * KS) void ql_skinny_kernel(const int32_t* __restrict__ x, int in, int kp,
                                                                const kt_hip_qscale* __restrict__ xs,
                                                                const int8_t* __restrict__ wb, int64_t* __restrict__ y,
                                                                int N, const int64_t* __restrict__ bias, QlSeg seg,
                                                                QlScales sc, QlState* __restrict__ st,
                                                                int64_t* __restrict__ part) {
-    constexpr int NG = 3 + PW - 1, QPT = MAXKP / 4 / QS_THREADS;
+    constexpr int NG = 3 + PW - 1, NT = QS_THREADS * KS, QPT = MAXKP / 4 / NT;
+    constexpr int NIT = MAXKP / 16 / (64 * KS);  // weight chunks per lane
+    static_assert(QPT * 4 * NT == MAXKP && NIT * 64 * KS * 16 == MAXKP, "the row divides over the CTA");
     __shared__ __attribute__((aligned(16))) int8_t xq[3 * MAXKP];
-    __shared__ uint32_t red[QS_WAVES];
+    __shared__ uint32_t red[NT / 64];
+    __shared__ int s_slice[KS > 1 ? KS - 1 : 1][QS_WAVES][CPW * NG];  // the other k slices' sums
     __shared__ int64_t s_max[QS_WAVES];
     __shared__ int64_t s_f[2];  // the bias factor of this CTA's segment (mant, shift), when it has a bias
     __shared__ int s_badd;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nb = ((int)blockIdx.x * QS_WAVES + wave) * QS_CPW;  // the wave's first column
-    const int g = ql_seg_of(seg, (int)blockIdx.x * QS_COLS);
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int wave = wv % QS_WAVES, ks = wv / QS_WAVES;           // the wave's columns, its k slice
+    const int nb = ((int)blockIdx.x * QS_WAVES + wave) * CPW;  // the wave's first column
+    const int g = ql_seg_of(seg, (int)blockIdx.x * QS_WAVES * CPW);
     const size_t wplane = (size_t)N * kp;
     const int nch = kp / 16;
 
-    // the weights of the wave's next chunk; non-temporal loads (read once per call), so the stream does not push the
-    // small tensors the next launches read (the sums, the records, the cache rows) out of the caches
-    v4i wn[QS_CPW][PW];
-    auto wload = [&](int q) {
+    // the wave's weights, chunks lane + 64 (ks + KS it); non-temporal loads (read once per call), so the stream does
+    // not push the small tensors the next launches read (the sums, the records, the cache rows) out of the caches
+    v4i wv4[NIT][CPW][PW];
 #pragma unroll
-        for (int c = 0; c < QS_CPW; c++)
+    for (int it = 0; it < NIT; it++) {  // in flight while the row is quantized
+        const int q = lane + 64 * (ks + KS * it);
+#pragma unroll
+        for (int c = 0; c < CPW; c++)
 #pragma unroll
             for (int j = 0; j < PW; j++)
-                wn[c][j] = q < nch && nb + c < N
-                               ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(
-                                     wb + j * wplane + (size_t)(nb + c) * kp + 16 * (size_t)q))
-                               : v4i{};
-    };
-    wload(lane);  // in flight while the row is quantized
+                wv4[it][c][j] = q < nch && nb + c < N
+                                    ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(
+                                          wb + j * wplane + (size_t)(nb + c) * kp + 16 * (size_t)q))
+                                    : v4i{};
+    }
 
     // the row, 4 columns per quad, QPT quads per thread held in registers; max |x| over the CTA
     int32_t xv[QPT][4];
     uint32_t m = 0;
 #pragma unroll
     for (int k = 0; k < QPT; k++) {
-        const int c0 = 4 * (tid + QS_THREADS * k);
+        const int c0 = 4 * (tid + NT * k);
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             xv[k][t] = c0 + t < in ? x[c0 + t] : 0;
@@ -299,17 +305,17 @@ __global__ __launch_bounds__(QS_THREADS) void ql_skinny_kernel(const int32_t* __
             m = a > m ? a : m;
         }
     }
-    {  // max |x| over the CTA: each wave's by DPP, then the QS_WAVES of them
+    {  // max |x| over the CTA: each wave's by DPP, then all of them
         m = wave_max_u32(m);
-        if (lane == 0) red[wave] = m;
+        if (lane == 0) red[wv] = m;
         __syncthreads();
 #pragma unroll
-        for (int w = 0; w < QS_WAVES; w++) m = red[w] > m ? red[w] : m;
+        for (int w = 0; w < NT / 64; w++) m = red[w] > m ? red[w] : m;
     }
     const double rinv = m != 0 ? 1.0 / (double)m : 0.0;
 #pragma unroll
     for (int k = 0; k < QPT; k++) {
-        const int c0 = 4 * (tid + QS_THREADS * k);
+        const int c0 = 4 * (tid + NT * k);
         if (c0 < kp) {
             uint32_t word[3] = {0, 0, 0};
             if (m != 0) ql_digits4r(xv[k], m, rinv, word);
@@ -334,42 +340,53 @@ __global__ __launch_bounds__(QS_THREADS) void ql_skinny_kernel(const int32_t* __
     }
     __syncthreads();
 
-    int acc[QS_CPW][NG];
+    int acc[CPW][NG];
 #pragma unroll
-    for (int c = 0; c < QS_CPW; c++)
+    for (int c = 0; c < CPW; c++)
 #pragma unroll
         for (int i = 0; i < NG; i++) acc[c][i] = 0;
-    for (int q = lane; q < nch; q += 64) {
-        v4i wv[QS_CPW][PW];
 #pragma unroll
-        for (int c = 0; c < QS_CPW; c++)
-#pragma unroll
-            for (int j = 0; j < PW; j++) wv[c][j] = wn[c][j];
-        wload(q + 64);
+    for (int it = 0; it < NIT; it++) {  // a chunk past the row: digits read within xq, zero weights
+        const int q = lane + 64 * (ks + KS * it);
         v4i xd[3];
 #pragma unroll
         for (int i = 0; i < 3; i++) xd[i] = *reinterpret_cast<const v4i*>(xq + i * kp + 16 * q);
 #pragma unroll
-        for (int c = 0; c < QS_CPW; c++)
+        for (int c = 0; c < CPW; c++)
 #pragma unroll
             for (int i = 0; i < 3; i++)
 #pragma unroll
                 for (int j = 0; j < PW; j++) {
                     int d = acc[c][i + j];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) d = __builtin_amdgcn_sdot4(xd[i][e], wv[c][j][e], d, false);
+                    for (int e = 0; e < 4; e++) d = __builtin_amdgcn_sdot4(xd[i][e], wv4[it][c][j][e], d, false);
                     acc[c][i + j] = d;
                 }
     }
 #pragma unroll
-    for (int c = 0; c < QS_CPW; c++)
+    for (int c = 0; c < CPW; c++)
 #pragma unroll
         for (int i = 0; i < NG; i++) acc[c][i] = wave_sum_i32(acc[c][i]);  // the wave's sums, in every lane
+    if constexpr (KS > 1) {
+        if (ks > 0 && lane == 0)
+#pragma unroll
+            for (int c = 0; c < CPW; c++)
+#pragma unroll
+                for (int i = 0; i < NG; i++) s_slice[ks - 1][wave][c * NG + i] = acc[c][i];
+        __syncthreads();
+        if (ks == 0)
+#pragma unroll
+            for (int k = 0; k < KS - 1; k++)
+#pragma unroll
+                for (int c = 0; c < CPW; c++)
+#pragma unroll
+                    for (int i = 0; i < NG; i++) acc[c][i] += s_slice[k][wave][c * NG + i];
+    }
     int64_t lmax = 0;
-    if (lane == 0) {
+    if (lane == 0 && ks == 0) {
         const bool badd = s_badd != 0;
 #pragma unroll
-        for (int c = 0; c < QS_CPW; c++) {
+        for (int c = 0; c < CPW; c++) {
             const int n = nb + c;
             if (n >= N) continue;
             uint64_t f = badd ? (uint64_t)scale_apply(s_f[0], (int32_t)s_f[1], bias[n]) : 0;
@@ -392,12 +409,13 @@ __global__ __launch_bounds__(QS_THREADS) void ql_skinny_kernel(const int32_t* __
 // y = requant_dyn(acc, ACT_LEVELS, ymax) per segment (layers.rs:33-39, 321-327). The grid's last CTA only writes
 // each segment's record (its Scale products run beside the other CTAs' divisions); the others requantize. Each
 // thread's first accumulator and the segments' states are read before the maximum is known. The
-// one-row product's: the maximum comes from `part`, that product's maximum per CTA of QS_COLS columns.
+// one-row product's: the maximum comes from `part`, that product's maximum per CTA of `cols` columns.
 __global__ __launch_bounds__(QL_THREADS) void ql_requant_kernel(const int64_t* __restrict__ acc, int64_t n,
                                                                 int64_t out, const int64_t* __restrict__ bias,
                                                                 const QlState* __restrict__ st, QlSeg seg,
                                                                 QlScales sc, QlOut yo,
-                                                                const int64_t* __restrict__ part, int nparts) {
+                                                                const int64_t* __restrict__ part, int nparts,
+                                                                int cols) {
     __shared__ int64_t s_ymax[KT_QL_MAX_SEG];
     __shared__ double s_rinv[KT_QL_MAX_SEG];
     __shared__ int32_t s_mode[KT_QL_MAX_SEG];
@@ -427,7 +445,7 @@ __global__ __launch_bounds__(QL_THREADS) void ql_requant_kernel(const int64_t* _
             }
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const int g = ql_seg_of(seg, (c0 + u * QL_THREADS) * QS_COLS);
+                const int g = ql_seg_of(seg, (c0 + u * QL_THREADS) * cols);
 #pragma unroll
                 for (int i = 0; i < KT_QL_MAX_SEG; i++)
                     if (i == g) pm[i] = v[u] > pm[i] ? v[u] : pm[i];
@@ -709,7 +727,13 @@ bool ql_sums_ok(int64_t in, int64_t out, int pw, int64_t flush_k) {
     return in >= 1 && out >= 1 && (kp <= QS_MAX_KP || long_row) && out <= QS_FUSED_OUT && kp <= flush_k &&
            (pw == 1 || pw == 3 || pw == 5);
 }
-// every CTA of QS_COLS columns within one segment
+// The columns of a CTA of that product: QS_COLS, or half of them for a long row whose CTAs of QS_COLS would leave more
+// than half of the 256 CUs without one (4864 -> 896 columns, 112 CTAs or 224: 10.6 or 8.7 us). At most 256 slots then,
+// within part 2 of the workspace.
+static int ql_skinny_cols(int64_t in, int64_t out) {
+    return (in + 63) / 64 * 64 > QS_MAX_KP && out <= 128 * QS_COLS ? QS_COLS / 2 : QS_COLS;
+}
+// every CTA of at most QS_COLS columns within one segment
 static bool ql_seg_cols_ok(const QlSeg& seg) {
     bool ok = true;
     for (int g = 1; g < seg.n; g++) ok = ok && seg.col0[g] % QS_COLS == 0;
@@ -728,13 +752,15 @@ static hipError_t launch_ql_skinny(const int32_t* x, int64_t in, const kt_hip_qs
     QlState* st = (QlState*)(base + off[4]);
     const int64_t kp = (in + 63) / 64 * 64;
     const bool long_row = kp > QS_MAX_KP && kp <= QS_LONG_KP && pw == 3;
-    const int ctas = (int)((out + QS_COLS - 1) / QS_COLS);
-#define KT_QS(P, K) ql_skinny_kernel<P, K><<<ctas, QS_THREADS, 0, s>>>(x, (int)in, (int)kp, xs, wb, acc, (int)out, bias, \
-                                                                      seg, sc, st, pm)
-    if (long_row) KT_QS(3, QS_LONG_KP);
-    else if (pw == 1) KT_QS(1, QS_MAX_KP);
-    else if (pw == 3) KT_QS(3, QS_MAX_KP);
-    else KT_QS(5, QS_MAX_KP);
+    const int cols = ql_skinny_cols(in, out), ctas = (int)((out + cols - 1) / cols);
+#define KT_QS(P, K, S, C)                                                                                            \
+    ql_skinny_kernel<P, K, S, C><<<ctas, QS_THREADS * S, 0, s>>>(x, (int)in, (int)kp, xs, wb, acc, (int)out, bias,  \
+                                                                seg, sc, st, pm)
+    if (long_row && cols < QS_COLS) KT_QS(3, QS_LONG_KP, 4, 1);
+    else if (long_row) KT_QS(3, QS_LONG_KP, 4, 2);
+    else if (pw == 1) KT_QS(1, QS_MAX_KP, 1, 2);
+    else if (pw == 3) KT_QS(3, QS_MAX_KP, 1, 2);
+    else KT_QS(5, QS_MAX_KP, 1, 2);
 #undef KT_QS
     return hipGetLastError();
 }
@@ -768,9 +794,10 @@ static hipError_t launch_ql_impl(const int32_t* x, int64_t rows, int64_t in, con
     if (!geom && !gelu && rows == 1 && ql_sums_ok(in, out, pw, flush_k) && ql_seg_cols_ok(seg)) {
         const hipError_t e = launch_ql_skinny(x, in, xs, wb, pw, out, seg, sc, bias, ws, s);
         if (e != hipSuccess) return e;
-        const int ctas = (int)((out + QS_COLS - 1) / QS_COLS);
+        const int cols = ql_skinny_cols(in, out), ctas = (int)((out + cols - 1) / cols);
         int64_t* pm = reinterpret_cast<int64_t*>(base + off[2]);
-        ql_requant_kernel<<<grid_for(n, 1) + 1, QL_THREADS, 0, s>>>(acc, n, out, bias, st, seg, sc, yo, pm, ctas);
+        ql_requant_kernel<<<grid_for(n, 1) + 1, QL_THREADS, 0, s>>>(acc, n, out, bias, st, seg, sc, yo, pm, ctas,
+                                                                     cols);
         return hipGetLastError();
     }
     // max |x| by its own pass, or inside every quant CTA when x is short (one launch fewer for a decode row)
