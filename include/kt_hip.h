@@ -305,6 +305,16 @@ int kt_hip_ref_swiglu(int dev, const int32_t* g_dev, const kt_hip_qscale* gs_dev
 int kt_hip_ref_swiglu_sums(int dev, const kt_hip_ql_sums* g, const kt_hip_ql_sums* u, int64_t n,
                            const int64_t* silu_codes_dev, const kt_hip_codelut* silu, int32_t* h_dev,
                            kt_hip_qscale* hs_dev, void* stream);
+/* kt_hip_ref_swiglu_sums followed by kt_hip_quant_linear_multi_sums of one call (in_f = n, out_f columns) on its
+ * output, without that output in memory: the SwiGLU's products are formed by many CTAs and requantized by the down
+ * product's. g and u are left as by kt_hip_ref_swiglu_sums (their records written), the down sums in ws_dev as by
+ * kt_hip_quant_linear_multi_sums with that in_f and out_f: the same integers. Requires kt_hip_quant_linear_sums_ok(n,
+ * out_f, pw); ws_dev of kt_hip_quant_linear_swiglu_workspace bytes (0: not this shape), not g's or u's. */
+size_t kt_hip_quant_linear_swiglu_workspace(int64_t n, int64_t out_f, int pw);
+int kt_hip_quant_linear_swiglu_sums(int dev, const kt_hip_ql_sums* g, const kt_hip_ql_sums* u, int64_t n,
+                                    const int64_t* silu_codes_dev, const kt_hip_codelut* silu,
+                                    const int8_t* w_planes_dev, int pw, int64_t out_f, int64_t w_mant, int32_t w_shift,
+                                    void* ws_dev, size_t ws_bytes, void* stream);
 /* apply_gelu (crates/03-models/kt-model-vision/src/nonlin.rs:30-45) of n codes at xs_dev through the GELU CodeLut
  * (KT_LUT_GELU over [-10, 10], 2^16 entries, 2^20 code scale, right_identity set; its codes at gelu_codes_dev): y_dev
  * (may alias x_dev) at the table's code scale, written to ys_dev (which may not alias xs_dev). */

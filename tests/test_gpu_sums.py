@@ -193,3 +193,60 @@ def test_sums_entries_refuse_what_they_cannot_take(torch_dev):
     with pytest.raises(B.HipError):  # 63 values against a 64-value output
         B.ref_add_rmsnorm_sums(y, ys, s, 63, y, ys, h, (1, 0), (1, 0), h, hs)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("mode", ["live", "zero_x", "zero_c", "levels"])
+@pytest.mark.parametrize("inp,n,out,wmax,apart", [(64, 8, 16, WLEVELS, True), (64, 256, 17, WLEVELS, False),
+                                                  (200, 264, 40, 127, True), (96, 250, 24, WLEVELS, True),
+                                                  (896, 4864, 896, WLEVELS, False), (64, 1032, 1032, WLEVELS, True),
+                                                  (1500, 1024, 64, WLEVELS, True), (64, 8192, 9, WLEVELS, False),
+                                                  (64, 900, 33, 2**30, True)])
+def test_swiglu_into_the_down_product_equals_the_two_calls(torch_dev, mode, inp, n, out, wmax, apart):
+    """kt_hip_quant_linear_swiglu_sums against ref_swiglu_sums + the product of its output, both read by the add and
+    norm: every code and record, at the edges of the 256-value CTAs, one to 32 of them, g and u from one launch or two
+    (widths that are no whole slot; a long row's 4-column slots), every plane count of the down weights; levels: an x
+    of few codes, where products tie at the maximum."""
+    torch = torch_dev
+    import tritify_amd as TA
+    from tritify_amd import backend as B
+
+    say(f"case: swiglu into down in={inp} n={n} out={out} mode={mode}")
+    rng = np.random.default_rng(inp + n + out)
+    members = [(nm, rng.integers(-WLEVELS, WLEVELS + 1, size=(n, inp)).astype(np.int32),
+                wscale(rng, mode == "zero_c" and nm == "u"), None) for nm in ("g", "u")]
+    down = TA.QuantLinear("d", rng.integers(-wmax, wmax + 1, size=(out, n)).astype(np.int32), out, n, wscale(rng))
+    if not down.sums_ok():
+        assert B.quant_linear_swiglu_workspace(n, out, down.pw) == 0
+        return
+    if apart:
+        qls = [TA.QuantLinear(nm, w, n, inp, s) for nm, w, s, _ in members]
+    else:
+        grp = TA.QuantLinearGroup("gu", members, inp)
+    x, xs = codes(torch, rng, inp, mag=2 if mode == "levels" else 2**27, zero=mode == "zero_x"), \
+        rec(torch, (1509949440, 58))
+    sc, silu = B.ref_codelut(B.LUT_SILU, -30.0, 30.0, 16, 20, True)
+    sc = torch.from_numpy(sc).cuda()
+    a0, a0s = codes(torch, rng, out, 2**28), (int(rng.integers(2**30, 2**31)), 60)
+    gam, gs, eps = codes(torch, rng, out, 2**20), (1 << 30, 50), B.ref_scale_from_f64(1e-6)
+    got = []
+    for path in ("two", "one"):
+        recs = torch.full((8,), 5, dtype=torch.int64, device="cuda")
+        mrec = rec(torch, (7, 7))
+        if apart:
+            gt, up = (q.forward_sums(x, xs, rec=recs[4 * i:4 * i + 4]) for i, q in enumerate(qls))
+        else:
+            gt, up = grp.forward_sums(x, xs, os_dev=recs)
+        if path == "two":
+            h, hs = torch.zeros(n, dtype=torch.int32, device="cuda"), rec(torch, (0, 0))
+            B.ref_swiglu_sums(gt, up, n, sc, silu, h, hs)
+            m = down.forward_sums(h, hs, rec=mrec)
+        else:
+            m = down.forward_swiglu_sums(gt, up, sc, silu, rec=mrec)
+        y, ys = a0.clone(), rec(torch, a0s)
+        o, os_ = torch.zeros(out, dtype=torch.int32, device="cuda"), rec(torch, (0, 0))
+        B.ref_add_rmsnorm_sums(y, ys, m, out, y, ys, gam, gs, eps, o, os_)
+        torch.cuda.synchronize()
+        got.append((y.cpu().numpy(), o.cpu().numpy(), words(ys), words(os_), words(mrec), words(recs)))
+    two, one = got
+    assert np.array_equal(two[0], one[0]) and np.array_equal(two[1], one[1])
+    assert two[2:] == one[2:]

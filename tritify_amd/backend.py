@@ -145,6 +145,8 @@ def _declare(L: C.CDLL) -> None:
                                           _P, _P, _SZ, _P, _P, _P]),
         "kt_hip_ref_moe_route": (_I, [_I, _P, _I64, _I64, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
         "kt_hip_ref_moe_combine": (_I, [_I, _P, _P, _I64, _I64, _P, _P, _P, _I64, _I, _P, _P, _P]),
+        "kt_hip_quant_linear_swiglu_workspace": (_SZ, [_I64, _I64, _I]),
+        "kt_hip_quant_linear_swiglu_sums": (_I, [_I, _P, _P, _I64, _P, _P, _P, _I, _I64, _I64, C.c_int32, _P, _SZ, _P]),
         "kt_hip_ref_moe_experts_workspace": (_SZ, [_I64, _I64, _I64, _I64]),
         "kt_hip_ref_moe_experts": (_I, [_I, _P, _P, _I64, _I64, _I64, _I64, _P, _I, _I64, _P, _P, _P, _P, _P, _SZ, _P,
                                         _P, _P]),
@@ -510,6 +512,20 @@ def quant_linear_multi_sums(x_dev, in_f: int, xs_dev, seg_out, w_planes_dev, pw:
                           _ptr(r) if r is not None else 0))
         col0 += int(o)
     return out
+
+
+def quant_linear_swiglu_workspace(n: int, out_f: int, pw: int) -> int:
+    """Bytes of quant_linear_swiglu_sums' workspace; 0 where it does not take the shape."""
+    return lib().kt_hip_quant_linear_swiglu_workspace(n, out_f, pw)
+
+
+def quant_linear_swiglu_sums(g: QlSums, u: QlSums, n: int, silu_codes_dev, silu, w_planes_dev, pw: int, out_f: int,
+                             w_scale, ws_dev, ws_bytes: int, rec=None, stream=None, dev: int = 0) -> QlSums:
+    """ref_swiglu_sums and the one-row product of its output (the down projection), stopped at that product's sums."""
+    check(lib().kt_hip_quant_linear_swiglu_sums(
+        dev, C.byref(g), C.byref(u), n, _ptr(silu_codes_dev), C.byref(silu), _ptr(w_planes_dev), pw, out_f,
+        int(w_scale[0]), int(w_scale[1]), _ptr(ws_dev), ws_bytes, _stream(stream)), "quant linear swiglu sums")
+    return QlSums(_ptr(ws_dev), n, out_f, 0, out_f, 0, 0, _ptr(rec) if rec is not None else 0)
 
 
 def quant_linear_noalloc(x_dev, rows: int, in_f: int, xs_dev, w_planes_dev, pw: int, out_f: int, w_scale,

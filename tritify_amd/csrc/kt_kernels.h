@@ -86,9 +86,20 @@ hipError_t launch_w12_swiglu(const int8_t* x, const int8_t* lo, const uint8_t* n
 size_t ql_workspace_bytes(int64_t rows, int64_t in, int64_t out, size_t off[KT_QL_WS_PARTS]);
 // The one-row product alone (kt_hip_quant_linear_multi_sums): no bias, the sums and states left in the workspace.
 bool ql_sums_ok(int64_t in, int64_t out, int pw, int64_t flush_k);
+int ql_skinny_cols(int64_t in, int64_t out);  // the columns of each CTA, and of each of its maxima at part 2
 hipError_t launch_quant_linear_sums(const int32_t* x, int64_t in, const kt_hip_qscale* xs, const int8_t* wb, int pw,
                                     int nseg, const int64_t* seg_out, const int64_t* w_mant, const int32_t* w_shift,
                                     int64_t flush_k, void* ws, hipStream_t s);
+// The row a SwiGLU leaves to the one-row product: its products (int64), their largest magnitude per part (nparts <= 64)
+// and the Scale they are at.
+struct QlHv {
+    const int64_t *v, *part;
+    int nparts;
+    const kt_hip_qscale* scale;
+};
+// That product of such a row (one output, no bias): the sums and state left in the workspace as above.
+hipError_t launch_quant_linear_hv(const QlHv& hv, int64_t in, const int8_t* wb, int pw, int64_t out, int64_t w_mant,
+                                  int32_t w_shift, int64_t flush_k, void* ws, hipStream_t s);
 // Several QuantLinear calls on one x (seg_out[g] output columns each, weights side by side in wb): one x pass, one
 // digit GEMM, each call's own requantization into y[g] with record os[g].
 hipError_t launch_quant_linear_multi(const int32_t* x, int64_t rows, int64_t in, const kt_hip_qscale* xs,

@@ -253,9 +253,13 @@ constexpr int64_t QS_FUSED_OUT = 16384;
 constexpr int QS_THREADS = 256, QS_WAVES = QS_THREADS / 64;
 constexpr int QS_COLS = QS_WAVES * 2;  // a CTA's columns (CPW = 2 per wave); long rows of few columns take CPW = 1
 
-template <int PW, int MAXKP, int KS, int CPW>
-__global__ __launch_bounds__(QS_THREADS * KS) void ql_skinny_kernel(const int32_t* __restrict__ x, int in, int kp,
-                                                               const kt_hip_qscale* __restrict__ xs,
+//
+// HV: the row is not codes but a SwiGLU's products (QlHv: int64 values, the partial maxima of their magnitudes, the
+// Scale they are at): its codes are requant_dyn of them, whose largest magnitude is 2^28 (quant_to is then a shift), or
+// zeros at Scale::ZERO where all products are zero; no pass writes or reads the codes.
+template <int PW, int MAXKP, int KS, int CPW, bool HV>
+__global__ __launch_bounds__(QS_THREADS * KS) void ql_skinny_kernel(const int32_t* __restrict__ x, QlHv hv, int in,
+                                                               int kp, const kt_hip_qscale* __restrict__ xs,
                                                                const int8_t* __restrict__ wb, int64_t* __restrict__ y,
                                                                int N, const int64_t* __restrict__ bias, QlSeg seg,
                                                                QlScales sc, QlState* __restrict__ st,
@@ -292,39 +296,82 @@ __global__ __launch_bounds__(QS_THREADS * KS) void ql_skinny_kernel(const int32_
                                     : v4i{};
     }
 
-    // the row, 4 columns per quad, QPT quads per thread held in registers; max |x| over the CTA
-    int32_t xv[QPT][4];
+    // the row, 4 columns per quad, QPT quads per thread held in registers; max |x| over the CTA (HV: known)
     uint32_t m = 0;
+    int64_t hm = 0;  // HV: the products' largest magnitude
+    if constexpr (HV) {
+        int64_t hq[QPT][4];
 #pragma unroll
-    for (int k = 0; k < QPT; k++) {
-        const int c0 = 4 * (tid + NT * k);
+        for (int k = 0; k < QPT; k++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            xv[k][t] = c0 + t < in ? x[c0 + t] : 0;
-            const uint32_t a = xv[k][t] < 0 ? 0u - (uint32_t)xv[k][t] : (uint32_t)xv[k][t];
-            m = a > m ? a : m;
-        }
-    }
-    {  // max |x| over the CTA: each wave's by DPP, then all of them
-        m = wave_max_u32(m);
-        if (lane == 0) red[wv] = m;
-        __syncthreads();
+            for (int t = 0; t < 4; t++) {
+                const int c = 4 * (tid + NT * k) + t;
+                hq[k][t] = c < in ? hv.v[c] : 0;
+            }
+        hm = wave_max_i64(lane < hv.nparts ? hv.part[lane] : 0);  // nparts <= 64
+        const RqDen d = rq_den(hm);
+        m = hm != 0 ? 1u << 28 : 0;
 #pragma unroll
-        for (int w = 0; w < NT / 64; w++) m = red[w] > m ? red[w] : m;
-    }
-    const double rinv = m != 0 ? 1.0 / (double)m : 0.0;
-#pragma unroll
-    for (int k = 0; k < QPT; k++) {
-        const int c0 = 4 * (tid + NT * k);
-        if (c0 < kp) {
+        for (int k = 0; k < QPT; k++) {
+            const int c0 = 4 * (tid + NT * k);
+            if (c0 >= kp) continue;
             uint32_t word[3] = {0, 0, 0};
-            if (m != 0) ql_digits4r(xv[k], m, rinv, word);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                if (hm == 0 || hq[k][t] == 0) continue;
+                const int32_t code = rq_apply(d, hq[k][t]);  // quant_to: round_half_away(code WLEVELS / 2^28)
+                const uint64_t u = ((uint64_t)(code < 0 ? -(int64_t)code : (int64_t)code) * WLEVELS + (1u << 27)) >> 28;
+                int64_t q = code < 0 ? -(int64_t)u : (int64_t)u;
+#pragma unroll
+                for (int p = 0; p < 3; p++) {
+                    const int64_t dg = ((q + 128) & 255) - 128;
+                    word[p] |= ((uint32_t)dg & 255u) << (8 * t);
+                    q = (q - dg) >> 8;
+                }
+            }
 #pragma unroll
             for (int p = 0; p < 3; p++) *reinterpret_cast<uint32_t*>(xq + p * kp + c0) = word[p];
         }
+    } else {
+        int32_t xv[QPT][4];
+#pragma unroll
+        for (int k = 0; k < QPT; k++) {
+            const int c0 = 4 * (tid + NT * k);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                xv[k][t] = c0 + t < in ? x[c0 + t] : 0;
+                const uint32_t a = xv[k][t] < 0 ? 0u - (uint32_t)xv[k][t] : (uint32_t)xv[k][t];
+                m = a > m ? a : m;
+            }
+        }
+        {  // max |x| over the CTA: each wave's by DPP, then all of them
+            m = wave_max_u32(m);
+            if (lane == 0) red[wv] = m;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < NT / 64; w++) m = red[w] > m ? red[w] : m;
+        }
+        const double rinv = m != 0 ? 1.0 / (double)m : 0.0;
+#pragma unroll
+        for (int k = 0; k < QPT; k++) {
+            const int c0 = 4 * (tid + NT * k);
+            if (c0 < kp) {
+                uint32_t word[3] = {0, 0, 0};
+                if (m != 0) ql_digits4r(xv[k], m, rinv, word);
+#pragma unroll
+                for (int p = 0; p < 3; p++) *reinterpret_cast<uint32_t*>(xq + p * kp + c0) = word[p];
+            }
+        }
     }
     if (blockIdx.x == 0 && tid < seg.n) {  // each segment's state, for ql_requant_kernel
-        const QlHead h = ql_head(m, xs, sc, tid);
+        kt_hip_qscale hrec{};
+        if constexpr (HV) {  // the codes' record
+            const Sc r = hm == 0 ? Sc{0, 0}
+                                 : sc_mul(from_ratio((u128)(uint64_t)hm, (u128)ACT_LEVELS),
+                                          Sc{hv.scale->mant, hv.scale->shift});
+            hrec.mant = r.mant, hrec.shift = r.shift;
+        }
+        const QlHead h = ql_head(m, HV ? &hrec : xs, sc, tid);
         QlState* q = st + tid;
         q->xmax = h.xmax, q->c_mant = h.c.mant, q->f_mant = h.f.mant;
         q->c_shift = h.c.shift, q->f_shift = h.f.shift, q->mode = h.mode;
@@ -730,7 +777,7 @@ bool ql_sums_ok(int64_t in, int64_t out, int pw, int64_t flush_k) {
 // The columns of a CTA of that product: QS_COLS, or half of them for a long row whose CTAs of QS_COLS would leave more
 // than half of the 256 CUs without one (4864 -> 896 columns, 112 CTAs or 224: 10.6 or 8.7 us). At most 256 slots then,
 // within part 2 of the workspace.
-static int ql_skinny_cols(int64_t in, int64_t out) {
+int ql_skinny_cols(int64_t in, int64_t out) {
     return (in + 63) / 64 * 64 > QS_MAX_KP && out <= 128 * QS_COLS ? QS_COLS / 2 : QS_COLS;
 }
 // every CTA of at most QS_COLS columns within one segment
@@ -743,7 +790,7 @@ static bool ql_seg_cols_ok(const QlSeg& seg) {
 // largest |sum| at part 2.
 static hipError_t launch_ql_skinny(const int32_t* x, int64_t in, const kt_hip_qscale* xs, const int8_t* wb, int pw,
                                    int64_t out, const QlSeg& seg, const QlScales& sc, const int64_t* bias, void* ws,
-                                   hipStream_t s) {
+                                   hipStream_t s, const QlHv* hv = nullptr) {
     size_t off[KT_QL_WS_PARTS];
     ql_workspace_bytes(1, in, out, off);
     char* base = (char*)ws;
@@ -753,9 +800,15 @@ static hipError_t launch_ql_skinny(const int32_t* x, int64_t in, const kt_hip_qs
     const int64_t kp = (in + 63) / 64 * 64;
     const bool long_row = kp > QS_MAX_KP && kp <= QS_LONG_KP && pw == 3;
     const int cols = ql_skinny_cols(in, out), ctas = (int)((out + cols - 1) / cols);
-#define KT_QS(P, K, S, C)                                                                                            \
-    ql_skinny_kernel<P, K, S, C><<<ctas, QS_THREADS * S, 0, s>>>(x, (int)in, (int)kp, xs, wb, acc, (int)out, bias,  \
-                                                                seg, sc, st, pm)
+#define KT_QS(P, K, S, C)                                                                                             \
+    do {                                                                                                              \
+        if (hv)                                                                                                       \
+            ql_skinny_kernel<P, K, S, C, true><<<ctas, QS_THREADS * S, 0, s>>>(nullptr, *hv, (int)in, (int)kp, nullptr, \
+                                                                              wb, acc, (int)out, bias, seg, sc, st, pm); \
+        else                                                                                                          \
+            ql_skinny_kernel<P, K, S, C, false><<<ctas, QS_THREADS * S, 0, s>>>(x, QlHv{}, (int)in, (int)kp, xs, wb,  \
+                                                                               acc, (int)out, bias, seg, sc, st, pm); \
+    } while (0)
     if (long_row && cols < QS_COLS) KT_QS(3, QS_LONG_KP, 4, 1);
     else if (long_row) KT_QS(3, QS_LONG_KP, 4, 2);
     else if (pw == 1) KT_QS(1, QS_MAX_KP, 1, 2);
@@ -911,6 +964,16 @@ hipError_t launch_quant_linear_sums(const int32_t* x, int64_t in, const kt_hip_q
     for (int g = nseg; g <= KT_QL_MAX_SEG; g++) seg.col0[g] = (int)at;
     if (!ql_sums_ok(in, at, pw, flush_k) || !ql_seg_cols_ok(seg)) return hipErrorInvalidValue;
     return launch_ql_skinny(x, in, xs, wb, pw, at, seg, sc, nullptr, ws, s);
+}
+
+hipError_t launch_quant_linear_hv(const QlHv& hv, int64_t in, const int8_t* wb, int pw, int64_t out, int64_t w_mant,
+                                  int32_t w_shift, int64_t flush_k, void* ws, hipStream_t s) {
+    QlSeg seg;
+    QlScales sc;
+    QlOut yo;
+    ql_one(out, w_mant, w_shift, nullptr, 0, 0, nullptr, nullptr, seg, sc, yo);
+    if (!ql_sums_ok(in, out, pw, flush_k) || hv.nparts > 64) return hipErrorInvalidValue;
+    return launch_ql_skinny(nullptr, in, nullptr, wb, pw, out, seg, sc, nullptr, ws, s, &hv);
 }
 
 hipError_t launch_ref_conv2d(const int32_t* x, const ConvGeom& g, const kt_hip_qscale* xs, const int8_t* wb, int pw,

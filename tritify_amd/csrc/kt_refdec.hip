@@ -707,6 +707,74 @@ __global__ __launch_bounds__(RD_THREADS) void rd_swiglu_kernel(const int32_t* __
         put_rec(hs, hmax == 0 ? Sc{0, 0} : sc_mul(from_ratio((u128)(uint64_t)hmax, (u128)ACT_LEVELS), hsc));
 }
 
+// The same activation of one row with g and u as sums, spread over the chip and left at its products for the down
+// projection (ql_skinny_kernel's HV form), whose CTAs requantize them: a CTA of 256 threads takes 256 values, the maxima
+// of g and u from the product's slots (one per CTA of 8 columns there) rather than from all the sums, and writes its
+// values' products, their largest magnitude (part[blockIdx.x]) and, CTA 0, the Scale they are at and g's and u's records.
+// One CTA for the row (above) forms two requantizations, a table read and a third requantization of 5 values a thread on
+// one CU: 13.8 us and 8.7 for the down product at 4864 values; here 5.6 and 9.1, the step of 2 layers 236 -> 220.
+constexpr int RD_SPLIT = 256;
+__global__ __launch_bounds__(RD_SPLIT) void rd_swiglu_split_kernel(RqSums gsum, RqSums usum,
+                                                                   const int64_t* __restrict__ gpart,
+                                                                   const int64_t* __restrict__ upart, int nparts, int n,
+                                                                   const int64_t* __restrict__ codes, kt_hip_codelut L,
+                                                                   int64_t* __restrict__ hv, int64_t* __restrict__ part,
+                                                                   kt_hip_qscale* __restrict__ scale) {
+    constexpr int NW = RD_SPLIT / 64;
+    __shared__ int64_t red[2][NW], hred[NW];
+    __shared__ Sc par[3];  // index factor, identity factor, h scale
+    const int tid = threadIdx.x, lane = tid & 63, wv = wave_id();
+    const int i = (int)blockIdx.x * RD_SPLIT + tid, ii = i < n ? i : n - 1;
+    const int64_t ga = gsum.acc[ii], ua = usum.acc[ii];
+    int64_t gmax = 0, umax = 0;  // the slots hold no negative value
+    for (int q = tid; q < nparts; q += RD_SPLIT) {
+        gmax = gpart[q] > gmax ? gpart[q] : gmax;
+        umax = upart[q] > umax ? upart[q] : umax;
+    }
+    gmax = wave_max_i64(gmax), umax = wave_max_i64(umax);
+    if (lane == 0) red[0][wv] = gmax, red[1][wv] = umax;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        gmax = red[0][w] > gmax ? red[0][w] : gmax;
+        umax = red[1][w] > umax ? red[1][w] : umax;
+    }
+    const Sc cs{L.code_mant, L.code_shift};
+    if (wv == 0) {  // g's factors (its Scale first)
+        const Sc gs = rqs_scale_u(gsum.st, uni64(gmax));
+        const Sc mi = sc_mul(gs, Sc{L.inv_mant, L.inv_shift}), idf = sc_mul(gs, sc_recip(cs));
+        if (lane == 0) {
+            par[0] = mi, par[1] = idf;
+            if (blockIdx.x == 0) rqs_record(gsum, gmax, gs);
+        }
+    } else if (wv == 1) {  // u's side
+        const Sc us = rqs_scale_u(usum.st, uni64(umax));
+        const Sc hs = sc_mul(cs, us);
+        if (lane == 0) {
+            par[2] = hs;
+            if (blockIdx.x == 0) rqs_record(usum, umax, us), put_rec(scale, hs);
+        }
+    }
+    const int32_t gd = rqs_live(gsum.st, gmax) ? rq_apply(rq_den(gmax), ga) : 0;
+    const int32_t ud = rqs_live(usum.st, umax) ? rq_apply(rq_den(umax), ua) : 0;
+    __syncthreads();
+    int64_t h = 0;
+    if (i < n) {
+        const int64_t idx = lut_index32(par[0], gd, L.lo_index);
+        h = wmul(idx < 0 ? 0 : (idx >= L.n ? sc_apply32(par[1], gd) : lut_code(codes, L.n, idx)), ud);
+        hv[i] = h;
+    }
+    const int64_t m = wave_max_i64(iabs(h));
+    if (lane == 0) hred[wv] = m;
+    __syncthreads();
+    if (tid == 0) {
+        int64_t b = 0;  // as the one-CTA kernel's maximum: from 0
+#pragma unroll
+        for (int w = 0; w < NW; w++) b = hred[w] > b ? hred[w] : b;
+        part[blockIdx.x] = b;
+    }
+}
+
 // apply_gelu (kt-model-vision/src/nonlin.rs:30-45): each code through the GELU CodeLut at x's scale (0 below the
 // table, the identity factor xs / code_scale above it), cast to i32, the output at the table's code scale with no
 // requantization. Grid-stride over n; each CTA forms the two factors from the record.
@@ -2240,6 +2308,63 @@ extern "C" int kt_hip_ref_swiglu_sums(int dev, const kt_hip_ql_sums* g, const kt
     kt::rd_swiglu_kernel<true><<<1, kt::RD_THREADS, 0, (hipStream_t)stream>>>(
         nullptr, nullptr, nullptr, nullptr, gs, us, (int)n, silu_codes_dev, *silu, h_dev, hs_dev);
     return (int)hipGetLastError();
+}
+
+// The workspace: the down product's (kt_hip_quant_linear_workspace of one row), then the products, their partial maxima
+// and their Scale.
+static size_t rd_swiglu_ws(int64_t n, int64_t out, size_t off[3]) {
+    size_t ql[KT_QL_WS_PARTS];
+    const size_t parts = (size_t)(n + kt::RD_SPLIT - 1) / kt::RD_SPLIT;
+    size_t at = kt::ql_workspace_bytes(1, n, out, ql);
+    const size_t sizes[3] = {(size_t)n * 8, parts * 8, sizeof(kt_hip_qscale)};
+    for (int i = 0; i < 3; i++) {
+        off[i] = at;
+        at += kt::rd_round256(sizes[i]);
+    }
+    return at;
+}
+
+extern "C" size_t kt_hip_quant_linear_swiglu_workspace(int64_t n, int64_t out_f, int pw) {
+    size_t off[3];
+    return kt_hip_quant_linear_sums_ok(n, out_f, pw) ? rd_swiglu_ws(n, out_f, off) : 0;
+}
+
+extern "C" int kt_hip_quant_linear_swiglu_sums(int dev, const kt_hip_ql_sums* g, const kt_hip_ql_sums* u, int64_t n,
+                                               const int64_t* silu_codes_dev, const kt_hip_codelut* silu,
+                                               const int8_t* w_planes_dev, int pw, int64_t out_f, int64_t w_mant,
+                                               int32_t w_shift, void* ws_dev, size_t ws_bytes, void* stream) {
+    kt::RqSums gs{}, us{};
+    if (!silu_codes_dev || !silu || !w_planes_dev || !ws_dev || n < 1 || w_mant < 0 || silu->n < 1 ||
+        !silu->right_identity || !rq_sums_of(g, n, &gs) || !rq_sums_of(u, n, &us) || (gs.rec && gs.rec == us.rec) ||
+        ws_dev == g->ws || ws_dev == u->ws || (reinterpret_cast<uintptr_t>(ws_dev) & 15))
+        return (int)hipErrorInvalidValue;
+    const size_t need = kt_hip_quant_linear_swiglu_workspace(n, out_f, pw);
+    if (need == 0 || ws_bytes < need) return (int)hipErrorInvalidValue;
+    // the maxima come from the slots of g's and u's product, one per 8 columns: the outputs are whole slots (as the
+    // product's boundaries are), of a row whose CTAs have 8 columns
+    const int64_t cols = kt::ql_skinny_cols(g->in_f, g->out_f);
+    const kt_hip_ql_sums* d[2] = {g, u};
+    const int64_t* part[2];
+    for (int i = 0; i < 2; i++) {
+        if (d[i]->col0 % 8 || (d[i]->n % 8 && d[i]->col0 + d[i]->n != d[i]->out_f) ||
+            kt::ql_skinny_cols(d[i]->in_f, d[i]->out_f) != cols)
+            return (int)hipErrorInvalidValue;
+        size_t off[KT_QL_WS_PARTS];
+        kt::ql_workspace_bytes(1, d[i]->in_f, d[i]->out_f, off);
+        part[i] = reinterpret_cast<const int64_t*>(static_cast<const char*>(d[i]->ws) + off[2]) + d[i]->col0 / cols;
+    }
+    RD_TRY(hipSetDevice(dev));
+    size_t off[3];
+    rd_swiglu_ws(n, out_f, off);
+    char* base = static_cast<char*>(ws_dev);
+    int64_t *hv = reinterpret_cast<int64_t*>(base + off[0]), *hp = reinterpret_cast<int64_t*>(base + off[1]);
+    kt_hip_qscale* scale = reinterpret_cast<kt_hip_qscale*>(base + off[2]);
+    const int ctas = (int)((n + kt::RD_SPLIT - 1) / kt::RD_SPLIT);
+    kt::rd_swiglu_split_kernel<<<ctas, kt::RD_SPLIT, 0, (hipStream_t)stream>>>(
+        gs, us, part[0], part[1], (int)((n + cols - 1) / cols), (int)n, silu_codes_dev, *silu, hv, hp, scale);
+    RD_TRY(hipGetLastError());
+    return (int)kt::launch_quant_linear_hv(kt::QlHv{hv, hp, ctas, scale}, n, w_planes_dev, pw, out_f, w_mant, w_shift,
+                                           kt_hip_flush_k(3, pw), ws_dev, (hipStream_t)stream);
 }
 
 extern "C" int kt_hip_ref_swiglu(int dev, const int32_t* g_dev, const kt_hip_qscale* gs_dev, const int32_t* u_dev,

@@ -113,6 +113,15 @@ class QuantLinear:
         return B.quant_linear_multi_sums(x_dev, self.in_features, xs_dev, [self.out_features], self.w_planes, self.pw,
                                          [self.w_scale], ws, n, recs=[rec], stream=stream, dev=self.dev)[0]
 
+    def forward_swiglu_sums(self, g, u, silu_codes, silu_lut, rec=None, stream=None):
+        """forward_sums of the SwiGLU of g and u (B.QlSums of a gate / up pair) without that row in memory."""
+        if not hasattr(self, "_ws_swiglu"):
+            n = B.quant_linear_swiglu_workspace(self.in_features, self.out_features, self.pw)
+            self._ws_swiglu = (self.torch.empty(n, dtype=self.torch.uint8, device=self.device), n)
+        ws, n = self._ws_swiglu
+        return B.quant_linear_swiglu_sums(g, u, self.in_features, silu_codes, silu_lut, self.w_planes, self.pw,
+                                          self.out_features, self.w_scale, ws, n, rec=rec, stream=stream, dev=self.dev)
+
     def forward_int_host(self, x_codes, x_scale):
         """forward_int on host codes at Scale x_scale = (mant, shift): (y codes, dict of the output scale)."""
         torch = self.torch

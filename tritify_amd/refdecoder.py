@@ -193,7 +193,8 @@ class RefDecoder:
 
     def _block_sums(self, i: int, blk, stream) -> None:
         """One block of decode_step with each projection stopped at its sums and requantized by its reader: q / k / v
-        -> attention, o -> add + post norm, gate / up -> SwiGLU, down -> add + the next norm (9 launches)."""
+        -> attention, o -> add + post norm, gate / up -> SwiGLU's products -> down -> add + the next norm (9
+        launches)."""
         b, r, dv = self.buf, self.rec, self.dev
         q, k, v = blk["qkv"].forward_sums(b["h"], r["h"], os_dev=self._rec_qkv, stream=stream)
         B.ref_attention_step_sums(q, k, v, self.pos, self.nh, self.nkv, self.hd, self.max_seq, self.kc[i], self.vc[i],
@@ -204,8 +205,7 @@ class RefDecoder:
         B.ref_add_rmsnorm_sums(b["x"], r["x"], a, self.dim, b["x"], r["x"], g_, gs_, self.eps, b["h"], r["h"], stream,
                                dv)
         gt, up = blk["gu"].forward_sums(b["h"], r["h"], os_dev=self._rec_gu, stream=stream)
-        B.ref_swiglu_sums(gt, up, self.hidden, self.silu_codes, self.silu_lut, b["hh"], r["hh"], stream, dv)
-        m = blk["down"].forward_sums(b["hh"], r["hh"], rec=r["m"], stream=stream)
+        m = blk["down"].forward_swiglu_sums(gt, up, self.silu_codes, self.silu_lut, rec=r["m"], stream=stream)
         g_, gs_ = self.blocks[i + 1]["in_norm"] if i + 1 < len(self.blocks) else self.final_norm
         B.ref_add_rmsnorm_sums(b["x"], r["x"], m, self.dim, b["x"], r["x"], g_, gs_, self.eps, b["h"], r["h"], stream,
                                dv)
