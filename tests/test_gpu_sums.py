@@ -250,3 +250,9 @@ def test_swiglu_into_the_down_product_equals_the_two_calls(torch_dev, mode, inp,
     two, one = got
     assert np.array_equal(two[0], one[0]) and np.array_equal(two[1], one[1])
     assert two[2:] == one[2:]
+
+
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 2049])
+def test_add_rmsnorm_sums_at_the_edges_of_a_thread_s_values(torch_dev, n):
+    """One value a thread up to 1024, several beyond: the sums path against requant + add_rmsnorm around that line."""
+    test_add_rmsnorm_sums_equals_requant_then_add_rmsnorm(torch_dev, "live", 200, n)

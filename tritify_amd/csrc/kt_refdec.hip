@@ -512,8 +512,10 @@ __global__ __launch_bounds__(RD_THREADS) void rd_add_kernel(const int32_t* a, co
 // y from the codes still in registers and the Scale thread 0 formed for ys. The same integers as rd_add_kernel and
 // rd_rmsnorm_kernel in sequence. SUMS: b is a QuantLinear's sums (bsum), its requant_dyn and record formed here
 // first, as ql_requant_kernel would.
+// NV: the values a thread holds, 1 or RD_AN: the values past n cost what the others do (a row of 896 in 4 a
+// thread: 13.0 us, in 1: 10.4).
 constexpr int RD_AN = 4;
-template <bool SUMS>
+template <bool SUMS, int NV>
 __global__ __launch_bounds__(RD_THREADS) void rd_add_norm_kernel(const int32_t* a, const kt_hip_qscale* as_rec,
                                                                  const int32_t* b, const kt_hip_qscale* bs_rec,
                                                                  RqSums bsum, int n, int32_t* y, kt_hip_qscale* ys,
@@ -523,10 +525,10 @@ __global__ __launch_bounds__(RD_THREADS) void rd_add_norm_kernel(const int32_t* 
                                                                  kt_hip_qscale* __restrict__ hs) {
     __shared__ int64_t red[RD_WAVES];
     __shared__ Sc par[3];  // common, fa, fb
-    int32_t av[RD_AN], bv[RD_AN], gv[RD_AN];
-    int64_t bacc[RD_AN];
+    int32_t av[NV], bv[NV], gv[NV];
+    int64_t bacc[NV];
 #pragma unroll
-    for (int k = 0; k < RD_AN; k++) {
+    for (int k = 0; k < NV; k++) {
         const int i = threadIdx.x + RD_THREADS * k, ic = i < n ? i : n - 1;
         av[k] = a[ic], gv[k] = g[ic];
         if constexpr (SUMS) bacc[k] = bsum.acc[ic];
@@ -535,12 +537,12 @@ __global__ __launch_bounds__(RD_THREADS) void rd_add_norm_kernel(const int32_t* 
     int64_t bmax = 0;
     if constexpr (SUMS) {  // b's maximum (the values past n repeat value n - 1), codes and Scale
 #pragma unroll
-        for (int k = 0; k < RD_AN; k++) bmax = iabs(bacc[k]) > bmax ? iabs(bacc[k]) : bmax;
+        for (int k = 0; k < NV; k++) bmax = iabs(bacc[k]) > bmax ? iabs(bacc[k]) : bmax;
         bmax = block_max_i64(bmax, red);
         const bool live = rqs_live(bsum.st, bmax);
         const RqDen d = rq_den(bmax);
 #pragma unroll
-        for (int k = 0; k < RD_AN; k++) bv[k] = live ? rq_apply(d, bacc[k]) : 0;
+        for (int k = 0; k < NV; k++) bv[k] = live ? rq_apply(d, bacc[k]) : 0;
     }
     const int wv = wave_id(), lane = threadIdx.x & 63;
     Sc common{0, 0};  // wave 0: the common Scale (uniform)
@@ -564,9 +566,9 @@ __global__ __launch_bounds__(RD_THREADS) void rd_add_norm_kernel(const int32_t* 
     __syncthreads();
     const Sc fa = par[1], fb = par[2];
     if (wv != 0) common = par[0];
-    int64_t m = 0, hv[RD_AN];
+    int64_t m = 0, hv[NV];
 #pragma unroll
-    for (int k = 0; k < RD_AN; k++) {
+    for (int k = 0; k < NV; k++) {
         hv[k] = 0;
         if (common.mant != 0 && (int)threadIdx.x + RD_THREADS * k < n)
             hv[k] = wadd(sc_apply32(fa, av[k]), sc_apply32(fb, bv[k]));
@@ -574,9 +576,9 @@ __global__ __launch_bounds__(RD_THREADS) void rd_add_norm_kernel(const int32_t* 
     }
     const int64_t gmax = block_max_i64(m, red);  // every read of a and b is done past here
     const RqDen rd_gmax = rq_den(gmax);
-    int32_t yv[RD_AN];
+    int32_t yv[NV];
 #pragma unroll
-    for (int k = 0; k < RD_AN; k++) {
+    for (int k = 0; k < NV; k++) {
         const int i = threadIdx.x + RD_THREADS * k;
         yv[k] = gmax == 0 ? 0 : rq_apply(rd_gmax, hv[k]);
         if (i < n) y[i] = yv[k];
@@ -586,7 +588,7 @@ __global__ __launch_bounds__(RD_THREADS) void rd_add_norm_kernel(const int32_t* 
         xs = gmax == 0 ? Sc{0, 0} : sc_mul(from_ratio((u128)(uint64_t)gmax, (u128)ACT_LEVELS), common);
         if (lane == 0) put_rec(ys, xs);
     }
-    rd_norm_row<RD_AN>(yv, gv, n, xs, Sc{g_mant, g_shift}, Sc{e_mant, e_shift}, h, hs, red);
+    rd_norm_row<NV>(yv, gv, n, xs, Sc{g_mant, g_shift}, Sc{e_mant, e_shift}, h, hs, red);
 }
 
 // SwiGluMlp::forward_int's activation (layers.rs:615-637): h = silu_code(g) * u, the SiLU code from the CodeLut at
@@ -1997,8 +1999,8 @@ hipError_t launch_rd_add(const int32_t* a, const kt_hip_qscale* as, const int32_
 hipError_t launch_rd_add_norm(const int32_t* a, const kt_hip_qscale* as, const int32_t* b, const kt_hip_qscale* bs,
                               int n, int32_t* y, kt_hip_qscale* ys, const int32_t* g, int64_t g_mant, int32_t g_shift,
                               int64_t e_mant, int32_t e_shift, int32_t* h, kt_hip_qscale* hs, hipStream_t s) {
-    rd_add_norm_kernel<false><<<1, RD_THREADS, 0, s>>>(a, as, b, bs, RqSums{}, n, y, ys, g, g_mant, g_shift, e_mant,
-                                                       e_shift, h, hs);
+    const auto kernel = n <= RD_THREADS ? rd_add_norm_kernel<false, 1> : rd_add_norm_kernel<false, RD_AN>;
+    kernel<<<1, RD_THREADS, 0, s>>>(a, as, b, bs, RqSums{}, n, y, ys, g, g_mant, g_shift, e_mant, e_shift, h, hs);
     return hipGetLastError();
 }
 hipError_t launch_rd_swiglu(const int32_t* g, const kt_hip_qscale* gs, const int32_t* u, const kt_hip_qscale* us,
@@ -2290,7 +2292,8 @@ extern "C" int kt_hip_ref_add_rmsnorm_sums(int dev, const int32_t* a_dev, const 
         bs.rec == hs_dev)
         return (int)hipErrorInvalidValue;
     RD_TRY(hipSetDevice(dev));
-    kt::rd_add_norm_kernel<true><<<1, kt::RD_THREADS, 0, (hipStream_t)stream>>>(
+    const auto kernel = n <= kt::RD_THREADS ? kt::rd_add_norm_kernel<true, 1> : kt::rd_add_norm_kernel<true, kt::RD_AN>;
+    kernel<<<1, kt::RD_THREADS, 0, (hipStream_t)stream>>>(
         a_dev, as_dev, nullptr, nullptr, bs, (int)n, y_dev, ys_dev, g_dev, g_mant, g_shift, eps_mant, eps_shift, h_dev,
         hs_dev);
     return (int)hipGetLastError();
