@@ -1122,12 +1122,16 @@ __host__ __device__ inline RdHeadsLayout rd_heads_layout(int max_seq, int nh, in
 // of the wave-uniform P.V path has in flight
 constexpr int RD_PV_U = 8, RD_PV_W = 16;
 // The heads kernel's dynamic LDS when its per-step arrays stay in LDS (max_seq up to about 2,400 at head_dim 64; the
-// static part is about 33 KB).
+// static part is about 37 KB).
 constexpr size_t RD_HEADS_LDS = 96 * 1024;
 
 // GA: the per-step arrays in the workspace (caches longer than LDS holds), else in LDS after q and k. SUMS: q, k and v
 // are the q / k / v product's sums (a.qsum, a.ksum, a.vsum): every CTA takes their maxima over the whole outputs,
 // forms their Scales and the codes it reads as ql_requant_kernel would (CTA 0 writes the records).
+// Bound by its chain of 64-bit Scale steps between barriers and the two round trips to the cache, not by bytes (14 / 2
+// heads of 64 at 512 positions: 0.5 MB of cache). So every phase uses waves that the phase beside it leaves idle: RoPE
+// a value a thread in the last waves, the v factors behind the numerators' waves, the Scale products a wave each; and
+// the v rows are loaded before the softmax that weighs them. 25.3 -> 20.8 us at 512 positions.
 template <bool GA, bool SUMS>
 __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a, RdHeadsLayout L) {
     __shared__ int64_t red[3 * RD_WAVES];
@@ -1136,6 +1140,7 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
     __shared__ Sc par[4];  // v_ref, s_ref, lut factor, 1 / v_ref
     __shared__ Sc sinv_s;
     __shared__ int64_t PV[RD_THREADS];
+    __shared__ int32_t VP[RD_THREADS];  // this step's v (hd <= RD_THREADS)
     extern __shared__ __align__(16) int32_t qk[];  // the rotated q_h (hd), then this step's rotated k (hd)
     const int P = L.parts, h = (int)blockIdx.x / P, part = (int)blockIdx.x % P;
     const int tid = threadIdx.x, hd = a.hd, half = hd / 2, nh = a.nh, nkv = a.nkv;
@@ -1159,21 +1164,6 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
         }
         __syncthreads();
     }
-    const bool lq = SUMS && rqs_live(a.qsum.st, ymax[0]), lk = SUMS && rqs_live(a.ksum.st, ymax[1]),
-               lv = SUMS && rqs_live(a.vsum.st, ymax[2]);
-    const RqDen dq = rq_den(ymax[0]), dk = rq_den(ymax[1]), dv = rq_den(ymax[2]);
-    auto qcode = [&](int i) -> int32_t {
-        if constexpr (SUMS) return lq ? rq_apply(dq, a.qsum.acc[i]) : 0;
-        else return a.q[i];
-    };
-    auto kcode = [&](int i) -> int32_t {
-        if constexpr (SUMS) return lk ? rq_apply(dk, a.ksum.acc[i]) : 0;
-        else return a.k[i];
-    };
-    auto vcode = [&](int i) -> int32_t {
-        if constexpr (SUMS) return lv ? rq_apply(dv, a.vsum.acc[i]) : 0;
-        else return a.v[i];
-    };
     const Sc qs = SUMS ? qkv_s[0] : rec_sc(a.qs), ksp = SUMS ? qkv_s[1] : rec_sc(a.ks),
              vsp = SUMS ? qkv_s[2] : rec_sc(a.vs);
     unsigned char* ws = a.ws;
@@ -1193,23 +1183,39 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
     Sc* VF = F + a.max_seq;                                    // v factors, per step
     int64_t* S = reinterpret_cast<int64_t*>(VF + a.max_seq);   // scores, then exp codes
 
-    // 1. RoPE (attention.rs:222-246) of q_h and of this step's k of kv head `kv`; the cache append
-    for (int j = tid; j < half; j += RD_THREADS) {
-        const kt_hip_sscale c = a.cos[(size_t)pos * half + j], sn = a.sin[(size_t)pos * half + j];
-        const Sc cm{c.mant, c.shift}, sm{sn.mant, sn.shift};
-        const int32_t qa = qcode(h * hd + j), qb = qcode(h * hd + j + half);
-        QD[j] = (int32_t)(c.sign * sc_apply32(cm, qa) - sn.sign * sc_apply32(sm, qb));
-        QD[j + half] = (int32_t)(c.sign * sc_apply32(cm, qb) + sn.sign * sc_apply32(sm, qa));
-        const int32_t ka = kcode(kv * hd + j), kb = kcode(kv * hd + j + half);
-        KP[j] = (int32_t)(c.sign * sc_apply32(cm, ka) - sn.sign * sc_apply32(sm, kb));
-        KP[j + half] = (int32_t)(c.sign * sc_apply32(cm, kb) + sn.sign * sc_apply32(sm, ka));
-    }
-    __syncthreads();
-    if (h == kv * group && part == 0)
-        for (int i = tid; i < hd; i += RD_THREADS) {
-            a.kc[(size_t)pos * kstride + kv * hd + i] = KP[i];
-            a.vc[(size_t)pos * kstride + kv * hd + i] = vcode(kv * hd + i);
+    // 1. RoPE (attention.rs:222-246) of q_h and of this step's k of kv head `kv`, this step's v, the cache append: a value
+    //    a thread, from the last thread down, so that the waves of few steps' scales (2.) work beside them; read past
+    //    the barriers of 2.
+    const bool append = h == kv * group && part == 0;
+    for (int t = RD_THREADS - 1 - tid; t < 3 * hd; t += RD_THREADS) {
+        const int w = t / hd, i = t - w * hd;  // value i of q_h (w = 0), k (1) or v (2)
+        const int j = i < half ? i : i - half, base = w == 0 ? h * hd : kv * hd;
+        const int own = base + i, other = base + (i < half ? i + half : j);
+        int32_t x, y = 0;
+        if constexpr (SUMS) {
+            const int64_t ym = w == 0 ? ymax[0] : (w == 1 ? ymax[1] : ymax[2]);
+            const int64_t* acc = w == 0 ? a.qsum.acc : (w == 1 ? a.ksum.acc : a.vsum.acc);
+            const bool live = w == 0 ? rqs_live(a.qsum.st, ymax[0])
+                                     : (w == 1 ? rqs_live(a.ksum.st, ymax[1]) : rqs_live(a.vsum.st, ymax[2]));
+            const RqDen dn = rq_den(ym);
+            x = live ? rq_apply(dn, acc[own]) : 0;
+            if (w != 2) y = live ? rq_apply(dn, acc[other]) : 0;
+        } else {
+            const int32_t* c = w == 0 ? a.q : (w == 1 ? a.k : a.v);
+            x = c[own];
+            if (w != 2) y = c[other];
         }
+        if (w == 2) {
+            VP[i] = x;
+            if (append) a.vc[(size_t)pos * kstride + own] = x;
+            continue;
+        }
+        const kt_hip_sscale c = a.cos[(size_t)pos * half + j], sn = a.sin[(size_t)pos * half + j];
+        const int64_t cx = c.sign * sc_apply32(Sc{c.mant, c.shift}, x), sy = sn.sign * sc_apply32(Sc{sn.mant, sn.shift}, y);
+        const int32_t r = (int32_t)(i < half ? cx - sy : cx + sy);
+        qk[w * hd + i] = r;
+        if (w == 1 && append) a.kc[(size_t)pos * kstride + own] = r;
+    }
     if (h == 0 && part == 0 && tid == 0) {
         a.kscale[pos] = kt_hip_sscale{ksp.mant, ksp.shift, 1};
         a.vscale[pos] = kt_hip_sscale{vsp.mant, vsp.shift, 1};
@@ -1234,9 +1240,9 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
     }
     if (tid == 0) {
         par[0] = bv.s, par[1] = bs.s;
-        par[2] = bs.s.mant ? sc_mul(bs.s, Sc{a.exp.inv_mant, a.exp.inv_shift}) : Sc{0, 0};
-        par[3] = bv.s.mant ? sc_recip(bv.s) : Sc{0, 0};  // the two reciprocals in two waves
+        par[3] = bv.s.mant ? sc_recip(bv.s) : Sc{0, 0};  // the two reciprocals and the product in three waves
     }
+    if (tid == 128) par[2] = bs.s.mant ? sc_mul(bs.s, Sc{a.exp.inv_mant, a.exp.inv_shift}) : Sc{0, 0};
     if (tid == 64) sinv_s = bs.s.mant ? sc_recip(bs.s) : Sc{0, 0};
     __syncthreads();
     const Sc v_ref = par[0], s_ref = par[1], lm = par[2], vinv = par[3], sinv = sinv_s;
@@ -1246,36 +1252,59 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
         return;
     }
 
-    // 3. scores: one thread per cached step, the whole dot (16-byte loads of the cache row where it allows)
+    // 3. scores: sp neighbouring lanes per cached step (16-byte loads of the cache row where it allows), so that few
+    //    steps still use every wave and a lane's share of the row is one batch of loads
     const bool vec = hd % 4 == 0 && (reinterpret_cast<uintptr_t>(a.kc) & 15) == 0 && ((size_t)kstride * 4) % 16 == 0;
+    const int sl = !vec || hd % 16 != 0 ? 0 : (steps <= RD_THREADS / 4 ? 2 : (steps <= RD_THREADS / 2 ? 1 : 0));
+    const int sp = 1 << sl, sub = tid & (sp - 1);
     int64_t m = INT64_MIN;
-    for (int j = tid; j < steps; j += RD_THREADS) {
-        VF[j] = v_ref.mant ? sc_mul(VF[j], vinv) : Sc{0, 0};
+    for (int j = tid >> sl; j < steps; j += RD_THREADS >> sl) {
         int64_t dot = 0;
-        if (j == pos) {
-            for (int d = 0; d < hd; d++) dot = wadd(dot, (int64_t)QD[d] * KP[d]);
-        } else if (vec) {
+        if (vec) {
             // 8 x 16 bytes of the cache row in flight at a time (16 spill registers)
             const int4* kr = reinterpret_cast<const int4*>(a.kc + (size_t)j * kstride + kv * hd);
-            for (int e4 = 0; e4 < hd / 4; e4 += 8) {
+            const int4 *kp = reinterpret_cast<const int4*>(KP), *qd = reinterpret_cast<const int4*>(QD);
+            const int n4 = hd / 4;  // a multiple of sp
+            for (int e0 = 0; e0 < n4; e0 += 8 * sp) {
                 int4 kk[8];
+                if (j != pos) {
 #pragma unroll
-                for (int u = 0; u < 8; u++) kk[u] = e4 + u < hd / 4 ? kr[e4 + u] : int4{0, 0, 0, 0};
+                    for (int u = 0; u < 8; u++) kk[u] = e0 + u * sp < n4 ? kr[e0 + u * sp + sub] : int4{0, 0, 0, 0};
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 8; u++) kk[u] = e0 + u * sp < n4 ? kp[e0 + u * sp + sub] : int4{0, 0, 0, 0};
+                }
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
-                    if (e4 + u >= hd / 4) break;
-                    const int d = 4 * (e4 + u);
-                    dot = wadd(dot, (int64_t)QD[d] * kk[u].x + (int64_t)QD[d + 1] * kk[u].y);  // each below 2^63
-                    dot = wadd(dot, (int64_t)QD[d + 2] * kk[u].z + (int64_t)QD[d + 3] * kk[u].w);
+                    if (e0 + u * sp >= n4) break;
+                    const int4 q = qd[e0 + u * sp + sub];
+                    dot = wadd(dot, (int64_t)q.x * kk[u].x + (int64_t)q.y * kk[u].y);  // each below 2^63
+                    dot = wadd(dot, (int64_t)q.z * kk[u].z + (int64_t)q.w * kk[u].w);
                 }
             }
+            for (int o = 1; o < sp; o <<= 1) dot = wadd(dot, (int64_t)__shfl_xor((long long)dot, o));
+        } else if (j == pos) {
+            for (int d = 0; d < hd; d++) dot = wadd(dot, (int64_t)QD[d] * KP[d]);
         } else {
             const int32_t* kr = a.kc + (size_t)j * kstride + kv * hd;
             for (int d = 0; d < hd; d++) dot = wadd(dot, (int64_t)QD[d] * kr[d]);
         }
         const int64_t sc = sc_apply(sc_mul(F[j], sinv), dot);
-        S[j] = sc;
+        if (sub == 0) S[j] = sc;
         m = sc > m ? sc : m;
+    }
+    // the first v values of the wave-uniform P.V (5.) are on their way during the softmax (the row of this step is not
+    // read: another CTA of this launch writes it)
+    const int slices = RD_THREADS / hd, d = tid % hd, js = tid / hd, ST = P * slices;
+    const int jw = __builtin_amdgcn_readfirstlane(js);
+    const int32_t* vcol = a.vc + kv * hd + d;
+    const bool wide = hd % 64 == 0 && jw < slices;
+    int32_t v0[RD_PV_U];
+#pragma unroll
+    for (int u = 0; u < RD_PV_U; u++) {
+        const int j = part * slices + jw + u * ST;
+        v0[u] = 0;
+        if (wide && j < pos) v0[u] = vcol[(size_t)j * kstride];
     }
     const int64_t dmax = block_max_i64(m, red);
 
@@ -1287,6 +1316,9 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
         S[j] = ec;
         sum += ec;
     }
+    // the v factors, from the other end of the CTA's waves (of few steps: the waves that have no numerators)
+    for (int j = (tid + RD_THREADS / 2) % RD_THREADS; j < steps; j += RD_THREADS)
+        VF[j] = v_ref.mant ? sc_mul(VF[j], vinv) : Sc{0, 0};
     sum = (int64_t)wave_sum_u64((uint64_t)sum);
     if ((tid & 63) == 0) red[tid >> 6] = sum;
     __syncthreads();
@@ -1299,8 +1331,7 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
 
     // 5. P.V: thread js * hd + d (hd <= RD_THREADS) sums the steps j = js (mod slices) of column d (wrapping i64:
     //    any order gives the reference's integers); the slices then add up in LDS
-    const int slices = RD_THREADS / hd, d = tid % hd, js = tid / hd;
-    const int32_t vpos = vcode(kv * hd + d);  // this step's v (its cache row is written in this same launch)
+    const int32_t vpos = VP[d];  // this step's v (its cache row is written in this same launch)
     int64_t acc = 0;
     if (hd % 64 == 0) {
         // a wave is one slice: its step, numerator and v factor are the same on every lane, so they are read once
@@ -1309,36 +1340,34 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
         // them in flight per lane at a time, so that a few dependent round trips, not one per RD_PV_U steps, pay
         // for the whole column.
         // slice jw of this CTA's share: the steps j = part * slices + jw (mod P * slices)
-        const int jw = __builtin_amdgcn_readfirstlane(js), ST = P * slices;
-        if (jw < slices) {
-            const int32_t* vcol = a.vc + kv * hd + d;
-            for (int j0 = part * slices + jw; j0 < steps; j0 += RD_PV_W * ST) {
+        if (wide) {
+            auto add = [&](int j, int32_t v) {  // j uniform
+                if (j >= steps) return;
+                const int64_t e = S[j];
+                const Sc f = VF[j];
+                const int64_t ec = ((int64_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)e >> 32)) << 32) |
+                                   (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)e);
+                Sc vf;
+                vf.mant = ((int64_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)f.mant >> 32)) << 32) |
+                          (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)f.mant);
+                vf.shift = __builtin_amdgcn_readfirstlane(f.shift);
+                acc = wadd(acc, wmul(ec, sc_apply32(vf, j == pos ? vpos : v)));
+            };
+            int j0 = part * slices + jw;
+#pragma unroll
+            for (int u = 0; u < RD_PV_U; u++) add(j0 + u * ST, v0[u]);
+            for (j0 += RD_PV_U * ST; j0 < steps; j0 += RD_PV_W * ST) {
                 int32_t vv[RD_PV_W];
 #pragma unroll
-                for (int u = 0; u < RD_PV_W; u++) {  // a step past the end reads the last one and adds nothing
-                    const int j = j0 + u * ST < steps ? j0 + u * ST : steps - 1;
-                    vv[u] = j == pos ? vpos : vcol[(size_t)j * kstride];
+                for (int u = 0; u < RD_PV_W; u++) {
+                    vv[u] = 0;
+                    if (j0 + u * ST < pos) vv[u] = vcol[(size_t)(j0 + u * ST) * kstride];
                 }
 #pragma unroll
-                for (int u = 0; u < RD_PV_W; u++) {
-                    const int j = j0 + u * ST;
-                    if (j < steps) {  // uniform
-                        const int64_t e = S[j];
-                        const Sc f = VF[j];
-                        const int64_t ec = ((int64_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)e >> 32)) << 32) |
-                                           (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)e);
-                        Sc vf;
-                        vf.mant = ((int64_t)__builtin_amdgcn_readfirstlane((int)((uint64_t)f.mant >> 32)) << 32) |
-                                  (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)f.mant);
-                        vf.shift = __builtin_amdgcn_readfirstlane(f.shift);
-                        acc = wadd(acc, wmul(ec, sc_apply32(vf, vv[u])));
-                    }
-                }
+                for (int u = 0; u < RD_PV_W; u++) add(j0 + u * ST, vv[u]);
             }
         }
     } else if (js < slices) {
-        const int ST = P * slices;
-        const int32_t* vcol = a.vc + kv * hd + d;
         for (int j0 = part * slices + js; j0 < steps; j0 += RD_PV_U * ST) {
             int32_t vv[RD_PV_U];
             int64_t ec[RD_PV_U];
@@ -1359,10 +1388,11 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
     __syncthreads();
     for (int dd = tid; dd < hd; dd += RD_THREADS) {  // this CTA's part of the head's sums (the combine adds the parts)
         int64_t t = 0;
+#pragma unroll 8
         for (int q = 0; q < slices; q++) t = wadd(t, PV[q * hd + dd]);
         HO[((size_t)h * P + part) * hd + dd] = t;
     }
-    if (tid == 0 && part == 0) HSC[h] = sc_mul(v_ref, from_ratio(1, (u128)(uint64_t)sumc));
+    if (tid == 64 && part == 0) HSC[h] = sc_mul(v_ref, from_ratio(1, (u128)(uint64_t)sumc));
 }
 
 // Step 4 of Attention::decode_step over the heads kernel's outputs: the heads' largest scale by the engine's fold,
