@@ -237,25 +237,31 @@ __device__ inline void fold_row(FoldKey& k) {
     fold_dpp<DPP_MIRROR>(k);
 }
 __device__ inline FoldKey fold_lane(const FoldKey& k, int l) { return FoldKey{lane64(k.e, l), lane64(k.m, l), lane64(k.i, l)}; }
-// The engine's fold over K sequences at once, one item per thread for each: the largest key of each wave by DPP
-// steps, one barrier, the 16 waves' keys folded in row 0 of every wave; the winners (their own Scales and indices)
-// are returned. Ends with a barrier. red: at least 3 K RD_WAVES words.
+// The engine's fold over K sequences at once, one item per thread for each, in two halves: each wave's largest key by
+// DPP steps into red (at least 3 K RD_WAVES words), ending with a barrier; then, on any whole wave, sequence q's
+// winner (its own Scale and index) out of the waves' keys. A wave without a live item writes dead keys at once, and a
+// caller lets only the waves that use a winner form it: four waves a SIMD would otherwise repeat those steps.
 template <int K>
-__device__ void block_fold_max_k(ScIdx (&v)[K], ScIdx* red) {
+__device__ void fold_waves(const ScIdx (&v)[K], ScIdx* red) {
     uint64_t* r64 = reinterpret_cast<uint64_t*>(red);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    FoldKey k[K];
+    FoldKey k[K] = {};
+    bool live = false;
 #pragma unroll
-    for (int q = 0; q < K; q++) {
-        k[q] = fold_key(v[q]);
-        fold_row(k[q]);
-        FoldKey b = fold_lane(k[q], 0);
+    for (int q = 0; q < K; q++) live = live || v[q].idx >= 0;
+    if (__ballot(live) != 0) {  // uniform
 #pragma unroll
-        for (int l = 16; l < 64; l += 16) {
-            const FoldKey c = fold_lane(k[q], l);
-            if (fold_gt(c, b)) b = c;
+        for (int q = 0; q < K; q++) {
+            k[q] = fold_key(v[q]);
+            fold_row(k[q]);
+            FoldKey b = fold_lane(k[q], 0);
+#pragma unroll
+            for (int l = 16; l < 64; l += 16) {
+                const FoldKey c = fold_lane(k[q], l);
+                if (fold_gt(c, b)) b = c;
+            }
+            k[q] = b;
         }
-        k[q] = b;
     }
     if (lane == 0)
 #pragma unroll
@@ -264,16 +270,24 @@ __device__ void block_fold_max_k(ScIdx (&v)[K], ScIdx* red) {
             d[0] = k[q].e, d[1] = k[q].m, d[2] = k[q].i;
         }
     __syncthreads();
-#pragma unroll
-    for (int q = 0; q < K; q++) {
-        FoldKey b{0, 0, 0};
-        if (lane < RD_WAVES) {
-            const uint64_t* d = r64 + (q * RD_WAVES + lane) * 3;
-            b = FoldKey{d[0], d[1], d[2]};
-        }
-        fold_row(b);
-        v[q] = fold_item(fold_lane(b, 0));
+}
+__device__ inline ScIdx fold_winner(int q, const ScIdx* red) {
+    const uint64_t* r64 = reinterpret_cast<const uint64_t*>(red);
+    const int lane = threadIdx.x & 63;
+    FoldKey b{0, 0, 0};
+    if (lane < RD_WAVES) {
+        const uint64_t* d = r64 + (q * RD_WAVES + lane) * 3;
+        b = FoldKey{d[0], d[1], d[2]};
     }
+    fold_row(b);
+    return fold_item(fold_lane(b, 0));
+}
+// Both halves, the winners in every thread. Ends with a barrier.
+template <int K>
+__device__ void block_fold_max_k(ScIdx (&v)[K], ScIdx* red) {
+    fold_waves<K>(v, red);
+#pragma unroll
+    for (int q = 0; q < K; q++) v[q] = fold_winner(q, red);
     __syncthreads();
 }
 // n: how many leading threads hold items (the rest hold idx -1); every thread of the CTA calls it. Ends with a
@@ -1131,7 +1145,8 @@ constexpr size_t RD_HEADS_LDS = 96 * 1024;
 // Bound by its chain of 64-bit Scale steps between barriers and the two round trips to the cache, not by bytes (14 / 2
 // heads of 64 at 512 positions: 0.5 MB of cache). So every phase uses waves that the phase beside it leaves idle: RoPE
 // a value a thread in the last waves, the v factors behind the numerators' waves, the Scale products a wave each; and
-// the v rows are loaded before the softmax that weighs them. 25.3 -> 20.8 us at 512 positions.
+// the v rows are loaded before the softmax that weighs them (25.3 -> 20.8 us at 512 positions); the fold's winners are
+// formed by the three waves that use them (20.8 -> 19.4).
 template <bool GA, bool SUMS>
 __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a, RdHeadsLayout L) {
     __shared__ int64_t red[3 * RD_WAVES];
@@ -1233,17 +1248,18 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
         bv = sc_pick(bv, ScIdx{vj, j});
         bs = sc_pick(bs, ScIdx{sj, j});
     }
-    {
-        ScIdx two[2] = {bv, bs};
-        block_fold_max_k<2>(two, redsc);
-        bv = two[0], bs = two[1];
+    fold_waves<2>({bv, bs}, redsc);
+    const int wv = wave_id();  // the winners and what follows from each, a wave for each chain
+    if (wv == 0) {
+        const Sc v = fold_winner(0, redsc).s, r = v.mant ? sc_recip(v) : Sc{0, 0};
+        if (tid == 0) par[0] = v, par[3] = r;
+    } else if (wv == 1) {
+        const Sc t = fold_winner(1, redsc).s, r = t.mant ? sc_recip(t) : Sc{0, 0};
+        if (tid == 64) par[1] = t, sinv_s = r;
+    } else if (wv == 2) {
+        const Sc t = fold_winner(1, redsc).s, r = t.mant ? sc_mul(t, Sc{a.exp.inv_mant, a.exp.inv_shift}) : Sc{0, 0};
+        if (tid == 128) par[2] = r;
     }
-    if (tid == 0) {
-        par[0] = bv.s, par[1] = bs.s;
-        par[3] = bv.s.mant ? sc_recip(bv.s) : Sc{0, 0};  // the two reciprocals and the product in three waves
-    }
-    if (tid == 128) par[2] = bs.s.mant ? sc_mul(bs.s, Sc{a.exp.inv_mant, a.exp.inv_shift}) : Sc{0, 0};
-    if (tid == 64) sinv_s = bs.s.mant ? sc_recip(bs.s) : Sc{0, 0};
     __syncthreads();
     const Sc v_ref = par[0], s_ref = par[1], lm = par[2], vinv = par[3], sinv = sinv_s;
     if (s_ref.mant == 0) {  // the head is skipped (the reference's `continue`): zeros at Scale::ZERO
@@ -1397,10 +1413,12 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a
 
 // Step 4 of Attention::decode_step over the heads kernel's outputs: the heads' largest scale by the engine's fold,
 // each head brought to it, requant_dyn of the concatenation, the record.
+// One wave forms the common Scale and its reciprocal (14 heads of 64: 7.2 -> 6.6 us; in every thread before).
 constexpr int RD_CB = 2;  // head-output values a combine thread holds (nh * hd up to 2048); longer rows recompute
 __global__ __launch_bounds__(RD_THREADS) void rd_attention_combine_kernel(RdAttn a, RdHeadsLayout L) {
     __shared__ int64_t red[RD_WAVES];
-    __shared__ ScIdx redsc[RD_THREADS];
+    __shared__ ScIdx redsc[2 * RD_WAVES];
+    __shared__ Sc par[2];  // the common Scale, its reciprocal
     const int tid = threadIdx.x, hd = a.hd, nh = a.nh, qstride = nh * hd, P = L.parts;
     const int64_t* HOP = reinterpret_cast<const int64_t*>(a.ws + L.ho);
     const Sc* HSC = reinterpret_cast<const Sc*>(a.ws + L.hsc);
@@ -1425,10 +1443,15 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_combine_kernel(RdAttn
         const int i = tid + RD_THREADS * k;
         hv[k] = held && i < qstride ? ho(i) : 0;
     }
-    const Sc common = block_fold_max(tid < nh ? ScIdx{HSC[tid], tid} : ScIdx{Sc{0, 0}, -1}, redsc, nh).s;
+    fold_waves<1>({tid < nh ? ScIdx{HSC[tid], tid} : ScIdx{Sc{0, 0}, -1}}, redsc);
+    if (wave_id() == 0) {  // the common Scale and its reciprocal once, not on four waves of each SIMD
+        const Sc c = fold_winner(0, redsc).s, r = c.mant != 0 ? sc_recip(c) : Sc{0, 0};
+        if (tid == 0) par[0] = c, par[1] = r;
+    }
+    __syncthreads();
+    const Sc common = par[0], cinv = par[1];
     int64_t m = 0;
     if (common.mant != 0) {
-        const Sc cinv = sc_recip(common);
         if (held) {
 #pragma unroll
             for (int k = 0; k < RD_CB; k++) {  // each value at the common scale, kept for the requant
@@ -1454,7 +1477,6 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_combine_kernel(RdAttn
             if (i < qstride) a.o[i] = rq_apply(rd_gmax, hv[k]);
         }
     } else {
-        const Sc cinv = sc_recip(common);
         for (int i = tid; i < qstride; i += RD_THREADS) a.o[i] = rq_apply(rd_gmax, sc_apply(sc_mul(HSC[i / hd], cinv), ho(i)));
     }
     if (tid == 0)
