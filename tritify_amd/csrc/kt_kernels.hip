@@ -247,19 +247,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plane_gemm_
                         atomicAdd(reinterpret_cast<unsigned long long*>(y + (size_t)m * N + n), (unsigned long long)v);
                 }
             }
-        // The hand-off in the memory model. The partial sums are agent-scope atomic read-modify-writes; each wave
-        // releases them at workgroup scope (its own atomics performed) before the barrier, which orders them before
-        // thread 0's arrival on the tile's counter, an agent-scope acquire-release. The CTA that completes the
-        // count has acquired every other CTA's sums there; the barrier after it carries that to all its waves,
-        // which read the sums with agent-scope atomic loads.
-        __shared__ int s_last;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        if (tid == 0)
-            s_last = __hip_atomic_fetch_add(&tile_cnt[blockIdx.x], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
-                     gridDim.y - 1;
-        __syncthreads();
-        if (!s_last) return;  // uniform
+        if (!split_last(&tile_cnt[blockIdx.x])) return;  // uniform
     }
 #pragma unroll
     for (int i = 0; i < WTM; i++)

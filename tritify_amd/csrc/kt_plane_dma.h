@@ -249,14 +249,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 #pragma unroll
         for (int o = 0; o < NO; o++)
             if (valid(o, i)) atomicAdd(reinterpret_cast<unsigned long long*>(y + i), (unsigned long long)f[o]);
-        __shared__ int s_last;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        if (tid == 0)
-            s_last = __hip_atomic_fetch_add(&tile_cnt[blockIdx.x], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
-                     gridDim.y - 1;
-        __syncthreads();
-        if (!s_last) return;
+        if (!split_last(&tile_cnt[blockIdx.x])) return;
 #pragma unroll
         for (int o = 0; o < NO; o++)
             if (valid(o, i)) {

@@ -400,6 +400,22 @@ __device__ __forceinline__ int ql_seg_of(const QlSeg& g, int col) {
     return s;
 }
 
+// Whether this CTA completes its tile's count of k shares (the same answer in every thread), after its own partial sums:
+// agent-scope atomic adds whose results nothing waits for. Each wave first waits for its adds to have been performed --
+// a workgroup-scope release or a barrier does not (a workgroup shares one L1, so outside threadgroup-split mode neither
+// waits on vmcnt), and thread 0's release on the counter waits for its own wave's alone. The barrier then puts all of
+// the CTA's adds before its arrival on the counter, and the CTA that completes the count reads every share's sums, by
+// agent-scope atomic loads, past the second barrier.
+__device__ __forceinline__ bool split_last(unsigned* cnt) {
+    __shared__ int s_last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.y - 1;
+    __syncthreads();
+    return s_last != 0;
+}
+
 // Raise the call's output maximum from CTA b (b > 0 only).
 __device__ __forceinline__ void ql_raise_ymax(QlState* ql, int64_t b) {
     atomicMax(&ql->ymax[blockIdx.x % KT_QL_YSLOTS].v, (unsigned long long)b);
