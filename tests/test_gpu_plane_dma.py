@@ -61,9 +61,10 @@ def test_largest_sums(torch_dev, m, n, k):
 
 
 @pytest.mark.parametrize("rows,inp,out,bias", [(27, 3584, 900, True), (256, 2000, 300, False), (5, 700, 130, True),
-                                               (70, 1100, 512, True), (1030, 100, 1030, True), (2100, 70, 2100, True)])
+                                               (5, 1300, 130, True), (70, 1100, 512, True), (1030, 100, 1030, True),
+                                               (2100, 70, 2100, True)])
 def test_quant_linear(torch_dev, rows, inp, out, bias):
-    """The layer on each tile class, k split over CTAs in the first four."""
+    """The layer on each tile class, k split over CTAs from 1100 on."""
     from test_gpu_quant import run
 
     rng = np.random.default_rng(rows + inp + out)

@@ -87,10 +87,11 @@ def test_config3_projection_shape(torch_dev):
 
 
 @pytest.mark.parametrize("rows,inp,out,with_bias", [(512, 4864, 896, True), (64, 2048, 1000, False),
-                                                      (65, 1600, 300, True)])
+                                                      (65, 1600, 300, True), (256, 4864, 896, True)])
 def test_split_k_shapes(torch_dev, rows, inp, out, with_bias):
-    """Shapes whose digit GEMM splits k across CTAs (few tiles: the config-3 down projection, one row tile, a ragged
-    second row tile), partial sums added with atomics and the bias and maximum taken by each tile's last CTA."""
+    """Shapes whose digit GEMM splits k across CTAs (few tiles: one row tile, a ragged second one, the config-3 down
+    projection at 256 rows; at 512 its tiles fill the chip whole), partial sums added with atomics and the bias and
+    maximum taken by each tile's last CTA."""
     rng = np.random.default_rng(rows + inp + out)
     x = rng.integers(-(2**28), 2**28, size=rows * inp).astype(np.int32)
     w = rng.integers(-WLEVELS, WLEVELS + 1, size=out * inp).astype(np.int32)
@@ -193,11 +194,17 @@ def group_case(torch, rng, rows, inp, outs, lims, biases, zero_x=False, w_zero_s
 
 @pytest.mark.parametrize("rows", [1, 3, 64, 512])
 def test_group_equals_separate_calls(torch_dev, rows):
-    """q / k / v- and gate / up-shaped groups (decode rows on the skinny product, prefill rows on MFMA tiles, a
-    split-k shape), biases on some members: every member's codes, Scale and maxima equal its own call's."""
+    """q / k / v- and gate / up-shaped groups (decode rows on the skinny product, prefill rows on MFMA tiles), biases on
+    some members: every member's codes, Scale and maxima equal its own call's."""
     rng = np.random.default_rng(rows)
     group_case(torch_dev, rng, rows, 896, (896, 128, 128), (WLEVELS,) * 3, (True, False, True))
     group_case(torch_dev, rng, rows, 896, (1024, 1024), (WLEVELS, WLEVELS), (False, False))
+
+
+@pytest.mark.parametrize("peak", [127, WLEVELS, 2**31 - 1])
+def test_group_over_split_k(torch_dev, peak):
+    """A group whose product splits k across CTAs, at 1, 3 and 5 weight planes."""
+    group_case(torch_dev, np.random.default_rng(peak), 40, 2048, (896, 128, 128), (peak,) * 3, (True, False, True))
 
 
 def test_group_plane_counts_and_zero_paths(torch_dev):

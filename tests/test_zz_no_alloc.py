@@ -36,7 +36,8 @@ def test_noalloc_equals_the_workspace_entry_on_calls_in_a_row(torch_dev):
     rng = np.random.default_rng(2024)
     xs, wsc, bsc = (1509949440, 58), (1657624235, 49), (1318646415, 57)
     # the first call is the largest; each later one is smaller and finds the earlier call's bytes in the scratch
-    shapes = [(512, 896, 896, True), (64, 896, 4864, False), (3, 130, 65, True), (1, 896, 896, False)]
+    shapes = [(512, 896, 896, True), (96, 3584, 896, True), (64, 896, 4864, False), (3, 130, 65, True),
+              (1, 896, 896, False)]
     for rows, inp, out, with_bias in shapes:
         say(f"case: quant_linear_noalloc rows={rows} in={inp} out={out} bias={with_bias}")
         x, w, bias = _case(rng, rows, inp, out, with_bias)
@@ -72,7 +73,7 @@ def test_noalloc_captured_in_a_graph_and_replayed(torch_dev):
 
     rng = np.random.default_rng(77)
     xs, wsc = (1509949440, 58), (1657624235, 49)
-    for rows, inp, out in ((512, 896, 896), (1, 896, 4864)):
+    for rows, inp, out in ((512, 896, 896), (96, 3584, 896), (1, 896, 4864)):
         say(f"case: quant_linear_noalloc graph rows={rows} in={inp} out={out}")
         x, w, _ = _case(rng, rows, inp, out, False)
         ql = TA.QuantLinear("g", w, out, inp, wsc, None)

@@ -1215,14 +1215,16 @@ static int plane_dma_shape(int px, int pw, int M, int N, int kp, const QlSeg& se
 }
 
 // k over several CTAs of the 32 x 64 tile: each k-tile of a CTA takes about 0.32 us there, the split costs an atomic
-// pass per share over the M x N sums (7 us a million) and about 1 us of hand-off, and must fit one CTA per CU.
-// 256 x 896, k 4864: 27.4 -> 20.1 us; 27 x 896, k 3584: 20.2 -> 9.0; 17 x 4864, k 896: left whole (7.9 against 8.5).
+// pass per share over the M x N sums (7 us a million) and 2.9 us of hand-off (the adds' way to memory and the sums' way
+// back), and must fit one CTA per CU. Whole -> split: 256 x 896, k 4864: 29.0 -> 24.6 us; 27 x 896, k 3584: 21.0 ->
+// 13.5; 5 x 896, k 896: 9.2 -> 8.2; left whole: 17 x 4864, k 896 (9.6 against 12.8), 64 x 2816, k 2048 (15.0 against
+// 16.6), 40 x 1152, k 896 (9.7 against 11.2).
 static int plane_dma_splits(int M, int N, int nk) {
     const int64_t tiles = ceil_div(N, 64) * ceil_div(M, 32), mn = (int64_t)M * N;
     int best = 1;
     int64_t cost = 320 * (int64_t)nk;  // ns
     for (int s = 2; s <= 4 && s <= nk && tiles * s <= 256; s *= 2) {
-        const int64_t c = 320 * (int64_t)((nk + s - 1) / s) + 1000 + mn * s * 7 / 1000;
+        const int64_t c = 320 * (int64_t)((nk + s - 1) / s) + 2900 + mn * s * 7 / 1000;
         if (c < cost) cost = c, best = s;
     }
     const int per = (nk + best - 1) / best;
@@ -1242,6 +1244,10 @@ int plane_gemm_splits(int px, int pw, int M, int N, int kp, int k0, int k1, cons
     want = want > 4 ? 4 : (want < 1 ? 1 : want);
     want = want > nk ? nk : want;
     const int per = (nk + want - 1) / want;
+    // what the k-tiles of the other shares take (0.47, 0.69 and 0.91 us each at 1, 3 and 5 weight planes) against the
+    // hand-off and the atomic passes: 9 x 896, k 4864: 40.0 -> 15.9 us (1 plane), 74.6 -> 25.4 (5); 64 x 896, k 448, 1
+    // plane: left whole (10.7 against 12.2), 64 x 112, k 128, 5 planes too (8.4 against 11.7)
+    if ((int64_t)(nk - per) * (360 + 110 * pw) < 2500 + (int64_t)M * N * want * 7 / 1000) return 1;
     return (nk + per - 1) / per;  // every run of k-tiles is non-empty
 }
 

@@ -12,8 +12,8 @@
 //   4096 x 448, k 1792    50.7 -> 36.9   64 x 64
 //   512 x 4864, k 896     36.4 -> 28.4   64 x 64
 //   256 x 1152, k 896     16.3 ->  8.4   32 x 64
-//   256 x 896, k 4864     33.0 -> 20.1   32 x 64, k over 2 CTAs (both sides split)
-//   64 x 2816, k 2048     22.5 -> 11.8   32 x 64, k over 2 CTAs (both sides split)
+//   256 x 896, k 4864             25     32 x 64, k over 2 CTAs (29.0 whole)
+//   64 x 2816, k 2048     22.5 -> 15.2   32 x 64
 // 128 x 128 tiles (8 waves, one CTA per CU) measured 47.5, 43.9 and 27.1 on the first three, 8 waves over the two
 // halves of each k-tile of a 64 x 128 tile 62.2, 38.0 and 38.0: a CTA alone on its CU hides neither end of its tile.
 #pragma once
