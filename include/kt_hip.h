@@ -784,7 +784,8 @@ int kt_hip_dec_rope_kv(int dev, int8_t* qkv_dev, int64_t tokens, int64_t nqkv, c
                        int8_t* vcache_dev, void* stream);
 /* Causal GQA attention with an integer softmax: head h of row t (kv head g = h / (nh / nkv)) attends positions
  * j <= p: s_j = q . k_j, m = max s_j, e_j = exp_tab[(m - s_j + 64) >> 7] (0 past its 1024 entries),
- * o = clamp(round_half_away(sum_j e_j v_j / sum_j e_j)). o is tokens x nh hd int8. hd = 64, max_pos <= 16384. */
+ * o = clamp(round_half_away(sum_j e_j v_j / sum_j e_j)). o is tokens x nh hd int8. hd = 64, max_pos <= 16384. A row
+ * whose position is outside [0, max_pos) is zeros. */
 int kt_hip_dec_attention(int dev, const int8_t* qkv_dev, int64_t tokens, int64_t nqkv, const int32_t* pos_dev,
                          const int8_t* kcache_dev, const int8_t* vcache_dev, int64_t nh, int64_t nkv, int64_t hd,
                          const int32_t* exp_tab_dev, int8_t* o_dev, int64_t max_pos, void* stream);

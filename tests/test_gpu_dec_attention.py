@@ -47,3 +47,32 @@ def test_prefill_attention(torch_dev, T, pos, nh, nkv, max_pos, table, flat):
             want = O.dec_attend(qkv[t, h * hd:(h + 1) * hd], kc.reshape(-1), vc.reshape(-1), pos + t, nkv, h // (nh // nkv),
                                 hd, exp)
             assert np.array_equal(got[t, h], want), (t, h)
+
+
+@pytest.mark.parametrize("T,pos,max_pos", [(100, -40, 30), (200, -40, 120), (130, -200, 64), (128, 300, 290), (64, 20, 20)])
+def test_positions_outside_the_caches(torch_dev, T, pos, max_pos):
+    """Rows before position 0 and from max_pos on read no cache row (the caches end where their tensors do) and give
+    zeros; the rows between are the oracle's."""
+    torch = torch_dev
+    from tritify_amd import backend as B
+    from tritify_amd import workloads as W
+
+    print(f"case: dec attention outside T={T} pos={pos} max_pos={max_pos}", file=sys.stderr, flush=True)
+    rng = np.random.default_rng(T + max_pos)
+    nh, nkv, hd = 4, 2, 64
+    qkv = rng.integers(-12, 12, size=(T, (nh + 2 * nkv) * hd)).astype(np.int8)
+    kc, vc = (rng.integers(-12, 12, size=max_pos * nkv * hd).astype(np.int8) for _ in range(2))
+    exp = W.exp_table().astype(np.int32)
+    o = torch.full((T * nh * hd,), 99, dtype=torch.int8, device="cuda")
+    d = [torch.from_numpy(a.reshape(-1)).cuda() for a in (qkv, kc, vc, exp)]
+    p = torch.tensor([pos], dtype=torch.int32, device="cuda")
+    B.check(B.lib().kt_hip_dec_attention(0, d[0].data_ptr(), T, qkv.shape[1], p.data_ptr(), d[1].data_ptr(),
+                                         d[2].data_ptr(), nh, nkv, hd, d[3].data_ptr(), o.data_ptr(), max_pos, 0),
+            "dec attention")
+    got = o.cpu().numpy().reshape(T, nh, hd)
+    for t in range(T):
+        for h in range(nh):
+            want = np.zeros(hd, np.int8)
+            if 0 <= pos + t < max_pos:
+                want = O.dec_attend(qkv[t, h * hd:(h + 1) * hd], kc, vc, pos + t, nkv, h // (nh // nkv), hd, exp)
+            assert np.array_equal(got[t, h], want), (t, h)

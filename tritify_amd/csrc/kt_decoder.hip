@@ -108,6 +108,10 @@ __global__ __launch_bounds__(256) void dec_attention_row_kernel(const int8_t* __
     __shared__ int s_part[64][HD + 1];
     const int t = blockIdx.x / nh, h = blockIdx.x - t * nh, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int p = pos[0] + t, g = h / (nh / nkv), L = p + 1;
+    if (p < 0 || p >= max_pos) {  // a position outside the caches: no access, a zero output
+        if (tid < HD) o[(size_t)t * nh * HD + h * HD + tid] = 0;
+        return;
+    }
     const int8_t* qr = qkv + (size_t)t * nqkv + h * HD;
     v4i q4[4];
 #pragma unroll
@@ -210,7 +214,8 @@ __global__ __launch_bounds__(64 * DA_WAVES) void dec_attention_kernel(
     const int nqb = (T + 31) / 32, h = (int)blockIdx.x % nh, q0 = 32 * (nqb - 1 - (int)blockIdx.x / nh);
     const int g = h / (nh / nkv), p0 = pos[0], ks = nkv * HD;
     const int rows = T - q0 < 32 ? T - q0 : 32;
-    const int plast = p0 + q0 + rows - 1 < max_pos ? p0 + q0 + rows - 1 : max_pos - 1;  // the last position any row attends
+    // the last position any row attends; position 0 is read (and no row's weights take it) where every row's is negative
+    const int pend = p0 + q0 + rows - 1, plast = pend < 0 ? 0 : (pend < max_pos ? pend : max_pos - 1);
     const int ntile = plast / 32 + 1, pq = p0 + q0 + ql;                                // this lane's row's own position
     const int8_t* kb = kc + (size_t)g * HD;
     const int8_t* vb = vc + (size_t)g * HD;
@@ -360,8 +365,9 @@ __global__ __launch_bounds__(64 * DA_WAVES) void dec_attention_kernel(
 #pragma unroll
     for (int i = 0; i < DA_WAVES; i++) dn += sDen[i][q];
     uint32_t out = 0;
+    if (p0 + q0 + q >= 0 && p0 + q0 + q < max_pos)  // a position outside the caches: a zero output
 #pragma unroll
-    for (int i = 0; i < 4; i++) out |= (uint32_t)(uint8_t)div_round_q8(sO[(4 * c + i) * OS + q], dn) << (8 * i);
+        for (int i = 0; i < 4; i++) out |= (uint32_t)(uint8_t)div_round_q8(sO[(4 * c + i) * OS + q], dn) << (8 * i);
     *reinterpret_cast<uint32_t*>(o + (size_t)(q0 + q) * nh * HD + h * HD + 4 * c) = out;
 }
 
