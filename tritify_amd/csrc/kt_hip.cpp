@@ -19,6 +19,7 @@
 #include <string>
 #include <tuple>
 
+#include "kt_fetch.h"
 #include "kt_kernels.h"
 
 namespace {
@@ -86,20 +87,28 @@ int planes_of(const int32_t* v, size_t n) {
     return plane_class(digits_for(v, n));
 }
 
-// A pinned host buffer.
-struct PinBuf {
-    void* ptr = nullptr;
-    hipError_t need(size_t bytes) { return ptr ? hipSuccess : hipHostMalloc(&ptr, bytes, hipHostMallocDefault); }
-    void release() {
-        if (ptr) (void)hipHostFree(ptr);
-        ptr = nullptr;
+// PinnedFetch's runtime. A refused allocation leaves no error behind for the next call's hipGetLastError.
+struct HipFetch {
+    typedef hipError_t Err;
+    typedef hipStream_t Stream;
+    typedef hipEvent_t Event;
+    static Err host_alloc(void** p, size_t n) {
+        const Err e = hipHostMalloc(p, n, hipHostMallocDefault);
+        if (e != hipSuccess) *p = nullptr, (void)hipGetLastError();
+        return e;
     }
+    static void host_free(void* p) { (void)hipHostFree(p); }
+    static Err event(Event* v) {
+        const Err e = hipEventCreateWithFlags(v, hipEventDisableTiming);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e;
+    }
+    static void event_free(Event v) { (void)hipEventDestroy(v); }
+    static Err copy(void* d, const void* s, size_t n, Stream st) { return hipMemcpyAsync(d, s, n, hipMemcpyDeviceToHost, st); }
+    static Err record(Event v, Stream st) { return hipEventRecord(v, st); }
+    static Err wait(Event v) { return hipEventSynchronize(v); }
+    static Err drain(Stream st) { return hipStreamSynchronize(st); }
 };
-
-// Results come back through two pinned blocks, one being filled by the copy engine while the other is moved to the
-// caller's memory: the runtime's own staging of a pageable copy does one after the other (2.5 MB: 155 us, against 53 for
-// the transfer and 80 for the move).
-constexpr size_t Y_BLOCK = 512 << 10;
 
 // k-chunk of the int32 accumulators: a group sums at most min(px, pw) plane pairs per k, each at most 128^2 in
 // magnitude, so floor((2^31 - 1) / (min(px,pw) * 16384)) terms cannot wrap; rounded down to 256.
@@ -147,8 +156,7 @@ struct kt_hip_backend {
     std::map<Key, Entry> cache;
     uint64_t bytes = 0, tick = 0;
     DevBuf xcodes, xplanes, ydev, wcodes;
-    PinBuf ypin[2];
-    hipEvent_t yev[2] = {nullptr, nullptr};
+    kt::PinnedFetch<HipFetch> fetch;
 };
 
 #define KT_TRY(expr)                          \
@@ -438,10 +446,7 @@ void kt_hip_close(kt_hip_backend* b) {
         b->xplanes.release();
         b->ydev.release();
         b->wcodes.release();
-        for (int i = 0; i < 2; i++) {
-            b->ypin[i].release();
-            if (b->yev[i]) (void)hipEventDestroy(b->yev[i]);
-        }
+        b->fetch.release();
         (void)hipStreamDestroy(b->stream);
     }
     delete b;
@@ -524,33 +529,6 @@ static hipError_t weights_for(kt_hip_backend* b, const int32_t* w, const uint64_
     return hipSuccess;
 }
 
-// The call's result (bytes of ydev) into the caller's memory, once the stream has come to it.
-static hipError_t fetch(kt_hip_backend* b, int64_t* y, size_t bytes) {
-    hipError_t e = hipSuccess;
-    for (int i = 0; i < 2 && e == hipSuccess; i++) {
-        e = b->ypin[i].need(Y_BLOCK);
-        if (e == hipSuccess && !b->yev[i]) e = hipEventCreateWithFlags(&b->yev[i], hipEventDisableTiming);
-    }
-    if (e != hipSuccess) return e;
-    char* dst = reinterpret_cast<char*>(y);
-    const char* src = static_cast<const char*>(b->ydev.ptr);
-    const size_t blocks = (bytes + Y_BLOCK - 1) / Y_BLOCK;
-    auto len = [&](size_t i) { return bytes - i * Y_BLOCK < Y_BLOCK ? bytes - i * Y_BLOCK : Y_BLOCK; };
-    auto start = [&](size_t i) {
-        const hipError_t c = hipMemcpyAsync(b->ypin[i & 1].ptr, src + i * Y_BLOCK, len(i), hipMemcpyDeviceToHost, b->stream);
-        return c != hipSuccess ? c : hipEventRecord(b->yev[i & 1], b->stream);
-    };
-    for (size_t i = 0; i < 2 && i < blocks && e == hipSuccess; i++) e = start(i);
-    for (size_t i = 0; i < blocks && e == hipSuccess; i++) {
-        e = hipEventSynchronize(b->yev[i & 1]);
-        if (e != hipSuccess) break;
-        memcpy(dst + i * Y_BLOCK, b->ypin[i & 1].ptr, len(i));
-        if (i + 2 < blocks) e = start(i + 2);
-    }
-    if (e != hipSuccess) (void)hipStreamSynchronize(b->stream);  // no copy may still write the blocks
-    return e;
-}
-
 // TcLinear::run (backend.rs:156-172) on the device.
 static int run(kt_hip_backend* b, const int32_t* x, const int32_t* w, const uint64_t* id, size_t rows, size_t out,
                size_t k, int64_t* y) {
@@ -569,11 +547,9 @@ static int run(kt_hip_backend* b, const int32_t* x, const int32_t* w, const uint
     bool temp = false;
     KT_TRY(weights_for(b, w, id, out, k, &wplanes, &pw, &temp));
     hipError_t e = hipSuccess;
-    auto fail = [&](hipError_t err) {
-        if (temp) {
-            (void)hipStreamSynchronize(b->stream);
-            (void)hipFree(wplanes);
-        }
+    auto fail = [&](hipError_t err) {  // nothing of the call is pending when it returns
+        (void)hipStreamSynchronize(b->stream);
+        if (temp) (void)hipFree(wplanes);
         return (int)err;
     };
     if ((e = b->xcodes.grow(rows * k * sizeof(int32_t))) != hipSuccess) return fail(e);
@@ -594,7 +570,7 @@ static int run(kt_hip_backend* b, const int32_t* x, const int32_t* w, const uint
                                        b->plant == KT_PLANT_DROP_TOP, b->stream)) != hipSuccess)
             return fail(e);
     }
-    if ((e = fetch(b, y, rows * out * sizeof(int64_t))) != hipSuccess) return fail(e);
+    if ((e = b->fetch(y, b->ydev.ptr, rows * out * sizeof(int64_t), b->stream)) != hipSuccess) return fail(e);
     if (temp) KT_TRY(hipFree(wplanes));
     return 0;
 }
