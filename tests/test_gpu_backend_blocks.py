@@ -1,7 +1,7 @@
 """LinearBackend results around the blocks they come back in: one value, one block less and more by a value, two and
 several blocks, resident and temporary weights, two backends at once. Against exact float64 products."""
 import sys
-import threading
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -34,22 +34,19 @@ def test_blocks(torch_dev, rows, out, keyed):
 def test_two_backends_in_two_threads(torch_dev):
     import tritify_amd as T
 
-    def work(seed, bad):
+    def work(seed):
         rng = np.random.default_rng(seed)
         b = T.HipBackend(0)
+        wrong = []
         for i in range(8):
             rows, out, k = int(rng.integers(1, 40)), int(rng.integers(1, 9000)), int(rng.integers(1, 60))
             x = rng.integers(-1000, 1000, size=(rows, k)).astype(np.int32)
             w = rng.integers(-265720, 265721, size=(out, k)).astype(np.int32)
             y = b.linear(x.reshape(-1), w.reshape(-1), rows, out, k).reshape(rows, out)
-            if not np.array_equal(y, (x.astype(np.float64) @ w.T.astype(np.float64)).astype(np.int64)):
-                bad.append((seed, i))
+            wrong.append(not np.array_equal(y, (x.astype(np.float64) @ w.T.astype(np.float64)).astype(np.int64)))
         b.close()
+        return wrong
 
-    bad = []
-    ts = [threading.Thread(target=work, args=(s, bad)) for s in (1, 2)]
-    for t in ts:
-        t.start()
-    for t in ts:
-        t.join()
-    assert not bad
+    with ThreadPoolExecutor(2) as pool:
+        for done in [pool.submit(work, s) for s in (1, 2)]:
+            assert done.result() == [False] * 8  # an exception of the thread is raised here
