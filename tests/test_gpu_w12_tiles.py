@@ -72,7 +72,8 @@ def test_dense(torch_dev, m, n, k, kind):
     assert np.array_equal(got[pad:-pad].reshape(m, n), want.astype(dt))
 
 
-@pytest.mark.parametrize("m,f,k", [(130, 64, 70), (150, 1024, 64), (300, 2432, 64), (600, 4864, 64), (1025, 1408, 128)])
+@pytest.mark.parametrize("m,f,k", [(130, 64, 70), (150, 1024, 64), (300, 2432, 64), (600, 4864, 64), (1025, 1408, 128),
+                                   (1500, 2048, 64)])
 def test_dense_swiglu(torch_dev, m, f, k):
     torch = torch_dev
     import tritify_amd as T
@@ -91,3 +92,22 @@ def test_dense_swiglu(torch_dev, m, f, k):
     got = y.cpu().numpy()
     assert (got[m * f:] == 99).all()
     assert np.array_equal(got[:m * f].reshape(m, f), want.astype(np.int8))
+
+
+# 64-row tiles in one round and in three (more tiles than CTAs), 128-row tiles, 256-row tiles
+@pytest.mark.parametrize("m,n,k", [(300, 1000, 70), (1500, 4096, 64), (2600, 4096, 64), (4096, 4096, 64)])
+def test_one_group_i8(torch_dev, m, n, k):
+    """The grouped product of one group with the int8 epilogue on each of its tiles."""
+    torch = torch_dev
+    import tritify_amd as T
+    from tritify_amd import backend as B
+
+    print(f"case: w12 one group m={m} n={n} k={k}", file=sys.stderr, flush=True)
+    x, w, mant, shift, xd, wd = inputs(torch, m, n, k, m + n + k)
+    lo, nib = pack(torch, wd, n, k)
+    y = torch.full((m * n + 64,), 99, dtype=torch.int8, device="cuda")
+    B.w12_grouped_linear(xd, m, None, 0, None, 1, m, lo, nib, n, k, torch.from_numpy(mant).cuda(),
+                         torch.from_numpy(shift).cuda(), B.EPI_I8, y, n)
+    got = y.cpu().numpy()
+    assert (got[m * n:] == 99).all()
+    assert np.array_equal(got[:m * n].reshape(m, n), requant(dot(x, w), mant, shift, -127, 127).astype(np.int8))

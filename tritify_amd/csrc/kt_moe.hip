@@ -527,14 +527,21 @@ hipError_t launch_w12_grouped(const int8_t* x, size_t x_bytes, const int32_t* li
     // CTAs share a CU), 11.5 + 0.58 for 256 x 128 (DMA-fed). SwiGLU, measured with 64, 128 and 256 rows: 512 x 4864, k
     // 896: 23.5, 22.0, 19.8 us; 300 x 4864: 17.1, 15.1, 19.3; 150 x 4864: 11.8, 13.7, 17.1; 600 x 4864: 25.4, 23.0, 21.5;
     // 2000 x 4864: 75.3, 52.9, 59.1; 1024 x 1408, k 4096: 41.6, 34.7, 48.3; 256 x 1408, k 4096: 20.9, 31.3, 47.2.
+    // Two to four rounds of 64-row tiles take 0.8 of that too where their row blocks share each column's weights (12 of
+    // them) or k is short: 2048 x 1024 (2 F = 2048), k 448: 10.1, 11.3, 14.7; 1500 x 1536, k 512: 13.6, 14.7, 15.2; with
+    // fewer row blocks they do not: 512 x 3072, k 512: 13.1, 11.3, 15.1. The int8 epilogue takes 3-7% less on every tile
+    // (9.7, 10.8, 13.5 on the first of these), so the choice is the same: over 426 shapes of each within 1.2% of the best
+    // of the three in the mean.
     int one = 0;  // rows of the tile
     if (groups == 1) {
         const int64_t nk = kp / 64;
         const auto cost = [&](int64_t bm, int64_t c, int64_t per) {
             return ((max_rows + bm - 1) / bm * tiles_n + 255) / 256 * (c + per * nk);
         };
-        const int64_t ch = cost(64, 440, 26), cd = cost(256, 1150, 58), c1 = cost(128, 880, 35);
-        const int64_t ca = c1 > 880 + 35 * nk ? c1 * 4 / 5 : c1;
+        const int64_t h1 = cost(64, 440, 26), cd = cost(256, 1150, 58), c1 = cost(128, 880, 35);
+        const int64_t rounds_h = h1 / (440 + 26 * nk);
+        const bool shared = rounds_h >= 2 && rounds_h <= 4 && (nk <= 6 || max_rows > 11 * 64);
+        const int64_t ch = shared ? h1 * 4 / 5 : h1, ca = c1 > 880 + 35 * nk ? c1 * 4 / 5 : c1;
         one = cd < ca && cd < ch && grouped_dma_lds_ok() ? 256 : (ca < ch ? 128 : 64);
     }
     // several: enough 256-row tiles (at full groups) to give every CU one: the DMA-fed kernel, one CTA per CU
