@@ -227,6 +227,7 @@ def layer_from(m: O.RefMoe, dev_sigmoid: bool):
     dict(seed=0x91, dim=256, E=32, k=4, hidden=128, norm=True, sig=1, bseed=0x92, shared=192, T=40),
     dict(seed=0x93, dim=128, E=16, k=2, hidden=64, norm=False, sig=1, bseed=0x94, shared=0, T=9),
     dict(seed=0x97, dim=128, E=16, k=4, hidden=64, norm=True, sig=1, bseed=0x98, shared=256, T=7),  # grouped gate/up
+    dict(seed=0x9A, dim=32, E=2, k=2, hidden=4160, norm=True, sig=1, bseed=0x9B, shared=0, T=5),  # one call a product
 ])
 def test_moe_layer_against_the_oracle(torch_dev, case):
     torch = torch_dev
@@ -234,6 +235,7 @@ def test_moe_layer_against_the_oracle(torch_dev, case):
     say(f"case: ref moe {c}")
     m = O.RefMoe(c["seed"], c["dim"], c["E"], c["k"], c["hidden"], c["norm"], c["sig"], c["bseed"], c["shared"])
     layer = layer_from(m, c["sig"] == 1)
+    assert layer.fused == (c["hidden"] <= 4096)
     x, xs, _ = O.rm_probe(c["seed"] + 1, c["T"] * c["dim"])
     xd, xr = i32(torch, x), recs(torch, [xs])
     # route, token by token
