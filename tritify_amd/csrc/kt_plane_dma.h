@@ -22,8 +22,8 @@
 
 namespace kt {
 
-// CTA = WM x WN x KW waves: WM row tiles of 32, WN column blocks of 32 WTN, and KW = 2 gives each half of the waves one
-// k32 half of every k-tile (their sums meet in LDS at the end).
+// CTA = WM x WN x KW waves: WM row tiles of 32, WN column blocks of 32 WTN, and KW = 2 (WTN = 1) gives each half of the
+// waves one k32 half of every k-tile (their sums meet in LDS at the end).
 template <int WM_, int WN_, int WTN_, int KW_, int NS_>
 struct PlaneTile {
     static constexpr int WM = WM_, WN = WN_, WTN = WTN_, KW = KW_, NS = NS_;
@@ -34,7 +34,7 @@ struct PlaneTile {
     static constexpr int ND = UPW + (REM ? 1 : 0);          // DMAs per wave and k-tile, the same on every wave
     static constexpr int STAGE = 1024 * UNITS, LDS = NS * STAGE;
     static_assert(REM == 0 || REM * 2 == W, "the units left over make one half unit per wave");
-    static_assert(KW == 1 || LDS >= NT * 16 * WTN * 4, "the exchange of the k halves fits the ring");
+    static_assert(KW == 1 || (WTN == 1 && LDS >= NT * 16 * 4), "the exchange of the k halves fits the ring");
     static_assert(NS >= 2 && ND * (NS - 2) <= 63, "vmcnt holds the DMAs of NS - 2 later tiles");
 };
 typedef PlaneTile<2, 2, 2, 1, 2> PlaneTile128;  // 64 x 128
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the ring is free
 
-    // outputs of the wave: index o = 16 j + r; with KW == 2 wave kw keeps half kw of them
+    // outputs of the wave: index o = 16 j + r; with KW == 2 (WTN = 1) wave kw keeps half kw of them
     constexpr int NO = 16 * WTN / KW;
     auto val = [&](int j, int r) {
         uint64_t v = 0;
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         uint64_t* ex = reinterpret_cast<uint64_t*>(ring);
 #pragma unroll
         for (int o = 0; o < NO; o++) {
-            const uint64_t v0 = val(o >> 4, o & 15), v1 = val((o + NO) >> 4, (o + NO) & 15);
+            const uint64_t v0 = val(0, o), v1 = val(0, o + NO);
             f[o] = kw ? v1 : v0;
             ex[(w * NO + o) * 64 + lane] = kw ? v0 : v1;
         }
@@ -228,11 +228,11 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         bc[j] = badd && n < N ? (uint64_t)scale_apply(ql->f_mant, ql->f_shift, ql_bias[n]) : 0;
     }
     auto at = [&](int o) {  // byte offset of output o; a column past N stays past the end (its rows' offsets saturate)
-        const int r = (ob + o) & 15, j = (ob + o) >> 4;
-        const uint32_t b = WTN == 1 ? vy[0] : (KW == 2 ? (kw ? vy[WTN - 1] : vy[0]) : vy[j]);
+        const int r = (ob + o) & 15;
+        const uint32_t b = vy[o >> 4];
         return b == KT_OOB ? KT_OOB : b + (uint32_t)(8 * (r >> 2) + (r & 3)) * (uint32_t)N * 8u;
     };
-    auto bias_of = [&](int o) { return WTN == 1 ? bc[0] : (KW == 2 ? (kw ? bc[WTN - 1] : bc[0]) : bc[o >> 4]); };
+    auto bias_of = [&](int o) { return bc[o >> 4]; };
     int64_t lmax = 0;
     auto raise = [&](uint64_t v) {
         const int64_t a = (int64_t)v < 0 ? (int64_t)(0 - v) : (int64_t)v;  // i64::abs, wrapping
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(C::NT) __attribute__((amdgpu_waves_per_eu(2, 2))) v
     if (gridDim.y > 1) {  // partial sums into y; the tile's last CTA goes on (the hand-off of plane_gemm_kernel)
         auto valid = [&](int o, size_t& i) {
             const int r = (ob + o) & 15, m = m0 + 32 * wm + 8 * (r >> 2) + 4 * half + (r & 3);
-            const int n = n0 + 32 * (WTN * wn + ((ob + o) >> 4)) + (lane & 31);
+            const int n = n0 + 32 * (WTN * wn + (o >> 4)) + (lane & 31);
             i = (size_t)m * N + n;
             return m < M && n < N;
         };

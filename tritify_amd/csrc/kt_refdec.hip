@@ -1136,7 +1136,7 @@ __host__ __device__ inline RdHeadsLayout rd_heads_layout(int max_seq, int nh, in
 // of the wave-uniform P.V path has in flight
 constexpr int RD_PV_U = 8, RD_PV_W = 16;
 // The heads kernel's dynamic LDS when its per-step arrays stay in LDS (max_seq up to about 2,400 at head_dim 64; the
-// static part is about 37 KB).
+// static part is about 13 KB).
 constexpr size_t RD_HEADS_LDS = 96 * 1024;
 
 // GA: the per-step arrays in the workspace (caches longer than LDS holds), else in LDS after q and k. SUMS: q, k and v
@@ -1151,7 +1151,7 @@ template <bool GA, bool SUMS>
 __global__ __launch_bounds__(RD_THREADS) void rd_attention_heads_kernel(RdAttn a, RdHeadsLayout L) {
     __shared__ int64_t red[3 * RD_WAVES];
     __shared__ Sc qkv_s[3];
-    __shared__ ScIdx redsc[RD_THREADS];
+    __shared__ ScIdx redsc[2 * RD_WAVES];
     __shared__ Sc par[4];  // v_ref, s_ref, lut factor, 1 / v_ref
     __shared__ Sc sinv_s;
     __shared__ int64_t PV[RD_THREADS];
@@ -1486,8 +1486,9 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_combine_kernel(RdAttn
 // The same ops over whole-sequence tensors on many CTAs (the batched forward's T-row tensors), two launches each: a
 // grid pass takes the largest magnitude, a grid pass requantizes and writes the record. Integers identical to the
 // one-CTA kernels.
-//  - Every wave forms the tensor's Scales itself on wave-uniform values (two or three Scale steps, under a
-//    microsecond): no one-CTA launch before the pass.
+//  - Every wave of add's and SwiGLU's first pass forms the tensor's Scales itself on wave-uniform values (two or three
+//    Scale steps, under a microsecond): no one-CTA launch before the pass. CTA 0 leaves them for the second pass, since
+//    y's record may overwrite an input's.
 //  - A CTA's largest magnitude goes to its own slot of the workspace and the second pass takes the largest slot. An
 //    atomic maximum on one word serialized (13 ns a CTA): SwiGLU's first pass at 256 x 4864 went from 28.3 (2,048
 //    CTAs) to 10.1 us, the add's at 256 x 896 from 13.1 (896 CTAs) to 5.5 us.
@@ -1498,8 +1499,8 @@ __global__ __launch_bounds__(RD_THREADS) void rd_attention_combine_kernel(RdAttn
 constexpr int RS_PARTS = 512;        // the first pass's CTAs at most
 constexpr int RS_FOLD_ROWS = 1024;   // RMSNorm rows that every CTA of the second pass folds itself
 struct RdSeqWs {
-    Sc par[4];               // RMSNorm past RS_FOLD_ROWS rows: the common Scale
-    uint64_t gmax;           // and the largest magnitude
+    Sc par[4];               // add and SwiGLU: RsPar's three; RMSNorm past RS_FOLD_ROWS rows: the common Scale
+    uint64_t gmax;           // those rows' largest magnitude
     int64_t part[RS_PARTS];  // the largest magnitude of each CTA of the first pass
     // then RMSNorm's rows: Sc crow[rows] (the row factor), int64_t pmax[rows] (the largest |x g| of the row)
 };
