@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
+from test_scale_dev import scale_out, sd  # noqa: F401  (sd: the device's Scale arithmetic on the host)
 
 pytestmark = pytest.mark.gpu
 
@@ -122,3 +123,43 @@ def test_attention_prefill_edges(torch_dev, nh, nkv, hd, T, mag):
                             torch.from_numpy(sin_t.view(np.uint8)).cuda(), B.ref_scale_from_f64(1.0 / np.sqrt(hd)),
                             torch.from_numpy(ec).cuda(), lut, w, n, o, os_)
     assert np.array_equal(o.cpu().numpy(), want) and rd(os_) == wsc
+
+
+@pytest.mark.parametrize("hd", [64, 96, 128])
+def test_attention_prefill_sums_at_the_i64_limit(torch_dev, sd, hd):  # noqa: F811
+    """A table of numerators 2^32 and v codes of -2^31: (row, head)s whose sums reach -2^63, alone and beside the largest
+    scale, where |sum| wraps. Against the engine's steps in Python on the host's Scales."""
+    torch = torch_dev
+    from tritify_amd import backend as B
+
+    print(f"case: attention_prefill i64 limit hd={hd}", file=sys.stderr, flush=True)
+    T, nh, num, act = 3, 2, 1 << 32, 1 << 28
+    rng = np.random.default_rng(hd)
+    for spread in (0, 2**20, 2**31 - 1):
+        v = rng.integers(-spread, spread + 1, size=(T, nh, hd)).astype(np.int64)
+        v[:, 0, 3] = -(2**31), 0, 0  # sums of -2^63 in every row, at factors 1, 1/2 and 1/3
+        vs = (1509949440, 58)
+        zero = torch.zeros(T * nh * hd, dtype=torch.int32, device="cuda")
+        cos_t, sin_t = B.ref_rope_tables(T, hd, 10000.0)
+        ec, lut = B.ref_codelut(B.LUT_EXP, -30.0, 0.0, 16, 20, False)
+        n = B.ref_attention_prefill_workspace(T, nh, nh, hd)
+        w = torch.full((n,), 0xA5, dtype=torch.uint8, device="cuda")
+        o, os_ = torch.zeros(T * nh * hd, dtype=torch.int32, device="cuda"), rec(torch, (0, 0))
+        one = rec(torch, (2**30, 60))
+        B.ref_attention_prefill(zero, one, zero, one, dev(torch, v), rec(torch, vs), T, nh, nh, hd, T,
+                                torch.from_numpy(cos_t.view(np.uint8)).cuda(),
+                                torch.from_numpy(sin_t.view(np.uint8)).cuda(), B.ref_scale_from_f64(1.0 / np.sqrt(hd)),
+                                torch.full((len(ec),), num, dtype=torch.int64, device="cuda"), lut, w, n, o, os_)
+        wrap = lambda x: (int(x) + 2**63) % 2**64 - 2**63  # noqa: E731
+        ratio = lambda a, b: scale_out(sd.sd_from_ratio, 0, a, 0, b)  # noqa: E731
+        sums = np.array([[[wrap(sum(num * int(v[j, h, d]) for j in range(i + 1))) for d in range(hd)] for h in range(nh)]
+                         for i in range(T)], dtype=np.int64)
+        sc = [scale_out(sd.sd_mul, *vs, *ratio(1, (i + 1) * num)) for i in range(T)]
+        cinv = scale_out(sd.sd_recip, *sc[0])  # the largest: one numerator
+        at = [[[sd.sd_apply(*scale_out(sd.sd_mul, *sc[i], *cinv), int(x)) for x in sums[i, h]] for h in range(nh)]
+              for i in range(T)]
+        gmax = max(0, max(wrap(abs(x)) for r in at for h in r for x in h))
+        want = [sd.sd_rq_apply(gmax, x) if gmax else 0 for r in at for h in r for x in h]
+        assert sums[0, 0, 3] == sums[1, 0, 3] == -(2**63)
+        assert o.cpu().numpy().tolist() == want, spread
+        assert rd(os_) == (scale_out(sd.sd_mul, *ratio(gmax, act), *sc[0]) if gmax else (0, 0)), spread

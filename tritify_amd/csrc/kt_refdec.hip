@@ -105,6 +105,8 @@ __device__ inline void put_rec(kt_hip_qscale* r, Sc s) {
     *r = o;
 }
 __device__ inline int64_t iabs(int64_t v) { return v < 0 ? (int64_t)(0 - (uint64_t)v) : v; }
+// |v|, INT64_MAX for INT64_MIN
+__device__ inline int64_t magnitude(int64_t v) { return v == INT64_MIN ? INT64_MAX : iabs(v); }
 __device__ inline int64_t wmul(int64_t a, int64_t b) { return (int64_t)((uint64_t)a * (uint64_t)b); }
 __device__ inline int64_t wadd(int64_t a, int64_t b) { return (int64_t)((uint64_t)a + (uint64_t)b); }
 
@@ -1633,10 +1635,12 @@ __global__ __launch_bounds__(256) void rs_rows_kernel(RdSeq q) {
 }
 
 // The largest of n Scales by the engine's fold over their order (of equal values the latest), and the largest
-// magnitude at that scale of the groups they scale, pmax holding each group's largest |value|; NT threads of the CTA.
-template <int NT>
+// magnitude at that scale of the groups they scale, pmax holding each group's largest |value| (INT64_MAX for a value of
+// INT64_MIN); NT threads of the CTA. Below 2^62 a factor of at most 1 keeps the order of the magnitudes; past(r, factor)
+// gives group r's largest from its values where they may wrap.
+template <int NT, class Past>
 __device__ inline void scale_fold(const Sc* scale, const int64_t* pmax, int n, uint64_t* redk, int64_t* red, Sc& cc,
-                                  int64_t& gmax) {
+                                  int64_t& gmax, Past past) {
     FoldKey k{0, 0, 0};
     for (int r = threadIdx.x; r < n; r += NT) {
         const FoldKey u = fold_key(ScIdx{scale[r], r});
@@ -1660,18 +1664,23 @@ __device__ inline void scale_fold(const Sc* scale, const int64_t* pmax, int n, u
     int64_t m = 0;
     if (cc.mant != 0) {
         const Sc cinv = sc_recip(cc);
-        for (int r = threadIdx.x; r < n; r += NT) m = max64(m, sc_apply(sc_mul(scale[r], cinv), pmax[r]));
+        for (int r = threadIdx.x; r < n; r += NT) {
+            const Sc f = sc_mul(scale[r], cinv);
+            m = max64(m, pmax[r] <= (int64_t)1 << 62 ? sc_apply(f, pmax[r]) : past(r, f));
+        }
     }
     if constexpr (NT == 256) gmax = block_max_4w(m, red);
     else gmax = block_max_i64(m, red);
 }
+// RMSNorm's |x g| is at most 2^62.
+__device__ inline int64_t rs_no_past(int, Sc) { return 0; }
 // past RS_FOLD_ROWS rows: the fold by one CTA
 __global__ __launch_bounds__(RD_THREADS) void rs_norm_fold_kernel(RdSeq q) {
     __shared__ uint64_t redk[3 * RD_THREADS / 16];
     __shared__ int64_t red[RD_WAVES];
     Sc cc;
     int64_t gmax;
-    scale_fold<RD_THREADS>(rs_crow(q.ws), rs_pmax(q.ws, q.rows), q.rows, redk, red, cc, gmax);
+    scale_fold<RD_THREADS>(rs_crow(q.ws), rs_pmax(q.ws, q.rows), q.rows, redk, red, cc, gmax, rs_no_past);
     if (threadIdx.x == 0) q.ws->par[0] = cc, q.ws->gmax = (uint64_t)gmax;
 }
 // RMSNorm's second pass: a CTA per row (grid-stride), FOLD: its CTAs fold the rows themselves.
@@ -1681,7 +1690,7 @@ __global__ __launch_bounds__(256) void rs_norm_out_kernel(RdSeq q) {
     __shared__ int64_t red[4];
     Sc cc;
     int64_t gmax;
-    if constexpr (FOLD) scale_fold<256>(rs_crow(q.ws), rs_pmax(q.ws, q.rows), q.rows, redk, red, cc, gmax);
+    if constexpr (FOLD) scale_fold<256>(rs_crow(q.ws), rs_pmax(q.ws, q.rows), q.rows, redk, red, cc, gmax, rs_no_past);
     else cc = q.ws->par[0], gmax = (int64_t)q.ws->gmax;
     const RqDen rd_gmax = rq_den(gmax);
     const Sc cinv = cc.mant != 0 ? sc_recip(cc) : Sc{0, 0};
@@ -1871,7 +1880,7 @@ __global__ __launch_bounds__(256) void rp_head_kernel(RdPrefill a) {
         int64_t t = wadd(wadd(part[0][w][d], part[1][w][d]), wadd(part[2][w][d], part[3][w][d]));
         if (sumc <= 0) t = 0;
         a.hout[ih * HD + d] = t;
-        pm = max64(pm, iabs(t));
+        pm = max64(pm, magnitude(t));
     }
     pm = wave_max_i64(pm);
     const int64_t su = uni64(sumc);
@@ -1919,7 +1928,7 @@ __global__ __launch_bounds__(256) void rp_head_any_kernel(RdPrefill a) {
         t = sumc > 0 ? t : 0;
         a.hout[ih * hd + tid] = t;
     }
-    const int64_t pm = block_max_4w(iabs(t), red);
+    const int64_t pm = block_max_4w(magnitude(t), red);
     if (tid == 0) {
         a.hmax[ih] = pm;
         a.fac[ih] = sumc > 0 ? sc_mul(rec_sc(a.vs), from_ratio(1, (u128)(uint64_t)sumc)) : Sc{0, 0};
@@ -1931,7 +1940,11 @@ __global__ __launch_bounds__(RD_THREADS) void rp_fold_kernel(RdPrefill a) {
     __shared__ int64_t red[RD_WAVES];
     Sc common;
     int64_t gmax;
-    scale_fold<RD_THREADS>(a.fac, a.hmax, a.T * a.nh, redk, red, common, gmax);
+    scale_fold<RD_THREADS>(a.fac, a.hmax, a.T * a.nh, redk, red, common, gmax, [&](int r, Sc f) {
+        int64_t b = 0;
+        for (int d = 0; d < a.hd; d++) b = max64(b, iabs(sc_apply(f, a.hout[(size_t)r * a.hd + d])));
+        return b;
+    });
     if (threadIdx.x == 0) *a.common = common, *a.gmax = (uint64_t)gmax;
 }
 
